@@ -2,25 +2,36 @@
 // bin_cmd_smooth (src/StarFormationHistories.jl:574-621), one template or many
 // templates per launch.
 //
-// Two kernels per call:
+// Kernels of a call:
 //   k_dep_prep    one thread per point: the reference's FP64 footprint / index
 //                 math (bit-exact, no FMA contraction) and every per-point
-//                 constant of the evaluation -> an 80-byte PointDesc.
-//   k_dep_gather  bin-owner gather: a thread owns one row and kCPT = 16
-//                 consecutive columns of one template, in registers; a
-//                 workgroup 256 such strips.  Every wave walks its template's
-//                 descriptors in order through scalar loads (the descriptor is
-//                 uniform across the wave, so it sits in scalar registers: no
-//                 LDS staging, no barriers), skips points whose rows miss its
-//                 strips, and adds each point's contribution to its bins, so
-//                 there are no atomics and every bin sums its points in point
-//                 order (deterministic).  Contributions accumulate in FP32 per
-//                 64 points and are flushed into FP64 accumulators.
-// The pair work is VALU bound (about 3 + DEG VALU operations and one exp2 per
-// GL node and bin for the series forms); HBM traffic is the descriptors in and
-// one write of each template out.
+//                 constant of the evaluation -> a 112-byte PointDesc.
+//   k_dep_wide    the wide kernels' sums on every fourth column (see sfh_psf.h).
+//   k_dep_gather  every other point, then the wide kernels' sums interpolated.
+//                 Both are bin-owner gathers: a thread owns one row and kCPT =
+//                 16 consecutive columns (or nodes) of one template, in
+//                 registers; a workgroup 256 such strips.  Every wave walks its
+//                 template's descriptors in order through scalar loads (the
+//                 descriptor is uniform across the wave, so it sits in scalar
+//                 registers: no LDS staging, no barriers), skips points whose
+//                 rows miss its strips, and adds each point's contribution to
+//                 its bins, so there are no atomics and every bin sums its
+//                 points in a fixed order (deterministic).  Contributions
+//                 accumulate in FP32 per 64 points and are flushed into FP64
+//                 accumulators.
+//   k_dep_finish  small launches, whose points are split into slices: their sums.
+// The pair work is VALU bound; HBM traffic is the descriptors in, the wide sums
+// out and in again (0.1 GB for 700 templates of 200 x 300 bins) and one write
+// of each template.  700 such templates (2.9e10 pairs, 74% of them in rows of
+// one node, 22% in rows of two): 7.5 ms with three nodes per row and every
+// column evaluated, 6.0 ms with the nodes merged, 4.0 ms (1.76 wide + 2.23)
+// with the wide kernels on a quarter of their columns and the accumulators
+// reached by LDS instead of flat accesses (VGPRs 112 -> 89).
 #include "sfh_internal.h"
 #include "sfh_psf.h"
+
+#include <algorithm>
+#include <type_traits>
 
 namespace sfh {
 
@@ -29,6 +40,12 @@ using psf::PointDesc;
 constexpr int kDepBlock = 256;
 constexpr int kCPT = psf::kCPT;  // columns per thread
 constexpr int kChunk = 64;       // points between FP32 -> FP64 flushes
+constexpr int64_t kWideBytes = (int64_t)512 << 20;   // scratch of the wide kernels' sums per launch
+// Workgroups that a sliced launch aims at: four per CU, one resident round.  A
+// launch of fewer splits its points: 50 templates of 75 x 100 bins are 100
+// workgroups (0.50 ms -> 0.25 ms of gather plus 0.01 ms for the slices' sums),
+// one of 100 x 151 bins 5 (0.45 -> 0.17 ms).
+constexpr int64_t kGatherSlots = 1024;
 
 __global__ __launch_bounds__(256) void k_dep_prep(
     const double* __restrict__ colors, const double* __restrict__ mags,
@@ -58,104 +75,236 @@ __global__ __launch_bounds__(256) void k_dep_prep(
     if ((threadIdx.x & 63) == 0 && cnt) atomicAdd(pairs, cnt);
 }
 
-// The FP64 accumulators live in LDS (16 per thread, 32 KiB per workgroup),
-// touched once per 64 points, so that the FP32 strip and the per-point
-// constants fit four waves per SIMD (a fifth, at 95 registers with the
-// series' coefficient products formed per column, measured slower).
-// Workgroup w of the gather takes (template, row band) order[w] = t * nblk + band
-// when an order is given: the (template, band) pairs by decreasing cost, so
-// the longest workgroups start first and the launch ends with short ones.
-// Without one, template t's band j is (j + t) mod nblk: consecutive workgroups
-// go to the 8 XCDs in turn, so without the rotation every template's band j
-// would land on XCD j mod 8 and the populated bands of a diagram would load
-// some XCDs far more than others.
+struct GatherArgs {
+    int nx, ny;
+    int ncg, nblk;               // strips per row, workgroups per template
+    int wcg;                     // strips per row of the wide kernels' nodes (0: none)
+    int wslices;                 // slices of the wide kernels' sums
+    double* wide;                // their sums: [slice][template][ny][16 wcg]
+    int64_t wstride;             // between slices
+    double* part;                // sliced: [slice][template][ny * nx], else NULL
+    float* out32;
+    double* out64;
+    int64_t ld_out;
+};
+
+// Workgroup -> (template, band): order[blockIdx.x] when an order is given (the
+// pairs by decreasing cost, so the longest workgroups start first and the
+// launch ends with short ones); otherwise template t's band j is (j + t) mod
+// nblk: consecutive workgroups go to the 8 XCDs in turn, so without the
+// rotation every template's band j would land on XCD j mod 8 and the populated
+// bands of a diagram would load some XCDs far more than others.
+__device__ __forceinline__ void gather_tile(const int32_t* __restrict__ order, int nblk, int64_t* t, int* blk)
+{
+    if (order) {
+        const int id = order[blockIdx.x];
+        *t = id / nblk;
+        *blk = id - (int)*t * nblk;
+    } else {
+        *t = blockIdx.x / nblk;
+        *blk = (int)((blockIdx.x - *t * nblk + *t) % nblk);
+    }
+}
+
+// FP64 accumulators in LDS, [column][thread].  Volatile, so that they stay
+// there instead of being promoted to registers, and through a pointer into the
+// LDS address space (a volatile access is not moved out of the generic one by
+// the compiler, and flat accesses would wait for the global loads too).
+typedef volatile __attribute__((address_space(3))) double lds_double;
+struct LdsAcc {
+    lds_double* p;
+    __device__ lds_double* operator[](int c) const { return p + c * kDepBlock; }
+};
+
+// One lane's point of a chunk: its footprint (the descriptor's first 16 bytes)
+// and form.
+struct Foot {
+    int4 f;
+    int kind;
+};
+__device__ inline Foot footprint(const PointDesc* td, int p, int np)
+{
+    Foot r;
+    if (p < np) {
+        r.f = *reinterpret_cast<const int4*>(td + p);
+        r.kind = td[p].kind;
+    } else {
+        r.f = make_int4(1, 0, 1, 0);
+        r.kind = psf::kDirect;
+    }
+    return r;
+}
+
+// f(descriptor) for each of a chunk's points in hits, in order.  Descriptors
+// are uniform across the wave, so they are read through scalar loads, two per
+// wait.
+template <class F>
+__device__ __forceinline__ void each(const PointDesc* __restrict__ chunk, uint64_t hits, F f)
+{
+    while (hits) {
+        const int i = __builtin_ctzll(hits);
+        hits &= hits - 1;
+        const bool two = hits != 0;
+        const int j = two ? __builtin_ctzll(hits) : i;
+        if (two) hits &= hits - 1;
+        const PointDesc d0 = chunk[i];
+        const PointDesc d1 = chunk[j];
+        f(d0);
+        if (two) f(d1);
+    }
+}
+
+// The wide kernels (kWide1, kWide2) of a template on their nodes, every
+// kStep-th column: the gather below with 16 nodes of one row per thread and
+// one form per loop, into the FP64 sums [slice][template][row][node] that
+// k_dep_gather (or k_dep_finish) interpolates.
+__global__ __launch_bounds__(kDepBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_dep_wide(
+    const PointDesc* __restrict__ desc, const int64_t* __restrict__ offsets, GatherArgs a)
+{
+    __shared__ double sacc_[kCPT][kDepBlock];
+    const LdsAcc sacc{(lds_double*)&sacc_[0][0]};
+    int64_t t;
+    int blk;
+    const int nblk = (a.wcg * a.ny + kDepBlock - 1) / kDepBlock;
+    gather_tile(nullptr, nblk, &t, &blk);
+    const int64_t p0 = offsets[t], p1 = offsets[t + 1];
+    const int slot = blk * kDepBlock + threadIdx.x;
+    const int row = slot / a.wcg;
+    const int col0 = (slot - row * a.wcg) * kCPT;
+    const bool valid = row < a.ny;
+    const int wslot = __builtin_amdgcn_readfirstlane(blk * kDepBlock + (int)(threadIdx.x & ~63u));
+    const int row_lo = wslot / a.wcg, row_hi = (wslot + 63) / a.wcg;
+    float part[kCPT];
+#pragma unroll
+    for (int c = 0; c < kCPT; ++c) {
+        sacc[c][threadIdx.x] = 0.0;
+        part[c] = 0.0f;
+    }
+    const PointDesc* __restrict__ td = desc + p0;
+    const int np = (int)(p1 - p0);
+    const int nch = (np + kChunk - 1) / kChunk;
+    const int c0 = (int)((int64_t)nch * blockIdx.y / gridDim.y), c1 = (int)((int64_t)nch * (blockIdx.y + 1) / gridDim.y);
+    const int lane = threadIdx.x & 63;
+    auto add = [&](const PointDesc& d, auto nodes) {
+        constexpr int NODES = decltype(nodes)::value;
+        if (!(valid && row >= d.ya && row <= d.yb)) return;
+        float M[NODES], L[NODES], h[NODES];
+        psf::merged_row<NODES>(d, row, M, L, h);
+        psf::gauss_strip<NODES, false>(d, M, L, h, col0, part);
+    };
+    Foot fn = footprint(td, c0 * kChunk + lane, np);
+    for (int ch = c0; ch < c1; ++ch) {
+        const Foot f = fn;
+        fn = footprint(td, (ch + 1) * kChunk + lane, np);           // next chunk's footprints in flight
+        const bool hit = f.f.x <= f.f.y && f.f.z <= row_hi && f.f.w >= row_lo;
+        const uint64_t h1 = __ballot(hit && f.kind == psf::kWide1), h2 = __ballot(hit && f.kind == psf::kWide2);
+        if (!(h1 | h2)) continue;
+        each(td + ch * kChunk, h1, [&](const PointDesc& d) { add(d, std::integral_constant<int, 1>{}); });
+        each(td + ch * kChunk, h2, [&](const PointDesc& d) { add(d, std::integral_constant<int, 2>{}); });
+#pragma unroll
+        for (int c = 0; c < kCPT; ++c) {
+            sacc[c][threadIdx.x] += (double)part[c];
+            part[c] = 0.0f;
+        }
+    }
+    if (!valid) return;
+    double* o = a.wide + blockIdx.y * a.wstride + (t * a.ny + row) * (int64_t)(a.wcg * kCPT) + col0;
+#pragma unroll
+    for (int c = 0; c < kCPT; c += 2)
+        *reinterpret_cast<double2*>(o + c) = make_double2(sacc[c][threadIdx.x], sacc[c + 1][threadIdx.x]);
+}
+
+// kStep columns from col (a multiple of kStep) of one row of template t: v plus
+// the wide kernels' sums interpolated from their nodes (slices added in
+// order), written to the outputs.
+__device__ inline void finish_cols(const GatherArgs& a, int64_t t, int row, int col, double* v)
+{
+    static constexpr psf::InterpWeights W = psf::interp_weights();
+    if (a.wcg) {
+        // column col + r lies r / kStep past node col / kStep + kLead
+        const int ldw = a.wcg * kCPT;
+        const double* w = a.wide + (t * a.ny + row) * (int64_t)ldw + col / psf::kStep;
+        double n[psf::kTaps];
+#pragma unroll
+        for (int k = 0; k < psf::kTaps; ++k) n[k] = w[k];
+        for (int s = 1; s < a.wslices; ++s) {
+            w += a.wstride;
+#pragma unroll
+            for (int k = 0; k < psf::kTaps; ++k) n[k] += w[k];
+        }
+        v[0] += n[psf::kLead];
+#pragma unroll
+        for (int r = 1; r < psf::kStep; ++r)
+#pragma unroll
+            for (int k = 0; k < psf::kTaps; ++k) v[r] = fma(W.w[r][k], n[k], v[r]);
+    }
+    const int64_t base = t * a.ld_out + (int64_t)row * a.nx + col;
+#pragma unroll
+    for (int r = 0; r < psf::kStep; ++r) {
+        if (col + r >= a.nx) continue;
+        if (a.out32) a.out32[base + r] = (float)v[r];
+        if (a.out64) a.out64[base + r] = v[r];
+    }
+}
+
+// The FP64 accumulators live in LDS (16 per thread, 32 KiB per workgroup: five
+// workgroups per CU), touched once per 64 points, so that the FP32 strip and
+// the per-point constants fit the registers of five waves per SIMD.
 template <bool kAsym>
 __global__ __launch_bounds__(kDepBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_dep_gather(
     const PointDesc* __restrict__ desc, const int64_t* __restrict__ offsets, const int32_t* __restrict__ order,
-    int nx, int ny, int ncg, int nblk_per_tpl, float* __restrict__ out32, double* __restrict__ out64,
-    int64_t ld_out)
+    GatherArgs a)
 {
-    __shared__ double sacc[kCPT][kDepBlock];
+    __shared__ double sacc_[kCPT][kDepBlock];
+    const LdsAcc sacc{(lds_double*)&sacc_[0][0]};
     int64_t t;
     int blk;
-    if (order) {
-        const int id = order[blockIdx.x];
-        t = id / nblk_per_tpl;
-        blk = id - (int)t * nblk_per_tpl;
-    } else {
-        t = blockIdx.x / nblk_per_tpl;
-        blk = (int)((blockIdx.x - t * nblk_per_tpl + t) % nblk_per_tpl);
-    }
+    gather_tile(order, a.nblk, &t, &blk);
+    const int nx = a.nx, ncg = a.ncg;
     const int64_t p0 = offsets[t], p1 = offsets[t + 1];
     const int slot = blk * kDepBlock + threadIdx.x;
     const int row = slot / ncg;
     const int col0 = (slot - row * ncg) * kCPT;
-    const bool valid = row < ny;
+    const bool valid = row < a.ny;
     // rows of this wave's 64 strips (wave-uniform)
     const int wslot = __builtin_amdgcn_readfirstlane(blk * kDepBlock + (int)(threadIdx.x & ~63u));
     const int row_lo = wslot / ncg, row_hi = (wslot + 63) / ncg;
 
-    // volatile: the accumulators stay in LDS instead of being promoted to registers
-    volatile double* acc = &sacc[0][threadIdx.x];
     float part[kCPT];
 #pragma unroll
     for (int c = 0; c < kCPT; ++c) {
-        acc[c * kDepBlock] = 0.0;
+        sacc[c][threadIdx.x] = 0.0;
         part[c] = 0.0f;
     }
-    // Each chunk of 64 points: every lane reads one point's footprint (the
-    // descriptor's first 16 bytes) and form, a ballot keeps the points whose
-    // rows meet this wave's strips, and only those descriptors are loaded --
-    // through scalar loads (uniform across the wave), two descriptors per
-    // wait.  The hits are taken in two passes: first the common case (the
-    // Gaussian form with a footprint spanning the whole grid width), then
-    // every other point.  Each pass has one code path, so the strip's registers
-    // carry through it without copies; a bin sums the chunk's common-case
-    // points, then the others, each in point order (deterministic).
+    // Each chunk of 64 points: every lane reads one point's footprint and form,
+    // ballots keep the points whose rows meet this wave's strips, and only
+    // those descriptors are loaded.  The hits are taken in passes: first the
+    // common cases (a Gaussian form with a footprint spanning the whole grid
+    // width, one node per row, then two -- the asymmetric kernel's second is
+    // the form with a y factor per row), then every other point but the wide
+    // kernels.  Each pass has one code path, so the strip's registers carry
+    // through it without copies; a bin sums a chunk's points pass by pass, each
+    // in point order (deterministic).
     const PointDesc* __restrict__ td = desc + p0;
     const int np = (int)(p1 - p0);
+    const int nch = (np + kChunk - 1) / kChunk;
+    const int c0 = (int)((int64_t)nch * blockIdx.y / gridDim.y), c1 = (int)((int64_t)nch * (blockIdx.y + 1) / gridDim.y);
     const int lane = threadIdx.x & 63;
     const int wave_id = (int)(threadIdx.x >> 6);
-    struct Foot {
-        int4 f;
-        int kind;
-    };
-    auto footprint = [&](int pc) {
-        const int p = pc + lane;
-        Foot r;
-        if (p < np) {
-            r.f = *reinterpret_cast<const int4*>(td + p);
-            r.kind = td[p].kind;
-        } else {
-            r.f = make_int4(1, 0, 1, 0);
-            r.kind = psf::kDirect;
-        }
-        return r;
-    };
     auto in_rows = [&](const PointDesc& d) { return valid && row >= d.ya && row <= d.yb; };
-    auto add_common = [&](const PointDesc& d) {
+    // the common forms: NODES merged nodes per row (0: the asymmetric kernel's
+    // y factor), no column mask
+    auto add_common = [&](const PointDesc& d, auto nodes) {
+        constexpr int N = decltype(nodes)::value, NODES = N ? N : 1;
         if (!in_rows(d)) return;
-        if constexpr (kAsym) {
-            float M[1], L[1] = {0.0f}, h[1] = {0.0f};
-            M[0] = d.pref * psf::y_factor(fmaf((float)(row - d.ya), d.dv, d.ay), d.ey);
-            psf::gauss_strip<1, false>(d, M, L, h, col0, part);
-        } else {
-            float M[3], L[3], h[3];
-            psf::cov_row_log(d, row, M, L, h);
-            psf::gauss_strip<3, false>(d, M, L, h, col0, part);
-        }
+        float M[NODES], L[NODES] = {}, h[NODES] = {};
+        if constexpr (N == 0) M[0] = d.pref * psf::y_factor(fmaf((float)(row - d.ya), d.dv, d.ay), d.ey);
+        else psf::merged_row<NODES>(d, row, M, L, h);
+        psf::gauss_strip<NODES, false>(d, M, L, h, col0, part);
     };
     auto add = [&](const PointDesc& d) {
         if (!in_rows(d) || col0 > d.xb || col0 + kCPT - 1 < d.xa) return;
-        if constexpr (kAsym) {
-            float W[1], h[1] = {0.0f};
-            W[0] = d.pref * psf::y_factor(fmaf((float)(row - d.ya), d.dv, d.ay), d.ey);
-            psf::add_point<1, true>(d, W, h, col0, part);
-        } else {
-            float W[3], h[3];
-            psf::cov_row(d, row, W, h);
-            psf::add_point<3, true>(d, W, h, col0, part);
-        }
+        psf::add_point<!kAsym, true>(d, row, col0, part);
     };
     // A point in the erf-difference form (a narrow kernel: its footprint is at
     // most 55 columns wide) with the whole wave cooperating, instead of the
@@ -191,66 +340,75 @@ __global__ __launch_bounds__(kDepBlock) __attribute__((amdgpu_waves_per_eu(4))) 
             }
         }
     };
-    Foot fn = footprint(0);
-    for (int pc = 0; pc < np; pc += kChunk) {
+    constexpr int kSecond = kAsym ? psf::kGauss : psf::kGauss2;
+    Foot fn = footprint(td, c0 * kChunk + lane, np);
+    for (int ch = c0; ch < c1; ++ch) {
         const Foot f = fn;
-        fn = footprint(pc + kChunk);                           // next chunk's footprints in flight
-        const bool hit = f.f.x <= f.f.y && f.f.z <= row_hi && f.f.w >= row_lo;
-        const bool common = f.kind == psf::kGauss && f.f.x == 0 && f.f.y == nx - 1;
-        uint64_t hits = __ballot(hit && common);
-        while (hits) {
-            const int i = __builtin_ctzll(hits);
-            hits &= hits - 1;
-            const bool two = hits != 0;
-            const int j = two ? __builtin_ctzll(hits) : i;
-            if (two) hits &= hits - 1;
-            const PointDesc d0 = td[pc + i];
-            const PointDesc d1 = td[pc + j];
-            add_common(d0);
-            if (two) add_common(d1);
-        }
-        hits = __ballot(hit && !common);
-        while (hits) {
-            const int i = __builtin_ctzll(hits);
-            hits &= hits - 1;
-            const bool two = hits != 0;
-            const int j = two ? __builtin_ctzll(hits) : i;
-            if (two) hits &= hits - 1;
-            const PointDesc d0 = td[pc + i];
-            const PointDesc d1 = td[pc + j];
-            // the narrow erf-difference kernels go to the wave-cooperative path
-            if (d0.kind == psf::kDirect && d0.xb - d0.xa < 63) direct(d0);
-            else add(d0);
-            if (two) {
-                if (d1.kind == psf::kDirect && d1.xb - d1.xa < 63) direct(d1);
-                else add(d1);
-            }
-        }
+        fn = footprint(td, (ch + 1) * kChunk + lane, np);           // next chunk's footprints in flight
+        const bool hit = f.f.x <= f.f.y && f.f.z <= row_hi && f.f.w >= row_lo && f.kind < psf::kWide1;
+        const bool full = f.f.x == 0 && f.f.y == nx - 1;
+        const uint64_t all = __ballot(hit);
+        if (!all) continue;
+        const uint64_t h1 = __ballot(hit && f.kind == psf::kGauss1);
+        const uint64_t h2 = __ballot(hit && full && f.kind == kSecond);
+        const PointDesc* __restrict__ chunk = td + ch * kChunk;
+        each(chunk, h1, [&](const PointDesc& d) { add_common(d, std::integral_constant<int, 1>{}); });
+        each(chunk, h2, [&](const PointDesc& d) { add_common(d, std::integral_constant<int, kAsym ? 0 : 2>{}); });
+        // the narrow erf-difference kernels go to the wave-cooperative path
+        const uint64_t h3 = __ballot(hit && f.kind == psf::kDirect && f.f.y - f.f.x < 63);
+        each(chunk, all & ~(h1 | h2 | h3), add);
+        each(chunk, h3, direct);
 #pragma unroll
         for (int c = 0; c < kCPT; ++c) {
-            acc[c * kDepBlock] += (double)part[c];
+            sacc[c][threadIdx.x] += (double)part[c];
             part[c] = 0.0f;
         }
     }
     if (!valid) return;
-    const int64_t base = t * ld_out + (int64_t)row * nx;
+    if (a.part) {
+        double* o = a.part + ((blockIdx.y * (int64_t)(gridDim.x / a.nblk) + t) * a.ny + row) * nx + col0;
 #pragma unroll
-    for (int c = 0; c < kCPT; ++c) {
-        const int col = col0 + c;
-        if (col < nx) {
-            const double v = acc[c * kDepBlock];
-            if (out32) out32[base + col] = (float)v;
-            if (out64) out64[base + col] = v;
-        }
+        for (int c = 0; c < kCPT; ++c)
+            if (col0 + c < nx) o[c] = sacc[c][threadIdx.x];
+        return;
     }
+#pragma unroll 1
+    for (int c = 0; c < kCPT && col0 + c < nx; c += psf::kStep) {
+        double v[psf::kStep];
+#pragma unroll
+        for (int r = 0; r < psf::kStep; ++r) v[r] = sacc[c + r][threadIdx.x];
+        finish_cols(a, t, row, col0 + c, v);
+    }
+}
+
+// The templates from the gather's slices, added in order, and the wide
+// kernels' sums: one thread per kStep columns of a row.
+__global__ __launch_bounds__(kDepBlock) void k_dep_finish(GatherArgs a, int64_t ntemplates, int slices)
+{
+    const int64_t g = (int64_t)blockIdx.x * kDepBlock + threadIdx.x;
+    const int nq = (a.nx + psf::kStep - 1) / psf::kStep;
+    const int64_t per = (int64_t)nq * a.ny;
+    if (g >= per * ntemplates) return;
+    const int64_t t = g / per;
+    const int row = (int)((g - t * per) / nq), col = (int)((g - t * per) % nq) * psf::kStep;
+    const double* p = a.part + (t * a.ny + row) * a.nx + col;
+    const int64_t stride = ntemplates * a.ny * a.nx;
+    double v[psf::kStep] = {};
+#pragma unroll 4
+    for (int s = 0; s < slices; ++s)
+#pragma unroll
+        for (int r = 0; r < psf::kStep; ++r) v[r] += p[s * stride + (col + r < a.nx ? r : 0)];
+    finish_cols(a, t, row, col, v);
 }
 
 // Relative cost per row strip of each x form (issue slots of the form's strip
 // code over the Gaussian form's).
 __device__ inline unsigned form_cost(int kind, bool full)
 {
-    if (kind == psf::kGauss) return full ? 4u : 6u;
-    if (kind == psf::kSeries2 || kind == psf::kSeries3) return 12u;
+    if (kind == psf::kGauss1) return 2u;
+    if (kind == psf::kGauss2) return 4u;
+    if (kind == psf::kGauss) return full ? 5u : 6u;
+    if (kind == psf::kSeries3) return 12u;
     return 32u;
 }
 
@@ -268,7 +426,7 @@ __global__ __launch_bounds__(256) void k_dep_cost(const PointDesc* __restrict__ 
     __syncthreads();
     for (int64_t p = offsets[t] + threadIdx.x; p < offsets[t + 1]; p += blockDim.x) {
         const int4 f = *reinterpret_cast<const int4*>(desc + p);
-        if (f.x > f.y) continue;
+        if (f.x > f.y || desc[p].kind >= psf::kWide1) continue;
         const bool full = f.x == 0 && f.y == nx - 1;
         const unsigned w = form_cost(desc[p].kind, full);
         const int nstrips = f.y / kCPT - f.x / kCPT + 1;
@@ -333,42 +491,81 @@ __global__ __launch_bounds__(1024) void k_dep_order(const unsigned long long* __
 }
 
 // The gather over descriptors of npoints points (template t owns
-// desc[offsets[t] .. offsets[t+1])), with the workgroups in decreasing
-// estimated cost when the launch is small enough to order in one pass.
+// desc[offsets[t] .. offsets[t+1])): the wide kernels on their nodes, then
+// everything else, with the workgroups in decreasing estimated cost when the
+// launch is small enough to order in one pass.  Where a launch would leave the
+// chip idle its points are split into slices, whose FP64 sums k_dep_finish
+// adds in order.
 static int launch_gather(sfh_ctx* ctx, const PointDesc* desc, const int64_t* d_offsets, int64_t ntemplates,
                          int64_t npoints, bool asym, int nx, int ny, float* out32, double* out64, int64_t ld_out)
 {
-    const int ncg = (int)cdiv(nx, kCPT);
-    const int nblk = (int)cdiv((int64_t)ncg * ny, kDepBlock);
-    const int64_t grid = (int64_t)nblk * ntemplates;
-    SFH_ARG_CHECK(ctx, grid < (int64_t)1 << 31, "too many templates for one launch");
-    if (grid == 0) return SFH_OK;
-    const int32_t* order = nullptr;
-    if (ntemplates > 1 && grid <= kOrderMax && npoints > 0) {
-        void *pc = nullptr, *po = nullptr;
-        if (int rc = scratch(ctx, "dep_cost", (size_t)grid * sizeof(unsigned long long), &pc)) return rc;
-        if (int rc = scratch(ctx, "dep_order", (size_t)grid * sizeof(int32_t), &po)) return rc;
-        {
-            TimedLaunch tl(ctx, "deposit_order");
-            hipLaunchKernelGGL(k_dep_cost, dim3((unsigned)ntemplates), dim3(256),
-                               (size_t)nblk * sizeof(unsigned long long), ctx->stream, desc, d_offsets, nx, ncg, nblk,
-                               (unsigned long long*)pc);
-            hipLaunchKernelGGL(k_dep_order, dim3(1), dim3(1024), 0, ctx->stream, (const unsigned long long*)pc,
-                               (int)grid, (int32_t*)po);
+    GatherArgs a{};
+    a.nx = nx;
+    a.ny = ny;
+    a.ncg = (int)cdiv(nx, kCPT);
+    a.nblk = (int)cdiv((int64_t)a.ncg * ny, kDepBlock);
+    a.wcg = psf::wide_pays(nx) ? (int)cdiv(psf::wide_nodes(nx), kCPT) : 0;
+    a.ld_out = ld_out;
+    const int64_t wblk = cdiv((int64_t)a.wcg * ny, kDepBlock), wbins = (int64_t)a.wcg * kCPT * ny;
+    SFH_ARG_CHECK(ctx, (int64_t)a.nblk * ntemplates < (int64_t)1 << 31, "too many templates for one launch");
+    // templates per launch: the wide kernels' sums within kWideBytes
+    const int64_t group = a.wcg ? std::max<int64_t>(1, std::min(ntemplates, kWideBytes / (wbins * 8))) : ntemplates;
+    for (int64_t t0 = 0; t0 < ntemplates; t0 += group) {
+        const int64_t nt = std::min(group, ntemplates - t0);
+        const int64_t grid = (int64_t)a.nblk * nt, chunks = cdiv(cdiv(npoints, ntemplates), kChunk);
+        auto slices = [&](int64_t workgroups) {
+            return (int)std::max<int64_t>(1, std::min(chunks, kGatherSlots / std::max<int64_t>(workgroups, 1)));
+        };
+        const int ns = slices(grid);
+        const int64_t* offsets = d_offsets + t0;
+        const int32_t* order = nullptr;
+        a.out32 = out32 ? out32 + t0 * ld_out : nullptr;
+        a.out64 = out64 ? out64 + t0 * ld_out : nullptr;
+        a.part = nullptr;
+        if (a.wcg) {
+            a.wslices = slices(wblk * nt);
+            a.wstride = wbins * nt;
+            void* p = nullptr;
+            if (int rc = scratch(ctx, "dep_wide", (size_t)(a.wslices * a.wstride) * sizeof(double), &p)) return rc;
+            a.wide = (double*)p;
+            TimedLaunch tl(ctx, "deposit_wide");
+            hipLaunchKernelGGL(k_dep_wide, dim3((unsigned)(wblk * nt), (unsigned)a.wslices), dim3(kDepBlock), 0,
+                               ctx->stream, desc, offsets, a);
         }
-        if (int rc = check_launch(ctx, "k_dep_order")) return rc;
-        order = (const int32_t*)po;
+        if (int rc = check_launch(ctx, "k_dep_wide")) return rc;
+        if (ns > 1) {
+            void* p = nullptr;
+            if (int rc = scratch(ctx, "dep_part", (size_t)ns * nt * nx * ny * sizeof(double), &p)) return rc;
+            a.part = (double*)p;
+        } else if (nt > 1 && grid <= kOrderMax && npoints > 0) {
+            void *pc = nullptr, *po = nullptr;
+            if (int rc = scratch(ctx, "dep_cost", (size_t)grid * sizeof(unsigned long long), &pc)) return rc;
+            if (int rc = scratch(ctx, "dep_order", (size_t)grid * sizeof(int32_t), &po)) return rc;
+            {
+                TimedLaunch tl(ctx, "deposit_order");
+                hipLaunchKernelGGL(k_dep_cost, dim3((unsigned)nt), dim3(256),
+                                   (size_t)a.nblk * sizeof(unsigned long long), ctx->stream, desc, offsets, nx,
+                                   a.ncg, a.nblk, (unsigned long long*)pc);
+                hipLaunchKernelGGL(k_dep_order, dim3(1), dim3(1024), 0, ctx->stream, (const unsigned long long*)pc,
+                                   (int)grid, (int32_t*)po);
+            }
+            if (int rc = check_launch(ctx, "k_dep_order")) return rc;
+            order = (const int32_t*)po;
+        }
+        {
+            TimedLaunch tl(ctx, asym ? "deposit_asym" : "deposit_cov");
+            const dim3 g((unsigned)grid, (unsigned)ns);
+            if (asym) hipLaunchKernelGGL(k_dep_gather<true>, g, dim3(kDepBlock), 0, ctx->stream, desc, offsets, order, a);
+            else hipLaunchKernelGGL(k_dep_gather<false>, g, dim3(kDepBlock), 0, ctx->stream, desc, offsets, order, a);
+        }
+        if (int rc = check_launch(ctx, "k_dep_gather")) return rc;
+        if (ns > 1) {
+            hipLaunchKernelGGL(k_dep_finish, dim3((unsigned)cdiv(cdiv(nx, psf::kStep) * ny * nt, kDepBlock)),
+                               dim3(kDepBlock), 0, ctx->stream, a, nt, ns);
+            if (int rc = check_launch(ctx, "k_dep_finish")) return rc;
+        }
     }
-    if (asym) {
-        TimedLaunch tl(ctx, "deposit_asym");
-        hipLaunchKernelGGL(k_dep_gather<true>, dim3((unsigned)grid), dim3(kDepBlock), 0, ctx->stream, desc, d_offsets,
-                           order, nx, ny, ncg, nblk, out32, out64, ld_out);
-    } else {
-        TimedLaunch tl(ctx, "deposit_cov");
-        hipLaunchKernelGGL(k_dep_gather<false>, dim3((unsigned)grid), dim3(kDepBlock), 0, ctx->stream, desc,
-                           d_offsets, order, nx, ny, ncg, nblk, out32, out64, ld_out);
-    }
-    return check_launch(ctx, "k_dep_gather");
+    return SFH_OK;
 }
 
 static int validate_ranges(sfh_ctx* ctx, sfh_range xe, sfh_range ye)

@@ -49,8 +49,23 @@ namespace sfh {
 namespace psf {
 
 constexpr float kSeriesEps = 0.1f;
-constexpr float kDeg1Eps = 0.026f;    // the Gaussian form below this half width
-constexpr float kDeg2Eps = 0.026f;    // (no degree-2 series: its range is the Gaussian form's)
+constexpr float kGaussEps = 0.026f;   // the Gaussian form below this half width
+// Covariant kernels in the Gaussian form: the row's three Gauss-Legendre nodes
+// merged into one node or two (set_row_nodes) up to these values of
+// h^2 (1 + 2 g^2), h = half row height / sigma_y
+constexpr double kOneNodeEta = 0.00135;
+constexpr double kTwoNodeEta = 0.03;
+// Wide kernels (merged Gaussian forms whose footprint spans the grid's width)
+// are evaluated on every kStep-th column only, and the sum over all of them is
+// interpolated to the columns between with kTaps-point Lagrange weights
+// (interp_weights).  A row of such a kernel is one Gaussian or two of the same
+// width sigma; the interpolation's largest error over all offsets is 2.0e-8 of
+// its peak for a step of sigma / 5 and 3.4e-9 for sigma / 6.  kStepDu: the
+// largest step in the scaled coordinate (where sigma = 0.849): sigma / 5.3.
+constexpr int kStep = 4;
+constexpr int kTaps = 10;
+constexpr int kLead = kTaps / 2 - 1;            // nodes before the first column
+constexpr double kStepDu = 0.16;
 constexpr double kGLNode = 0.7745966692414834;   // :303
 constexpr float kW0 = 0.5555555555555556f;      // :304
 constexpr float kW1 = 0.8888888888888888f;
@@ -58,9 +73,11 @@ constexpr double kLog2e = 1.4426950408889634;
 constexpr double kSqrtLog2e = 1.2011224087864498;
 constexpr int kCPT = 16;                        // consecutive columns evaluated per thread
 
-// x evaluation of a point: the erf difference, the Gaussian form, or the
-// series of degree 2..3
-enum : int32_t { kDirect = 0, kGauss = 1, kSeries2 = 2, kSeries3 = 3 };
+// Evaluation of a point: the erf difference, the Gaussian form (its rows'
+// Gauss-Legendre nodes one by one, or merged into one node or two), or the
+// series of degree 3
+// (kWide1, kWide2: the merged forms on every kStep-th column)
+enum : int32_t { kDirect = 0, kGauss = 1, kSeries3 = 3, kGauss1 = 4, kGauss2 = 5, kWide1 = 6, kWide2 = 7 };
 
 // One prepared kernel: the clipped footprint and its FP32 parameters.
 // Footprint indices are 0-based and inclusive; xa > xb marks "nothing to
@@ -76,12 +93,14 @@ struct alignas(16) PointDesc {
     float dv;     // t (or v) step per row
     float ey;     // covariant: GL node offset xi*hy/sy; asymmetric: half row width in v
     float pref;   // amplitude prefactor (see header), with the series form factors
-    float s0, s1, s2, s3;   // x series coefficients in w' (series kinds; kGauss: s0 = 1)
-    int32_t kind;           // kDirect, kGauss or kSeriesN for the x factor
-    float gf, gfi;          // kGauss, covariant: 2^(2 g ey du) and its inverse (the
-                            // outer GL nodes' strip multipliers relative to the middle node's)
+    float s0, s1, s2, s3;   // kSeries3: x series coefficients in w'; kGauss1 / kGauss2: a
+                            // row's y weight 2^(s1 t^2 +- s2 t) and the nodes' x shifts g t -+ s3
+    int32_t kind;
+    float gf, gfi;          // kGauss, covariant, and kGauss2: 2^(2 v du) and its inverse, v the x
+                            // distance of a row's outer nodes from its middle (g ey, or s3): the
+                            // nodes' strip multipliers relative to the middle's
     int32_t pad0;
-    float q[8];             // kGauss: q[j] = 2^-(du (j + 1/2))^2, the strip's column factors
+    float q[8];             // Gaussian forms: q[j] = 2^-(du (j + 1/2))^2, the strip's column factors
 };
 
 struct Range {
@@ -138,48 +157,153 @@ __host__ __device__ inline Series series_coeffs(float e)
     return s;
 }
 
-// The x-factor form of half width e (in u): its kind, and for the series
-// kinds the coefficients rescaled to w' = w log2(e) in d.
-__host__ __device__ inline void set_x_form(PointDesc* d, float e)
+// Nodes of a wide kernel's row on a grid of nx columns (node k at column
+// kStep (k - kLead)), and whether they take fewer strips than the columns.
+__host__ __device__ inline int wide_nodes(int nx) { return (nx + kStep - 1) / kStep + kTaps - 1; }
+__host__ __device__ inline bool wide_pays(int nx)
 {
+    return (wide_nodes(nx) + kCPT - 1) / kCPT < (nx + kCPT - 1) / kCPT;
+}
+
+// Lagrange weights of nodes -kLead .. kTaps - 1 - kLead at x = r / kStep.
+struct InterpWeights {
+    double w[kStep][kTaps];
+};
+__host__ __device__ constexpr InterpWeights interp_weights()
+{
+    InterpWeights t{};
+    for (int r = 0; r < kStep; ++r)
+        for (int i = 0; i < kTaps; ++i) {
+            double w = 1.0;
+            for (int j = 0; j < kTaps; ++j)
+                if (j != i) w *= ((double)r / kStep - (j - kLead)) / (double)(i - j);
+            t.w[r][i] = w;
+        }
+    return t;
+}
+
+// The strip constants of a Gaussian form with column step du and the rows'
+// outer nodes a coordinate distance v from the middle, from the rounded
+// values that the kernel uses (gauss_strip).
+__host__ __device__ inline void set_strip(PointDesc* d, double v)
+{
+    const double du = (double)d->du;
+    for (int j = 0; j < 8; ++j) {
+        const double sj = du * ((double)j + 0.5);
+        d->q[j] = (float)exp2(-sj * sj);
+    }
+    const double r = 2.0 * v * du;
+    d->gf = (float)exp2(r);
+    d->gfi = (float)exp2(-r);
+}
+
+// The x coordinates of a merged Gaussian form (ax, du: scaled), whose footprint
+// spans the nx columns: on the wide kernels' nodes where the kernel is smooth
+// enough, else on the columns.
+__host__ __device__ inline void set_merged_x(PointDesc* d, int32_t kind, double ax, double du, int nx)
+{
+    d->kind = kind;
+    if (wide_pays(nx) && fabs(kStep * du) <= kStepDu) {
+        d->kind = kind == kGauss1 ? kWide1 : kWide2;
+        du *= kStep;
+        ax -= kLead * du;
+    }
+    d->ax = (float)ax;
+    d->du = (float)du;
+    set_strip(d, (double)d->s3);
+}
+
+// A covariant kernel in the Gaussian form with its rows' Gauss-Legendre nodes
+// merged (only for a footprint that spans the grid's width); false where the
+// row is too high for that (the three nodes stay).
+// Around a row centre t, phi = t^2/2 + gam (u + g t)^2 (gam = 1 - b) has the
+// t-derivative s = k2 t + 2 gam g u, k2 = 1 + 2 gam g^2, and the three nodes at
+// t, t +- dl (dl = xi hy / sy) sum exactly to
+//   S exp(-phi) F(x),  F = 1 - p + p cosh x,  x = dl s,
+//   S = 8/9 + (10/9) exp(-dl^2 k2 / 2),  p = 1 - (8/9) / S.
+// One node: F = exp(p x^2 / 2), the x^2 joining the quadratic form, which
+// stays one Gaussian of a rescaled coordinate, shear and y weight.  The first
+// dropped term of ln F, 0.0154 x^4, is (h^2 k2 = eta) at most 0.012 eta^2 =
+// 2.2e-8 of the kernel's peak for eta < 0.00135: the bound of the Gaussian form
+// itself at its limit e = 0.026 (e^2 = eta / 2).
+// Two nodes: F = exp(al x^2) cosh(be x) with the x^2 and x^4 terms of ln F
+// (be^4 = (3 p^2 - p) / 2, al = p/2 - be^2/2): two Gaussians with the shifts
+// g' t -+ v.  Its first dropped term, 2.9e-4 x^6, is at most 6.6e-4 eta^3 =
+// 1.8e-8 of the peak for eta < 0.03.
+__host__ __device__ inline bool set_row_nodes(PointDesc* d, double ax, double du, double gam, double g, int nx)
+{
+    const double dl = (double)d->ey, k2 = 1.0 + 2.0 * gam * g * g;
+    const double eta = dl * dl * k2 / (kGLNode * kGLNode);
+    if (!(eta <= kTwoNodeEta)) return false;
+    const bool one = eta <= kOneNodeEta;
+    const double e2 = (10.0 / 9.0) * exp(-0.5 * dl * dl * k2);
+    const double S = 8.0 / 9.0 + e2, p = e2 / S;
+    const double be2 = one ? 0.0 : sqrt(0.5 * p * (3.0 * p - 1.0));
+    const double q = 0.5 * (p - be2) * dl * dl;            // the x^2 term's share in the exponent: q s^2
+    const double A = gam * (1.0 - 4.0 * q * gam * g * g);
+    const double g1 = gam * g * (1.0 - 2.0 * q * k2) / A;
+    const double rho = 0.5 + gam * g * g - q * k2 * k2 - A * g1 * g1;
+    const double scale = sqrt(A * kLog2e);
+    double v = 0.0, lam = 0.0, pre = S;
+    if (!one) {
+        const double bd = sqrt(be2) * dl;
+        v = bd * gam * g / A;
+        lam = bd * (k2 - 2.0 * gam * g * g1);
+        pre *= 0.5 * exp(A * v * v);
+    }
+    d->pref = (float)((double)d->pref * pre);
+    d->g = (float)(g1 * scale);
+    d->s1 = (float)(-rho * kLog2e);
+    d->s2 = (float)(lam * kLog2e);
+    d->s3 = (float)(v * scale);
+    set_merged_x(d, one ? kGauss1 : kGauss2, ax * scale, du * scale, nx);
+    return true;
+}
+
+// The form of a point with x coordinate ax of its first column, column step du
+// and half width d->ex (in u) on a grid of nx columns: its kind and, for the
+// series kinds, the coefficients rescaled to w' = w log2(e).  cov: a covariant
+// kernel of shear g; else an asymmetric one, whose y factor joins a merged
+// Gaussian form (one node, no shear) where it has the Gaussian form itself.
+__host__ __device__ inline void set_x_form(PointDesc* d, double ax, double du, bool cov, double g, int nx)
+{
+    const float e = d->ex;
+    double scale = kSqrtLog2e;
     if (!(e < kSeriesEps)) {
         d->kind = kDirect;
-        return;
-    }
-    d->kind = e < kDeg1Eps ? kGauss : e < kDeg2Eps ? kSeries2 : kSeries3;
-    const Series s = series_coeffs(e);
-    const double l1 = 1.0 / kLog2e, l2 = l1 * l1, l3 = l2 * l1;
-    double scale = kSqrtLog2e;
-    if (d->kind == kGauss) {
+        scale = 1.0;
+    } else if (e < kGaussEps) {
         // s0 exp(-(1 - b) w), b = s1 / s0: the coordinates carry sqrt(1 - b),
         // the amplitude s0
-        const double b = (double)s.s1 / (double)s.s0;
-        scale *= sqrt(1.0 - b);
+        const Series s = series_coeffs(e);
+        const double gam = 1.0 - (double)s.s1 / (double)s.s0;
+        d->kind = kGauss;
         d->pref = (float)((double)d->pref * (double)s.s0);
         d->s0 = 1.0f;
-        d->s1 = d->s2 = d->s3 = 0.0f;
+        scale *= sqrt(gam);
+        const bool full = e > 0.0f && d->xa == 0 && d->xb == nx - 1;
+        if (full && cov && set_row_nodes(d, ax, du, gam, g, nx)) return;
+        if (full && !cov && d->ey > 0.0f && d->ey < kGaussEps) {
+            const Series y = series_coeffs(d->ey);
+            d->pref = (float)((double)d->pref * (double)y.s0);
+            d->s1 = (float)(-(1.0 - (double)y.s1 / (double)y.s0) * kLog2e);
+            set_merged_x(d, kGauss1, ax * scale, du * scale, nx);
+            return;
+        }
     } else {
+        const Series s = series_coeffs(e);
+        const double l1 = 1.0 / kLog2e, l2 = l1 * l1, l3 = l2 * l1;
+        d->kind = kSeries3;
         d->s0 = s.s0;
         d->s1 = (float)(s.s1 * l1);
         d->s2 = (float)(s.s2 * l2);
         d->s3 = (float)(s.s3 * l3);
     }
     // coordinates of the series forms in a' = a sqrt(log2 e) (times sqrt(1 - b))
-    d->ax = (float)((double)d->ax * scale);
-    d->du = (float)((double)d->du * scale);
-    d->g = (float)((double)d->g * scale);
-    if (d->kind == kGauss) {
-        // the column factors of the strip recurrence (gauss_strip) and the
-        // outer nodes' multiplier ratios, from the rounded values the kernel uses
-        const double du = (double)d->du;
-        for (int j = 0; j < 8; ++j) {
-            const double sj = du * ((double)j + 0.5);
-            d->q[j] = (float)exp2(-sj * sj);
-        }
-        const double r = 2.0 * (double)d->g * (double)d->ey * du;
-        d->gf = (float)exp2(r);
-        d->gfi = (float)exp2(-r);
-    }
+    d->ax = (float)(ax * scale);
+    d->du = (float)(du * scale);
+    d->g = (float)(g * scale);
+    if (d->kind == kGauss) set_strip(d, (double)d->g * (double)d->ey);
 }
 
 // Covariant kernel centred at (x0, y0) (real units) -- addstar! :366-408.
@@ -216,17 +340,14 @@ __host__ __device__ inline int64_t prep_covariant(double x0, double y0, double s
     d.xb = (int32_t)(xb - 1);
     d.ya = (int32_t)(ya - 1);
     d.yb = (int32_t)(yb - 1);
-    d.ax = (float)((xs - x0) / s2x);
-    d.du = (float)(xst / s2x);
     d.ex = (float)(hx / s2x);
-    d.g = (float)(c * sy / s2x);
     d.ay = (float)((ys - y0) / sy);
     d.dv = (float)(yst / sy);
     d.ey = (float)(kGLNode * hy / sy);
     double pref = A * hy / (2.0 * 2.5066282746310002 * sy);          // prefac*h_y, :318,:323
     if (d.ex < kSeriesEps) pref *= 4.0 * hx / s2x / 1.7724538509055160;   // series form factor
     d.pref = (float)pref;
-    set_x_form(&d, d.ex);
+    set_x_form(&d, (xs - x0) / s2x, xst / s2x, true, c * sy / s2x, (int)nx);
     *out = d;
     return lx * ly;
 }
@@ -258,10 +379,7 @@ __host__ __device__ inline int64_t prep_asymmetric(double col, double mag, doubl
     d.xb = (int32_t)(xb - 1);
     d.ya = (int32_t)(ya - 1);
     d.yb = (int32_t)(yb - 1);
-    d.ax = (float)(((double)xa + 0.5 - x0) / s2x);                  // evaluate at i + 1/2 :361
-    d.du = (float)(1.0 / s2x);
     d.ex = (float)(0.5 / s2x);
-    d.g = 0.0f;
     d.ay = (float)(((double)ya + 0.5 - y0) / s2y);
     d.dv = (float)(1.0 / s2y);
     d.ey = (float)(0.5 / s2y);
@@ -269,7 +387,8 @@ __host__ __device__ inline int64_t prep_asymmetric(double col, double mag, doubl
     if (d.ex < kSeriesEps) pref *= 4.0 * (0.5 / s2x) / 1.7724538509055160;
     if (d.ey < kSeriesEps) pref *= 4.0 * (0.5 / s2y) / 1.7724538509055160;
     d.pref = (float)pref;
-    set_x_form(&d, d.ex);
+    // evaluate at i + 1/2 :361
+    set_x_form(&d, ((double)xa + 0.5 - x0) / s2x, 1.0 / s2x, false, 0.0, (int)nx);
     *out = d;
     return lx * ly;
 }
@@ -386,6 +505,25 @@ __host__ __device__ inline void cov_row_log(const PointDesc& d, int row, float* 
     h[2] = d.g * t2;
 }
 
+// The same for a row of merged nodes (kGauss1: one, kGauss2: two; see
+// set_row_nodes).
+template <int NODES>
+__host__ __device__ inline void merged_row(const PointDesc& d, int row, float* M, float* L, float* h)
+{
+    const float t = fmaf((float)(row - d.ya), d.dv, d.ay);
+    if constexpr (NODES == 1) {
+        M[0] = d.pref;
+        L[0] = d.s1 * t * t;
+        h[0] = d.g * t;
+    } else {
+        M[0] = M[1] = d.pref;
+        L[0] = fmaf(d.s1, t, d.s2) * t;
+        L[1] = fmaf(d.s1, t, -d.s2) * t;
+        h[0] = fmaf(d.g, t, -d.s3);
+        h[1] = fmaf(d.g, t, d.s3);
+    }
+}
+
 // c du + a for a compile-time column offset c.  On the device the offset is a
 // literal of v_fmamk_f32 (D = S0 K + S1, fused): written as a plain fmaf the
 // compiler keeps every column's offset in a register of its own (VOP3 takes no
@@ -442,23 +580,31 @@ __host__ __device__ __forceinline__ void gauss_strip(const PointDesc& d, const f
                                                      const float* h, int col0, float* part)
 {
     static_assert(kCPT == 16, "the recurrence runs 8 columns each way from the strip's middle");
-    static_assert(NODES == 1 || NODES == 3, "one node (asymmetric) or three GL nodes (covariant)");
+    static_assert(NODES >= 1 && NODES <= 3, "one node, two merged ones or three GL nodes");
     const float base = fmaf((float)(col0 - d.xa), d.du, d.ax);
     const int lo = d.xa - col0, hi = d.xb - col0;
     const float du = d.du;
-    constexpr int mid = NODES / 2;
     float pf[NODES], B[NODES], Bi[NODES];
+    float m0 = 0.0f;                       // the coordinate whose B is computed: the nodes' middle
 #pragma unroll
     for (int k = 0; k < NODES; ++k) {
         const float m = fmaf(7.5f, du, base + h[k]);
         pf[k] = M[k] * fast_exp2(L[k] - m * (m + du));
-        if (k == mid) {
-            const float md2 = 2.0f * m * du;
-            B[k] = fast_exp2(-md2);
-            Bi[k] = fast_exp2(md2);
-        }
+        if (NODES == 2 || k == NODES / 2) m0 += NODES == 2 ? 0.5f * m : m;
     }
-    if constexpr (NODES == 3) {
+    const float md2 = 2.0f * m0 * du;
+    const float Bm = fast_exp2(-md2), Bmi = fast_exp2(md2);
+    if constexpr (NODES == 1) {
+        B[0] = Bm;
+        Bi[0] = Bmi;
+    } else if constexpr (NODES == 2) {
+        B[0] = Bm * d.gf;
+        Bi[0] = Bmi * d.gfi;
+        B[1] = Bm * d.gfi;
+        Bi[1] = Bmi * d.gf;
+    } else {
+        B[1] = Bm;
+        Bi[1] = Bmi;
         B[0] = B[1] * d.gf;
         Bi[0] = Bi[1] * d.gfi;
         B[2] = B[1] * d.gfi;
@@ -499,7 +645,7 @@ template <int NODES, int DEG, bool MASK>
 __host__ __device__ __forceinline__ void add_strip(const PointDesc& d, const float* W, const float* h, int col0,
                                                    float* part)
 {
-    static_assert(DEG == kDirect || DEG == 2 || DEG == 3, "the Gaussian form is gauss_strip");
+    static_assert(DEG == kDirect || DEG == 3, "the Gaussian form is gauss_strip");
     const float base = fmaf((float)(col0 - d.xa), d.du, d.ax);
     const int lo = d.xa - col0, hi = d.xb - col0;
     const float du = d.du;
@@ -541,7 +687,7 @@ __host__ __device__ __forceinline__ void add_strip(const PointDesc& d, const flo
             c0[k] = W[k] * d.s0;
             c1[k] = W[k] * d.s1;
             c2[k] = W[k] * d.s2;
-            c3[k] = DEG >= 3 ? W[k] * d.s3 : 0.0f;
+            c3[k] = W[k] * d.s3;
         }
         static_for<0, kCPT>([&](auto cc) {
             constexpr int c = decltype(cc)::value;
@@ -550,9 +696,7 @@ __host__ __device__ __forceinline__ void add_strip(const PointDesc& d, const flo
             for (int k = 0; k < NODES; ++k) {
                 const float a = col_fma<c>(du, a0[k]);
                 const float w = a * a;
-                float S;
-                if constexpr (DEG == 2) S = fmaf(fmaf(c2[k], w, c1[k]), w, c0[k]);
-                else S = fmaf(fmaf(fmaf(c3[k], w, c2[k]), w, c1[k]), w, c0[k]);
+                const float S = fmaf(fmaf(fmaf(c3[k], w, c2[k]), w, c1[k]), w, c0[k]);
                 v = fmaf(S, fast_exp2(-w), v);
             }
             if (MASK) masked_set(part[c], v, c >= lo && c <= hi);
@@ -574,21 +718,29 @@ __host__ __device__ inline float direct_edge(const PointDesc& d, int l, float h)
     return fmaf((float)l, d.du, d.ax - d.ex) + h;
 }
 
-// One point's contributions to one row's strip, dispatched on its form.
-template <int NODES, bool MASK>
-__host__ __device__ __forceinline__ void add_point(const PointDesc& d, const float* W, const float* h, int col0,
-                                                   float* part)
+// One point's contributions to one row's strip, dispatched on its form (any but
+// the merged ones).  COV: the covariant kernel (else the asymmetric one).
+template <bool COV, bool MASK>
+__host__ __device__ __forceinline__ void add_point(const PointDesc& d, int row, int col0, float* part)
 {
-    switch (d.kind) {
-    case kGauss: {
-        const float L[NODES] = {};
-        gauss_strip<NODES, MASK>(d, W, L, h, col0, part);
-        break;
+    constexpr int NODES = COV ? 3 : 1;
+    float W[NODES], L[NODES] = {}, h[NODES] = {};
+    if constexpr (COV) {
+        if (d.kind == kGauss) {
+            cov_row_log(d, row, W, L, h);
+            gauss_strip<3, MASK>(d, W, L, h, col0, part);
+            return;
+        }
+        cov_row(d, row, W, h);
+    } else {
+        W[0] = d.pref * y_factor(fmaf((float)(row - d.ya), d.dv, d.ay), d.ey);
+        if (d.kind == kGauss) {
+            gauss_strip<1, MASK>(d, W, L, h, col0, part);
+            return;
+        }
     }
-    case kSeries2: add_strip<NODES, 2, MASK>(d, W, h, col0, part); break;
-    case kSeries3: add_strip<NODES, 3, MASK>(d, W, h, col0, part); break;
-    default: add_strip<NODES, kDirect, MASK>(d, W, h, col0, part); break;
-    }
+    if (d.kind == kSeries3) add_strip<NODES, 3, MASK>(d, W, h, col0, part);
+    else add_strip<NODES, kDirect, MASK>(d, W, h, col0, part);
 }
 
 }  // namespace psf
