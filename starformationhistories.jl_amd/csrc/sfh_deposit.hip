@@ -190,7 +190,7 @@ __global__ __launch_bounds__(kDepBlock) __attribute__((amdgpu_waves_per_eu(4))) 
         if (!(valid && row >= d.ya && row <= d.yb)) return;
         float M[NODES], L[NODES], h[NODES];
         psf::merged_row<NODES>(d, row, M, L, h);
-        psf::gauss_strip<NODES, false>(d, M, L, h, col0, part);
+        psf::gauss_strip<NODES>(d, M, L, h, col0, part);
     };
     Foot fn = footprint(td, c0 * kChunk + lane, np);
     for (int ch = c0; ch < c1; ++ch) {
@@ -300,43 +300,49 @@ __global__ __launch_bounds__(kDepBlock) __attribute__((amdgpu_waves_per_eu(4))) 
         float M[NODES], L[NODES] = {}, h[NODES] = {};
         if constexpr (N == 0) M[0] = d.pref * psf::y_factor(fmaf((float)(row - d.ya), d.dv, d.ay), d.ey);
         else psf::merged_row<NODES>(d, row, M, L, h);
-        psf::gauss_strip<NODES, false>(d, M, L, h, col0, part);
+        psf::gauss_strip<NODES>(d, M, L, h, col0, part);
     };
     auto add = [&](const PointDesc& d) {
         if (!in_rows(d) || col0 > d.xb || col0 + kCPT - 1 < d.xa) return;
-        psf::add_point<!kAsym, true>(d, row, col0, part);
+        psf::add_point<!kAsym>(d, row, col0, part);
     };
-    // A point in the erf-difference form (a narrow kernel: its footprint is at
-    // most 55 columns wide) with the whole wave cooperating, instead of the
+    // A point in the erf-difference form (a kernel so narrow that its footprint
+    // is at most 37 columns wide) with the whole wave cooperating, instead of
     // strip code in which only the few lanes whose strips meet the footprint
-    // would work: lane l takes footprint column xa + l, the point's rows inside
-    // this wave's strips one after another; lanes 0 .. nc evaluate erfc at
-    // their column's left edge and a column's right edge is the next lane's.
-    // Each bin's value (nodes summed in order, in FP32) is added to its
-    // owner's FP64 accumulator in LDS: the bins are distinct, so no two lanes
-    // write one word, and the owner's own flush comes later in program order.
+    // would work: segments of 16, 32 or 64 lanes take one of the point's rows
+    // inside this wave's strips each, lane l of a segment footprint column
+    // xa + l; lanes 0 .. nc evaluate erfc at their column's left edge (its sign
+    // that of the edge) and a column's right edge is the next lane's.  Each
+    // bin's value (nodes summed in order, in FP32) is added to its owner's
+    // FP64 accumulator in LDS: the bins are distinct, so no two lanes write one
+    // word, and the owner's own flush comes later in program order.
     auto direct = [&](const PointDesc& d) {
         constexpr int NODES = kAsym ? 1 : 3;
         const int nc = d.xb - d.xa + 1;
+        const int lw = nc < 16 ? 4 : nc < 32 ? 5 : 6;          // nc + 1 edges per segment
+        const int l = lane & ((1 << lw) - 1);
         const int r0 = d.ya > row_lo ? d.ya : row_lo, r1 = d.yb < row_hi ? d.yb : row_hi;
-        for (int r = r0; r <= r1; ++r) {
+        for (int rp = r0; rp <= r1; rp += 64 >> lw) {
+            const int r = rp + (lane >> lw);
             float W[3], h[3] = {0.0f, 0.0f, 0.0f};
             if constexpr (kAsym) W[0] = d.pref * psf::y_factor(fmaf((float)(r - d.ya), d.dv, d.ay), d.ey);
             else psf::cov_row(d, r, W, h);
             float v = 0.0f;
 #pragma unroll
             for (int k = 0; k < NODES; ++k) {
-                const float b = psf::direct_edge(d, lane, h[k]);
-                const float e = psf::erfc_pos(fabsf(b));
-                const int n = b < 0.0f ? 1 : 0;
-                const float e1 = __shfl_down(e, 1, 64);
-                const int n1 = __shfl_down(n, 1, 64);
-                v = fmaf(W[k], psf::erf_diff(e, n != 0, e1, n1 != 0), v);
+                const float e = psf::signed_erfc(psf::direct_edge(d, l, h[k]));
+                // the next lane's value (wave_shl:1)
+                const float e1 = __int_as_float(
+                    __builtin_amdgcn_update_dpp(0, __float_as_int(e), 0x130, 0xf, 0xf, false));
+                v = fmaf(W[k], psf::erf_diff(e, e1), v);
             }
-            if (lane < nc) {
-                const int col = d.xa + lane;
+            if (l < nc && r <= r1) {
+                const int col = d.xa + l;
                 const int o = r * ncg + col / kCPT - wslot;
-                if (o >= 0 && o < 64) sacc[col % kCPT][wave_id * 64 + o] += (double)v;
+                if (o >= 0 && o < 64) {
+                    lds_double* p = &sacc[col % kCPT][wave_id * 64 + o];
+                    *p = *p + (double)v;
+                }
             }
         }
     };
@@ -354,8 +360,7 @@ __global__ __launch_bounds__(kDepBlock) __attribute__((amdgpu_waves_per_eu(4))) 
         const PointDesc* __restrict__ chunk = td + ch * kChunk;
         each(chunk, h1, [&](const PointDesc& d) { add_common(d, std::integral_constant<int, 1>{}); });
         each(chunk, h2, [&](const PointDesc& d) { add_common(d, std::integral_constant<int, kAsym ? 0 : 2>{}); });
-        // the narrow erf-difference kernels go to the wave-cooperative path
-        const uint64_t h3 = __ballot(hit && f.kind == psf::kDirect && f.f.y - f.f.x < 63);
+        const uint64_t h3 = __ballot(hit && f.kind == psf::kDirect);
         each(chunk, all & ~(h1 | h2 | h3), add);
         each(chunk, h3, direct);
 #pragma unroll
@@ -408,7 +413,7 @@ __device__ inline unsigned form_cost(int kind, bool full)
     if (kind == psf::kGauss1) return 2u;
     if (kind == psf::kGauss2) return 4u;
     if (kind == psf::kGauss) return full ? 5u : 6u;
-    if (kind == psf::kSeries3) return 12u;
+    if (kind == psf::kSum) return 10u;
     return 32u;
 }
 

@@ -16,27 +16,21 @@
 //                with t_k = (y_j + xi_k hy - y0)/sy (3-point Gauss-Legendre, :303-304),
 //                g = c sy / (sqrt(2) sx)  (the reference's Δx = dx + c Δy, :328);
 //   asymmetric : A/4 * D(u_i, ex) * D(v_j, ey)  (:203-204; the two sign flips cancel).
-// For e < kSeriesEps, D is evaluated without the erf-difference cancellation:
-//   D = (4 e / sqrt(pi)) exp(-u^2) S(u^2),  S(w) = sum_n H_2n(sqrt w) e^2n / (2n+1)!
-// (the mean of exp(-(u+s)^2) over |s| < e; Hermite polynomials H_2n), whose
-// coefficients in powers of w are kept up to w^3.  Relative to the local
-// value at |u| <= 4 the dropped terms are below ~1e-7 when e < 0.1 (the
-// terms of order e^2n |H_2n(4)| / (2n+1)! are ~10 e^2, 28 e^4, 30 e^6, 15 e^8).
-// For e < 0.026 the factor is kept in the exponent instead (the Gaussian
-// form): s0 + s1 w = s0 exp(b w) (1 + O(b^2 w^2)), b = s1 / s0 = 2e^2/3 +
-// O(e^4), so D = (4 e / sqrt(pi)) s0 exp(-(1 - b) w), one Gaussian of a
-// rescaled coordinate.  ln S(w) = ln s0 + b w - (4/45) e^4 w^2 + ..., so the
-// dropped term is (4/45) e^4 w^2 relative to the local value: <= 1.1e-5 at
-// |u| = 4 for e < 0.026 (below 8e-8 for e < 0.0077, and always below the
-// degree-1 polynomial's own truncation error (2/15) e^4 w^2); relative to
-// the kernel's peak it is at most (4/45) e^4 max(w^2 e^-w) = 0.048 e^4,
-// below 2.2e-8, under the FP32 rounding of the sums.  On the 700-template
-// workload 97% of the pairs take this form.
-//
-// The series forms run in scaled coordinates a' = a sqrt(log2 e) (the
-// Gaussian form: a sqrt((1 - b) log2 e)), so exp(-a^2) = exp2(-a'^2) is one
-// hardware exp2, with the coefficients of S rescaled to w' = a'^2.  The direct form shares erf values between adjacent
-// columns: the right edge of column c is the left edge of column c + 1.
+// For e < kSumEps, D is evaluated without the erf-difference cancellation as
+//   D = (4 e / sqrt(pi)) <exp(-(u+s)^2)>, the mean over |s| < e:
+// e < 0.026, the Gaussian form: the mean is exp(-u^2) S(u^2), S(w) =
+//   sum_n H_2n(sqrt w) e^2n / (2n+1)! = s0 exp(b w) (1 + O(b^2 w^2)), b = s1 / s0
+//   = 2e^2/3 + O(e^4), so D = (4 e / sqrt(pi)) s0 exp(-(1 - b) u^2), one Gaussian
+//   of a rescaled coordinate.  ln S(w) = ln s0 + b w - (4/45) e^4 w^2 + ..., so the
+//   dropped term is (4/45) e^4 w^2 relative to the local value: <= 1.1e-5 at
+//   |u| = 4 for e < 0.026; relative to the kernel's peak it is at most
+//   (4/45) e^4 max(w^2 e^-w) = 0.048 e^4, below 2.2e-8, under the FP32 rounding of
+//   the sums.  On the 700-template workload 97% of the pairs take this form.
+// 0.026 <= e < kSumEps, the sum form: the mean as two Gaussians (e < kPairEps),
+//   whose first wrong term of ln is 3e-5 (2 u e)^6, at most 2.6e-3 e^6 of the
+//   peak, or three, with 1.4e-7 (2 u e)^8, at most 1.7e-4 e^8 (set_sum).
+// Both run in scaled coordinates a = u sqrt(log2 e) times the square root of
+// their Gaussian's own factor, so a Gaussian is one hardware exp2 of -a^2.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -48,7 +42,9 @@
 namespace sfh {
 namespace psf {
 
-constexpr float kSeriesEps = 0.1f;
+constexpr float kSeriesEps = 0.1f;    // an asymmetric kernel's y factor as a series below this half height
+constexpr float kPairEps = 0.06f;     // x: the sum form's two Gaussians below this half width, three above
+constexpr float kSumEps = 0.2f;       // the sum form below, erf differences above
 constexpr float kGaussEps = 0.026f;   // the Gaussian form below this half width
 // Covariant kernels in the Gaussian form: the row's three Gauss-Legendre nodes
 // merged into one node or two (set_row_nodes) up to these values of
@@ -70,19 +66,17 @@ constexpr double kGLNode = 0.7745966692414834;   // :303
 constexpr float kW0 = 0.5555555555555556f;      // :304
 constexpr float kW1 = 0.8888888888888888f;
 constexpr double kLog2e = 1.4426950408889634;
-constexpr double kSqrtLog2e = 1.2011224087864498;
 constexpr int kCPT = 16;                        // consecutive columns evaluated per thread
 
 // Evaluation of a point: the erf difference, the Gaussian form (its rows'
 // Gauss-Legendre nodes one by one, or merged into one node or two), or the
-// series of degree 3
-// (kWide1, kWide2: the merged forms on every kStep-th column)
-enum : int32_t { kDirect = 0, kGauss = 1, kSeries3 = 3, kGauss1 = 4, kGauss2 = 5, kWide1 = 6, kWide2 = 7 };
+// sum form (kWide1, kWide2: the merged forms on every kStep-th column)
+enum : int32_t { kDirect = 0, kGauss = 1, kSum = 2, kGauss1 = 3, kGauss2 = 4, kWide1 = 5, kWide2 = 6 };
 
 // One prepared kernel: the clipped footprint and its FP32 parameters.
 // Footprint indices are 0-based and inclusive; xa > xb marks "nothing to
 // deposit" (the reference's length>1 guard, :359 / :401).
-// Series kinds store ax, du and g in the scaled coordinate a' (see header).
+// All kinds but kDirect store ax, du and g in a scaled coordinate (see header).
 struct alignas(16) PointDesc {
     int32_t xa, xb, ya, yb;
     float ax;     // x coordinate of the first footprint column centre
@@ -93,12 +87,14 @@ struct alignas(16) PointDesc {
     float dv;     // t (or v) step per row
     float ey;     // covariant: GL node offset xi*hy/sy; asymmetric: half row width in v
     float pref;   // amplitude prefactor (see header), with the series form factors
-    float s0, s1, s2, s3;   // kSeries3: x series coefficients in w'; kGauss1 / kGauss2: a
-                            // row's y weight 2^(s1 t^2 +- s2 t) and the nodes' x shifts g t -+ s3
+    float s1, s2, s3;       // kGauss1 / kGauss2: a row's y weight 2^(s1 t^2 +- s2 t) and the
+                            // nodes' x shifts g t -+ s3; kSum: the outer Gaussians' x shifts
+                            // -+ s3 and the middle one's amplitude s1 over theirs
     int32_t kind;
     float gf, gfi;          // kGauss, covariant, and kGauss2: 2^(2 v du) and its inverse, v the x
                             // distance of a row's outer nodes from its middle (g ey, or s3): the
                             // nodes' strip multipliers relative to the middle's
+    int32_t terms;          // kGauss: 1; kSum: 2 or 3 Gaussians
     int32_t pad0;
     float q[8];             // Gaussian forms: q[j] = 2^-(du (j + 1/2))^2, the strip's column factors
 };
@@ -260,50 +256,77 @@ __host__ __device__ inline bool set_row_nodes(PointDesc* d, double ax, double du
     return true;
 }
 
+// The sum form of half column width e.  With r = 2u, the mean over the column is
+//   <exp(-(u+s)^2)> = exp(-u^2) Z exp(k2 r^2 / 2 + k4 r^4 / 24 + k6 r^6 / 720 + ...),
+// Z the mean and k_n the cumulants of s under the weight exp(-s^2) on |s| < e.
+// exp(a r^2) (1 - P + P cosh(b r)) has the cumulants 2a + P b^2, P (1 - 3P) b^4 and
+// P (1 - 15 P + 30 P^2) b^6.  P = 1 (two Gaussians) with b and a from k4 and k2
+// leaves k6 off by 0.08 of its value for the uniform weight, 16 e^6 / 63; P =
+// 0.63747 (three) gives that value too, and its k8 to half a percent.
+__host__ __device__ inline void set_sum(PointDesc* d, double ax, double du, double g)
+{
+    const double e = (double)d->ex;
+    // the moments by 5-point Gauss-Legendre quadrature (exact to e^10)
+    constexpr double x1 = 0.5384693101056831, x2 = 0.9061798459386640;
+    constexpr double w0 = 0.2844444444444444, w1 = 0.2393143352496832, w2 = 0.1184634425280945;
+    const double s1 = e * e * x1 * x1, s2 = e * e * x2 * x2;
+    const double f1 = 2.0 * w1 * exp(-s1), f2 = 2.0 * w2 * exp(-s2);
+    const double Z = w0 + f1 + f2;
+    const double m2 = (f1 * s1 + f2 * s2) / Z, k4 = (f1 * s1 * s1 + f2 * s2 * s2) / Z - 3.0 * m2 * m2;
+    const double P = d->ex < kPairEps ? 1.0 : 0.63747;
+    const double b2 = sqrt(k4 / (P * (1.0 - 3.0 * P)));
+    // exp(-u^2 + a r^2 -+ b r) = exp(b^2 / gam) exp(-gam (u +- b / gam)^2), gam = 1 - 4a
+    const double gam = 1.0 - 2.0 * (m2 - P * b2), scale = sqrt(gam * kLog2e);
+    const double grow = exp(b2 / gam);
+    d->kind = kSum;
+    d->terms = P < 1.0 ? 3 : 2;
+    d->pref = (float)((double)d->pref * Z * 0.5 * P * grow);
+    d->s1 = (float)(2.0 * (1.0 - P) / (P * grow));
+    d->s3 = (float)(sqrt(b2) / gam * scale);
+    d->ax = (float)(ax * scale);
+    d->du = (float)(du * scale);
+    d->g = (float)(g * scale);
+    set_strip(d, (double)d->g * (double)d->ey);
+}
+
 // The form of a point with x coordinate ax of its first column, column step du
-// and half width d->ex (in u) on a grid of nx columns: its kind and, for the
-// series kinds, the coefficients rescaled to w' = w log2(e).  cov: a covariant
+// and half width d->ex (in u) on a grid of nx columns.  cov: a covariant
 // kernel of shear g; else an asymmetric one, whose y factor joins a merged
 // Gaussian form (one node, no shear) where it has the Gaussian form itself.
 __host__ __device__ inline void set_x_form(PointDesc* d, double ax, double du, bool cov, double g, int nx)
 {
     const float e = d->ex;
-    double scale = kSqrtLog2e;
-    if (!(e < kSeriesEps)) {
+    if (!(e < kSumEps)) {
         d->kind = kDirect;
-        scale = 1.0;
-    } else if (e < kGaussEps) {
-        // s0 exp(-(1 - b) w), b = s1 / s0: the coordinates carry sqrt(1 - b),
-        // the amplitude s0
-        const Series s = series_coeffs(e);
-        const double gam = 1.0 - (double)s.s1 / (double)s.s0;
-        d->kind = kGauss;
-        d->pref = (float)((double)d->pref * (double)s.s0);
-        d->s0 = 1.0f;
-        scale *= sqrt(gam);
-        const bool full = e > 0.0f && d->xa == 0 && d->xb == nx - 1;
-        if (full && cov && set_row_nodes(d, ax, du, gam, g, nx)) return;
-        if (full && !cov && d->ey > 0.0f && d->ey < kGaussEps) {
-            const Series y = series_coeffs(d->ey);
-            d->pref = (float)((double)d->pref * (double)y.s0);
-            d->s1 = (float)(-(1.0 - (double)y.s1 / (double)y.s0) * kLog2e);
-            set_merged_x(d, kGauss1, ax * scale, du * scale, nx);
-            return;
-        }
-    } else {
-        const Series s = series_coeffs(e);
-        const double l1 = 1.0 / kLog2e, l2 = l1 * l1, l3 = l2 * l1;
-        d->kind = kSeries3;
-        d->s0 = s.s0;
-        d->s1 = (float)(s.s1 * l1);
-        d->s2 = (float)(s.s2 * l2);
-        d->s3 = (float)(s.s3 * l3);
+        d->ax = (float)ax;
+        d->du = (float)du;
+        d->g = (float)g;
+        return;
     }
-    // coordinates of the series forms in a' = a sqrt(log2 e) (times sqrt(1 - b))
+    if (e >= kGaussEps) {
+        set_sum(d, ax, du, g);
+        return;
+    }
+    // s0 exp(-(1 - b) w), b = s1 / s0: the coordinates carry sqrt(1 - b), the
+    // amplitude s0
+    const Series s = series_coeffs(e);
+    const double gam = 1.0 - (double)s.s1 / (double)s.s0, scale = sqrt(gam * kLog2e);
+    d->kind = kGauss;
+    d->terms = 1;
+    d->pref = (float)((double)d->pref * (double)s.s0);
+    const bool full = e > 0.0f && d->xa == 0 && d->xb == nx - 1;
+    if (full && cov && set_row_nodes(d, ax, du, gam, g, nx)) return;
+    if (full && !cov && d->ey > 0.0f && d->ey < kGaussEps) {
+        const Series y = series_coeffs(d->ey);
+        d->pref = (float)((double)d->pref * (double)y.s0);
+        d->s1 = (float)(-(1.0 - (double)y.s1 / (double)y.s0) * kLog2e);
+        set_merged_x(d, kGauss1, ax * scale, du * scale, nx);
+        return;
+    }
     d->ax = (float)(ax * scale);
     d->du = (float)(du * scale);
     d->g = (float)(g * scale);
-    if (d->kind == kGauss) set_strip(d, (double)d->g * (double)d->ey);
+    set_strip(d, (double)d->g * (double)d->ey);
 }
 
 // Covariant kernel centred at (x0, y0) (real units) -- addstar! :366-408.
@@ -345,7 +368,7 @@ __host__ __device__ inline int64_t prep_covariant(double x0, double y0, double s
     d.dv = (float)(yst / sy);
     d.ey = (float)(kGLNode * hy / sy);
     double pref = A * hy / (2.0 * 2.5066282746310002 * sy);          // prefac*h_y, :318,:323
-    if (d.ex < kSeriesEps) pref *= 4.0 * hx / s2x / 1.7724538509055160;   // series form factor
+    if (d.ex < kSumEps) pref *= 4.0 * hx / s2x / 1.7724538509055160;   // series form factor
     d.pref = (float)pref;
     set_x_form(&d, (xs - x0) / s2x, xst / s2x, true, c * sy / s2x, (int)nx);
     *out = d;
@@ -384,7 +407,7 @@ __host__ __device__ inline int64_t prep_asymmetric(double col, double mag, doubl
     d.dv = (float)(1.0 / s2y);
     d.ey = (float)(0.5 / s2y);
     double pref = A / 4.0;
-    if (d.ex < kSeriesEps) pref *= 4.0 * (0.5 / s2x) / 1.7724538509055160;
+    if (d.ex < kSumEps) pref *= 4.0 * (0.5 / s2x) / 1.7724538509055160;
     if (d.ey < kSeriesEps) pref *= 4.0 * (0.5 / s2y) / 1.7724538509055160;
     d.pref = (float)pref;
     // evaluate at i + 1/2 :361
@@ -449,11 +472,13 @@ __host__ __device__ inline float erfc_pos(float x)
     return t * fast_exp(fmaf(-x, x, p));
 }
 
-// erf(b1) - erf(b0) of a column from e = erfc(|b|) and the sign of its two
-// edges: both >= 0: e0 - e1; both < 0: e1 - e0; across 0: 2 - e1 - e0
-__host__ __device__ inline float erf_diff(float e0, bool n0, float e1, bool n1)
+// erfc(|b|) with the sign of b, and erf(b1) - erf(b0) of a column from its two
+// edges' values: both >= 0: e0 - e1; both < 0: |e1| - |e0|; across 0: 2 - |e1| - |e0|
+__host__ __device__ inline float signed_erfc(float b) { return copysignf(erfc_pos(fabsf(b)), b); }
+__host__ __device__ inline float erf_diff(float e0, float e1)
 {
-    return n1 ? e1 - e0 : (n0 ? 2.0f - e1 - e0 : e0 - e1);
+    const float d = e0 - e1;
+    return __builtin_signbitf(e0) && !__builtin_signbitf(e1) ? 2.0f + d : d;
 }
 
 // erf(u + e) - erf(u - e) through erfc of non-negative arguments (D is even
@@ -524,22 +549,6 @@ __host__ __device__ inline void merged_row(const PointDesc& d, int row, float* M
     }
 }
 
-// c du + a for a compile-time column offset c.  On the device the offset is a
-// literal of v_fmamk_f32 (D = S0 K + S1, fused): written as a plain fmaf the
-// compiler keeps every column's offset in a register of its own (VOP3 takes no
-// literal), which costs the kernel sixteen registers.
-template <int C>
-__host__ __device__ __forceinline__ float col_fma(float du, float a)
-{
-#if defined(__HIP_DEVICE_COMPILE__)
-    float r;
-    asm("v_fmamk_f32 %0, %1, %2, %3" : "=v"(r) : "v"(du), "i"(__builtin_bit_cast(int, (float)C)), "v"(a));
-    return r;
-#else
-    return fmaf((float)C, du, a);
-#endif
-}
-
 // part = in ? v : part, as a select: v is computed for every lane first (the
 // register barrier keeps the compiler from sinking its computation into a
 // branch per column, which serialises the columns' dependency chains)
@@ -575,14 +584,13 @@ __host__ __device__ __forceinline__ void static_for(F&& f)
 // steps.  The Gaussian form has du < 0.064 (half bin width e < 0.026), so B
 // stays within [2^-2, 2^2] for |m| < 15.  Each column adds the nodes in order
 // k = 0, 1, 2.
-template <int NODES, bool MASK>
+template <int NODES>
 __host__ __device__ __forceinline__ void gauss_strip(const PointDesc& d, const float* M, const float* L,
                                                      const float* h, int col0, float* part)
 {
     static_assert(kCPT == 16, "the recurrence runs 8 columns each way from the strip's middle");
     static_assert(NODES >= 1 && NODES <= 3, "one node, two merged ones or three GL nodes");
     const float base = fmaf((float)(col0 - d.xa), d.du, d.ax);
-    const int lo = d.xa - col0, hi = d.xb - col0;
     const float du = d.du;
     float pf[NODES], B[NODES], Bi[NODES];
     float m0 = 0.0f;                       // the coordinate whose B is computed: the nodes' middle
@@ -617,95 +625,12 @@ __host__ __device__ __forceinline__ void gauss_strip(const PointDesc& d, const f
         static_for<0, 8>([&](auto jj) {
             constexpr int j = decltype(jj)::value;
             constexpr int cf = 8 + j, cb = 7 - j;
-            const float vf = fmaf(f, d.q[j], part[cf]);
-            const float vb = fmaf(b, d.q[j], part[cb]);
-            if (MASK) {
-                masked_set(part[cf], vf, cf >= lo && cf <= hi);
-                masked_set(part[cb], vb, cb >= lo && cb <= hi);
-            } else {
-                part[cf] = vf;
-                part[cb] = vb;
-            }
+            part[cf] = fmaf(f, d.q[j], part[cf]);
+            part[cb] = fmaf(b, d.q[j], part[cb]);
             if constexpr (j < 7) {
                 f *= Bk;
                 b *= Bik;
             }
-        });
-    }
-}
-
-// Adds the contributions of one point to the kCPT columns col0 .. col0+kCPT-1
-// of one row: part[c] += sum_k W[k] X(a_k(c)), a_k(c) the x coordinate of
-// column col0 + c shifted by h[k] (NODES = 3: covariant GL nodes; NODES = 1:
-// asymmetric, W[0] = pref * y factor).  DEG: the x form (kDirect or a series
-// degree 2, 3).  MASK: only columns inside [xa, xb] receive anything (without
-// it every column does: the footprint spans the whole grid and columns past
-// the grid are never written).  Each column adds the nodes in order.
-template <int NODES, int DEG, bool MASK>
-__host__ __device__ __forceinline__ void add_strip(const PointDesc& d, const float* W, const float* h, int col0,
-                                                   float* part)
-{
-    static_assert(DEG == kDirect || DEG == 3, "the Gaussian form is gauss_strip");
-    const float base = fmaf((float)(col0 - d.xa), d.du, d.ax);
-    const int lo = d.xa - col0, hi = d.xb - col0;
-    const float du = d.du;
-    if constexpr (DEG == kDirect) {
-        // erf at the column edges b(c) = a(c) - ex, c = 0..kCPT, as erfc(|b|) so
-        // that D(c) = erf(b(c+1)) - erf(b(c)) keeps its relative accuracy in
-        // the tails: both edges >= 0: erfc(b0) - erfc(b1); both < 0:
-        // erfc(-b1) - erfc(-b0); across 0: 2 - erfc(b1) - erfc(-b0).  Node by
-        // node (each column still adds the nodes in order), so that one
-        // node's edge values are live at a time.
-#pragma unroll
-        for (int k = 0; k < NODES; ++k) {
-            const float b0 = base + h[k] - d.ex;
-            bool pneg = b0 < 0.0f;
-            float prev = erfc_pos(fabsf(b0));
-            static_for<0, kCPT>([&](auto cc) {
-                constexpr int c = decltype(cc)::value;
-                const float b1 = col_fma<c + 1>(du, b0);
-                const bool neg = b1 < 0.0f;
-                const float e1 = erfc_pos(fabsf(b1));
-                const float dd = erf_diff(prev, pneg, e1, neg);
-                const float v = fmaf(W[k], dd, part[c]);
-                if (MASK) masked_set(part[c], v, c >= lo && c <= hi);
-                else part[c] = v;
-                prev = e1;
-                pneg = neg;
-#if defined(__HIP_DEVICE_COMPILE__)
-                // one column at a time: interleaving the columns' erfc sequences
-                // would raise the register count of the whole kernel
-                __builtin_amdgcn_sched_barrier(0);
-#endif
-            });
-        }
-    } else {
-        float a0[NODES], c0[NODES], c1[NODES], c2[NODES], c3[NODES];
-#pragma unroll
-        for (int k = 0; k < NODES; ++k) {
-            a0[k] = base + h[k];
-            c0[k] = W[k] * d.s0;
-            c1[k] = W[k] * d.s1;
-            c2[k] = W[k] * d.s2;
-            c3[k] = W[k] * d.s3;
-        }
-        static_for<0, kCPT>([&](auto cc) {
-            constexpr int c = decltype(cc)::value;
-            float v = part[c];
-#pragma unroll
-            for (int k = 0; k < NODES; ++k) {
-                const float a = col_fma<c>(du, a0[k]);
-                const float w = a * a;
-                const float S = fmaf(fmaf(fmaf(c3[k], w, c2[k]), w, c1[k]), w, c0[k]);
-                v = fmaf(S, fast_exp2(-w), v);
-            }
-            if (MASK) masked_set(part[c], v, c >= lo && c <= hi);
-            else part[c] = v;
-#if defined(__HIP_DEVICE_COMPILE__)
-            // columns in groups of four: enough independent work per wave, without
-            // every column's temporaries live at once
-            if constexpr ((c & 3) == 3) __builtin_amdgcn_sched_barrier(0);
-#endif
         });
     }
 }
@@ -718,29 +643,32 @@ __host__ __device__ inline float direct_edge(const PointDesc& d, int l, float h)
     return fmaf((float)l, d.du, d.ax - d.ex) + h;
 }
 
-// One point's contributions to one row's strip, dispatched on its form (any but
-// the merged ones).  COV: the covariant kernel (else the asymmetric one).
-template <bool COV, bool MASK>
+// A point in the Gaussian form (its rows' nodes not merged) or the sum form on
+// one row's strip, only columns inside its footprint receiving anything.  COV:
+// the covariant kernel (else the asymmetric one).  The sum form's Gaussians
+// are one loop over the same code.
+template <bool COV>
 __host__ __device__ __forceinline__ void add_point(const PointDesc& d, int row, int col0, float* part)
 {
     constexpr int NODES = COV ? 3 : 1;
-    float W[NODES], L[NODES] = {}, h[NODES] = {};
-    if constexpr (COV) {
-        if (d.kind == kGauss) {
-            cov_row_log(d, row, W, L, h);
-            gauss_strip<3, MASK>(d, W, L, h, col0, part);
-            return;
-        }
-        cov_row(d, row, W, h);
-    } else {
-        W[0] = d.pref * y_factor(fmaf((float)(row - d.ya), d.dv, d.ay), d.ey);
-        if (d.kind == kGauss) {
-            gauss_strip<1, MASK>(d, W, L, h, col0, part);
-            return;
-        }
+    float M[NODES], L[NODES] = {}, h[NODES] = {}, sum[kCPT] = {};
+    if constexpr (COV) cov_row_log(d, row, M, L, h);
+    else M[0] = d.pref * y_factor(fmaf((float)(row - d.ya), d.dv, d.ay), d.ey);
+    float shift = -d.s3;                                       // -s3, s3, then 0
+    for (int i = 0;;) {
+        float hs[NODES];
+#pragma unroll
+        for (int k = 0; k < NODES; ++k) hs[k] = h[k] + shift;
+        gauss_strip<NODES>(d, M, L, hs, col0, sum);
+        if (++i == d.terms) break;
+        shift = i == 1 ? d.s3 : 0.0f;
+        const float amp = i == 1 ? 1.0f : d.s1;
+#pragma unroll
+        for (int k = 0; k < NODES; ++k) M[k] *= amp;
     }
-    if (d.kind == kSeries3) add_strip<NODES, 3, MASK>(d, W, h, col0, part);
-    else add_strip<NODES, kDirect, MASK>(d, W, h, col0, part);
+    const int lo = d.xa - col0, hi = d.xb - col0;
+#pragma unroll
+    for (int c = 0; c < kCPT; ++c) masked_set(part[c], part[c] + sum[c], c >= lo && c <= hi);
 }
 
 }  // namespace psf

@@ -3,10 +3,11 @@
 // k_dep_gather: FP32 per-point contributions summed per 64-point chunk -- the
 // chunk's common-case points (Gaussian form with one node per row, then with
 // two, footprint spanning the grid width) first, then the others, each in
-// point order -- then flushed into
-// FP64, the wide kernels' sums (on every kStep-th column) apart and
-// interpolated at the end; narrow erf-difference kernels add each bin straight into FP64.  Lets the CPU test-suite check the FP32 formulation and the footprint
-// index math against the FP64 oracle without a GPU.
+// point order -- then flushed into FP64, the wide kernels' sums (on every
+// kStep-th column) apart and interpolated at the end; erf-difference kernels
+// add each bin straight into FP64.  Lets the CPU test-suite check the FP32
+// formulation and the footprint index math against the FP64 oracle without a
+// GPU.
 #include "../../starformationhistories.jl_amd/csrc/sfh_psf.h"
 
 #include <cstring>
@@ -47,10 +48,10 @@ extern "C" int64_t emu_bin_cmd_smooth(const double* colors, const double* mags, 
                     float* pp = &wpart[((size_t)row * wcg + cg) * kCPT];
                     if (d.kind == kWide1) {
                         merged_row<1>(d, row, M, L, h);
-                        gauss_strip<1, false>(d, M, L, h, cg * kCPT, pp);
+                        gauss_strip<1>(d, M, L, h, cg * kCPT, pp);
                     } else {
                         merged_row<2>(d, row, M, L, h);
-                        gauss_strip<2, false>(d, M, L, h, cg * kCPT, pp);
+                        gauss_strip<2>(d, M, L, h, cg * kCPT, pp);
                     }
                 }
         }
@@ -61,9 +62,9 @@ extern "C" int64_t emu_bin_cmd_smooth(const double* colors, const double* mags, 
                 const bool full = d.xa == 0 && d.xb == nx - 1;
                 const int in = d.kind == kGauss1 ? 0 : full && d.kind == (asym ? kGauss : kGauss2) ? 1 : 2;
                 if (in != pass) continue;
-                // narrow erf-difference kernels: the kernel's wave-cooperative
+                // erf-difference kernels: the kernel's wave-cooperative
                 // path, one column at a time, each bin straight into FP64
-                const bool coop = d.kind == kDirect && d.xb - d.xa < 63;
+                const bool coop = d.kind == kDirect;
                 for (int row = d.ya; row <= d.yb; ++row) {
                     float W[3], L[3] = {0.0f, 0.0f, 0.0f}, h[3] = {0.0f, 0.0f, 0.0f};
                     if (pass == 0) merged_row<1>(d, row, W, L, h);
@@ -75,9 +76,8 @@ extern "C" int64_t emu_bin_cmd_smooth(const double* colors, const double* mags, 
                         for (int l = 0; l <= d.xb - d.xa; ++l) {
                             float v = 0.0f;
                             for (int k = 0; k < nodes; ++k) {
-                                const float b0 = direct_edge(d, l, h[k]), b1 = direct_edge(d, l + 1, h[k]);
-                                v = fmaf(W[k], erf_diff(erfc_pos(fabsf(b0)), b0 < 0.0f, erfc_pos(fabsf(b1)), b1 < 0.0f),
-                                         v);
+                                const float e0 = signed_erfc(direct_edge(d, l, h[k]));
+                                v = fmaf(W[k], erf_diff(e0, signed_erfc(direct_edge(d, l + 1, h[k]))), v);
                             }
                             acc[(size_t)row * ld + d.xa + l] += (double)v;
                         }
@@ -86,11 +86,11 @@ extern "C" int64_t emu_bin_cmd_smooth(const double* colors, const double* mags, 
                     for (int cg = 0; cg < ncg; ++cg) {
                         const int col0 = cg * kCPT;
                         float* pp = &part[(size_t)row * ld + col0];
-                        if (pass == 0 || (asym && pass == 1)) gauss_strip<1, false>(d, W, L, h, col0, pp);
-                        else if (pass == 1) gauss_strip<2, false>(d, W, L, h, col0, pp);
+                        if (pass == 0 || (asym && pass == 1)) gauss_strip<1>(d, W, L, h, col0, pp);
+                        else if (pass == 1) gauss_strip<2>(d, W, L, h, col0, pp);
                         else if (col0 <= d.xb && col0 + kCPT - 1 >= d.xa) {
-                            if (asym) add_point<false, true>(d, row, col0, pp);
-                            else add_point<true, true>(d, row, col0, pp);
+                            if (asym) add_point<false>(d, row, col0, pp);
+                            else add_point<true>(d, row, col0, pp);
                         }
                     }
                 }
