@@ -159,14 +159,12 @@ __device__ __forceinline__ void each(const PointDesc* __restrict__ chunk, uint64
 // one form per loop, into the FP64 sums [slice][template][row][node] that
 // k_dep_gather (or k_dep_finish) interpolates.
 __global__ __launch_bounds__(kDepBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_dep_wide(
-    const PointDesc* __restrict__ desc, const int64_t* __restrict__ offsets, GatherArgs a)
+    const PointDesc* __restrict__ desc, const int64_t* __restrict__ offsets, const int32_t* __restrict__ order,
+    GatherArgs a)
 {
-    __shared__ double sacc_[kCPT][kDepBlock];
-    const LdsAcc sacc{(lds_double*)&sacc_[0][0]};
     int64_t t;
     int blk;
-    const int nblk = (a.wcg * a.ny + kDepBlock - 1) / kDepBlock;
-    gather_tile(nullptr, nblk, &t, &blk);
+    gather_tile(order, (a.wcg * a.ny + kDepBlock - 1) / kDepBlock, &t, &blk);
     const int64_t p0 = offsets[t], p1 = offsets[t + 1];
     const int slot = blk * kDepBlock + threadIdx.x;
     const int row = slot / a.wcg;
@@ -174,10 +172,11 @@ __global__ __launch_bounds__(kDepBlock) __attribute__((amdgpu_waves_per_eu(4))) 
     const bool valid = row < a.ny;
     const int wslot = __builtin_amdgcn_readfirstlane(blk * kDepBlock + (int)(threadIdx.x & ~63u));
     const int row_lo = wslot / a.wcg, row_hi = (wslot + 63) / a.wcg;
+    double acc[kCPT];
     float part[kCPT];
 #pragma unroll
     for (int c = 0; c < kCPT; ++c) {
-        sacc[c][threadIdx.x] = 0.0;
+        acc[c] = 0.0;
         part[c] = 0.0f;
     }
     const PointDesc* __restrict__ td = desc + p0;
@@ -203,7 +202,7 @@ __global__ __launch_bounds__(kDepBlock) __attribute__((amdgpu_waves_per_eu(4))) 
         each(td + ch * kChunk, h2, [&](const PointDesc& d) { add(d, std::integral_constant<int, 2>{}); });
 #pragma unroll
         for (int c = 0; c < kCPT; ++c) {
-            sacc[c][threadIdx.x] += (double)part[c];
+            acc[c] += (double)part[c];
             part[c] = 0.0f;
         }
     }
@@ -211,7 +210,7 @@ __global__ __launch_bounds__(kDepBlock) __attribute__((amdgpu_waves_per_eu(4))) 
     double* o = a.wide + blockIdx.y * a.wstride + (t * a.ny + row) * (int64_t)(a.wcg * kCPT) + col0;
 #pragma unroll
     for (int c = 0; c < kCPT; c += 2)
-        *reinterpret_cast<double2*>(o + c) = make_double2(sacc[c][threadIdx.x], sacc[c + 1][threadIdx.x]);
+        *reinterpret_cast<double2*>(o + c) = make_double2(acc[c], acc[c + 1]);
 }
 
 // kStep columns from col (a multiple of kStep) of one row of template t: v plus
@@ -417,36 +416,48 @@ __device__ inline unsigned form_cost(int kind, bool full)
     return 32u;
 }
 
-// Estimated cost of every (template, row band) workgroup of the gather: per
-// point, the rows x strips of its footprint inside each band it meets, times
-// its form's cost.  One workgroup per template, the band sums in LDS (integer
-// atomics: the sums do not depend on the order); nblk * 8 bytes of dynamic LDS.
+// Adds a point's cost to every band of 256 strips (ncg per row) that its rows
+// meet: the rows x strips inside the band, times w.
+__device__ inline void band_cost(unsigned long long* band, int nblk, int ncg, int ya, int yb, unsigned w)
+{
+    const int b0 = (int)(((int64_t)ya * ncg) / kDepBlock);
+    int b1 = (int)(((int64_t)yb * ncg + ncg - 1) / kDepBlock);
+    if (b1 > nblk - 1) b1 = nblk - 1;
+    for (int b = b0; b <= b1; ++b) {
+        const int rlo = (int)(((int64_t)b * kDepBlock) / ncg);
+        const int rhi = (int)(((int64_t)b * kDepBlock + kDepBlock - 1) / ncg);
+        const int r0 = ya > rlo ? ya : rlo, r1 = yb < rhi ? yb : rhi;
+        if (r1 >= r0) atomicAdd(&band[b], (unsigned long long)(r1 - r0 + 1) * w);
+    }
+}
+
+// Estimated cost of every (template, row band) workgroup of the gather (cost)
+// and of the wide kernels' gather (wcost).  One workgroup per template, the
+// band sums in LDS (integer atomics: the sums do not depend on the order);
+// (nblk + wblk) * 8 bytes of dynamic LDS.
 __global__ __launch_bounds__(256) void k_dep_cost(const PointDesc* __restrict__ desc,
                                                   const int64_t* __restrict__ offsets, int nx, int ncg, int nblk,
-                                                  unsigned long long* __restrict__ cost)
+                                                  int wcg, int wblk, unsigned long long* __restrict__ cost,
+                                                  unsigned long long* __restrict__ wcost)
 {
     extern __shared__ unsigned long long band[];
     const int64_t t = blockIdx.x;
-    for (int b = threadIdx.x; b < nblk; b += blockDim.x) band[b] = 0;
+    for (int b = threadIdx.x; b < nblk + wblk; b += blockDim.x) band[b] = 0;
     __syncthreads();
     for (int64_t p = offsets[t] + threadIdx.x; p < offsets[t + 1]; p += blockDim.x) {
         const int4 f = *reinterpret_cast<const int4*>(desc + p);
-        if (f.x > f.y || desc[p].kind >= psf::kWide1) continue;
-        const bool full = f.x == 0 && f.y == nx - 1;
-        const unsigned w = form_cost(desc[p].kind, full);
-        const int nstrips = f.y / kCPT - f.x / kCPT + 1;
-        const int b0 = (int)(((int64_t)f.z * ncg) / kDepBlock);
-        int b1 = (int)(((int64_t)f.w * ncg + ncg - 1) / kDepBlock);
-        if (b1 > nblk - 1) b1 = nblk - 1;
-        for (int b = b0; b <= b1; ++b) {
-            const int rlo = (int)(((int64_t)b * kDepBlock) / ncg);
-            const int rhi = (int)(((int64_t)b * kDepBlock + kDepBlock - 1) / ncg);
-            const int r0 = f.z > rlo ? f.z : rlo, r1 = f.w < rhi ? f.w : rhi;
-            if (r1 >= r0) atomicAdd(&band[b], (unsigned long long)(r1 - r0 + 1) * nstrips * w);
+        if (f.x > f.y) continue;
+        const int kind = desc[p].kind;
+        if (kind >= psf::kWide1) {
+            band_cost(band + nblk, wblk, wcg, f.z, f.w, (unsigned)wcg * (kind == psf::kWide1 ? 2u : 3u));
+        } else {
+            const unsigned w = form_cost(kind, f.x == 0 && f.y == nx - 1);
+            band_cost(band, nblk, ncg, f.z, f.w, w * (unsigned)(f.y / kCPT - f.x / kCPT + 1));
         }
     }
     __syncthreads();
     for (int b = threadIdx.x; b < nblk; b += blockDim.x) cost[t * nblk + b] = band[b];
+    for (int b = threadIdx.x; b < wblk; b += blockDim.x) wcost[t * wblk + b] = band[nblk + b];
 }
 
 constexpr int kOrderMax = 16384;    // workgroups one ordering launch takes
@@ -456,9 +467,15 @@ constexpr int kOrderBuckets = 1024;
 // a counting sort over 1024 cost buckets in one workgroup (the order inside
 // a bucket is that of the LDS atomics; it only schedules the gather, whose
 // workgroups each write their own band, so the templates do not depend on it).
-__global__ __launch_bounds__(1024) void k_dep_order(const unsigned long long* __restrict__ cost, int n,
+// One workgroup per list: the gather's n costs, then the wide kernels' nwide.
+__global__ __launch_bounds__(1024) void k_dep_order(const unsigned long long* __restrict__ cost, int n, int nwide,
                                                     int32_t* __restrict__ order)
 {
+    if (blockIdx.x == 1) {
+        cost += n;
+        order += n;
+        n = nwide;
+    }
     __shared__ unsigned long long smax[16];
     __shared__ int start[kOrderBuckets];
     __shared__ int wsum[16];
@@ -523,10 +540,32 @@ static int launch_gather(sfh_ctx* ctx, const PointDesc* desc, const int64_t* d_o
         };
         const int ns = slices(grid);
         const int64_t* offsets = d_offsets + t0;
-        const int32_t* order = nullptr;
+        const int32_t *order = nullptr, *worder = nullptr;
         a.out32 = out32 ? out32 + t0 * ld_out : nullptr;
         a.out64 = out64 ? out64 + t0 * ld_out : nullptr;
         a.part = nullptr;
+        if (ns > 1) {
+            void* p = nullptr;
+            if (int rc = scratch(ctx, "dep_part", (size_t)ns * nt * nx * ny * sizeof(double), &p)) return rc;
+            a.part = (double*)p;
+        } else if (nt > 1 && grid <= kOrderMax && npoints > 0) {
+            const int64_t wgrid = wblk * nt;
+            void *pc = nullptr, *po = nullptr;
+            if (int rc = scratch(ctx, "dep_cost", (size_t)(grid + wgrid) * sizeof(unsigned long long), &pc)) return rc;
+            if (int rc = scratch(ctx, "dep_order", (size_t)(grid + wgrid) * sizeof(int32_t), &po)) return rc;
+            {
+                TimedLaunch tl(ctx, "deposit_order");
+                hipLaunchKernelGGL(k_dep_cost, dim3((unsigned)nt), dim3(256),
+                                   (size_t)(a.nblk + wblk) * sizeof(unsigned long long), ctx->stream, desc, offsets, nx,
+                                   a.ncg, a.nblk, a.wcg, (int)wblk, (unsigned long long*)pc,
+                                   (unsigned long long*)pc + grid);
+                hipLaunchKernelGGL(k_dep_order, dim3(a.wcg ? 2 : 1), dim3(1024), 0, ctx->stream,
+                                   (const unsigned long long*)pc, (int)grid, (int)wgrid, (int32_t*)po);
+            }
+            if (int rc = check_launch(ctx, "k_dep_order")) return rc;
+            order = (const int32_t*)po;
+            worder = order + grid;
+        }
         if (a.wcg) {
             a.wslices = slices(wblk * nt);
             a.wstride = wbins * nt;
@@ -535,28 +574,9 @@ static int launch_gather(sfh_ctx* ctx, const PointDesc* desc, const int64_t* d_o
             a.wide = (double*)p;
             TimedLaunch tl(ctx, "deposit_wide");
             hipLaunchKernelGGL(k_dep_wide, dim3((unsigned)(wblk * nt), (unsigned)a.wslices), dim3(kDepBlock), 0,
-                               ctx->stream, desc, offsets, a);
+                               ctx->stream, desc, offsets, worder, a);
         }
         if (int rc = check_launch(ctx, "k_dep_wide")) return rc;
-        if (ns > 1) {
-            void* p = nullptr;
-            if (int rc = scratch(ctx, "dep_part", (size_t)ns * nt * nx * ny * sizeof(double), &p)) return rc;
-            a.part = (double*)p;
-        } else if (nt > 1 && grid <= kOrderMax && npoints > 0) {
-            void *pc = nullptr, *po = nullptr;
-            if (int rc = scratch(ctx, "dep_cost", (size_t)grid * sizeof(unsigned long long), &pc)) return rc;
-            if (int rc = scratch(ctx, "dep_order", (size_t)grid * sizeof(int32_t), &po)) return rc;
-            {
-                TimedLaunch tl(ctx, "deposit_order");
-                hipLaunchKernelGGL(k_dep_cost, dim3((unsigned)nt), dim3(256),
-                                   (size_t)a.nblk * sizeof(unsigned long long), ctx->stream, desc, offsets, nx,
-                                   a.ncg, a.nblk, (unsigned long long*)pc);
-                hipLaunchKernelGGL(k_dep_order, dim3(1), dim3(1024), 0, ctx->stream, (const unsigned long long*)pc,
-                                   (int)grid, (int32_t*)po);
-            }
-            if (int rc = check_launch(ctx, "k_dep_order")) return rc;
-            order = (const int32_t*)po;
-        }
         {
             TimedLaunch tl(ctx, asym ? "deposit_asym" : "deposit_cov");
             const dim3 g((unsigned)grid, (unsigned)ns);
