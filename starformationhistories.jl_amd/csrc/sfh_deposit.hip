@@ -36,6 +36,7 @@
 namespace sfh {
 
 using psf::PointDesc;
+using psf::PointKey;
 
 constexpr int kDepBlock = 256;
 constexpr int kCPT = psf::kCPT;  // columns per thread
@@ -52,7 +53,7 @@ __global__ __launch_bounds__(256) void k_dep_prep(
     const double* __restrict__ cerr, const double* __restrict__ merr,
     const double* __restrict__ weights, const double* __restrict__ cmult, double cov_mult,
     int64_t npoints, psf::Range ex, psf::Range ey, int asym, PointDesc* __restrict__ out,
-    unsigned long long* __restrict__ pairs, int* __restrict__ bad)
+    PointKey* __restrict__ keys, unsigned long long* __restrict__ pairs, int* __restrict__ bad)
 {
     const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     unsigned long long cnt = 0;
@@ -69,6 +70,7 @@ __global__ __launch_bounds__(256) void k_dep_prep(
             cnt = (unsigned long long)psf::prep_covariant(x, y, sx, sy, c, A, ex, ey, &d);
         }
         out[p] = d;
+        keys[p] = psf::point_key(d, (int)(ex.length - 1), asym != 0);
     }
     // wave-level sum of pair counts, one atomic per wave
     for (int off = 32; off > 0; off >>= 1) cnt += __shfl_xor(cnt, off, 64);
@@ -116,23 +118,10 @@ struct LdsAcc {
     __device__ lds_double* operator[](int c) const { return p + c * kDepBlock; }
 };
 
-// One lane's point of a chunk: its footprint (the descriptor's first 16 bytes)
-// and form.
-struct Foot {
-    int4 f;
-    int kind;
-};
-__device__ inline Foot footprint(const PointDesc* td, int p, int np)
+// One lane's point of a chunk (class none past the end).
+__device__ inline PointKey key_of(const PointKey* __restrict__ keys, int p, int np)
 {
-    Foot r;
-    if (p < np) {
-        r.f = *reinterpret_cast<const int4*>(td + p);
-        r.kind = td[p].kind;
-    } else {
-        r.f = make_int4(1, 0, 1, 0);
-        r.kind = psf::kDirect;
-    }
-    return r;
+    return p < np ? keys[p] : PointKey{1u, 0u};
 }
 
 // f(descriptor) for each of a chunk's points in hits, in order.  Descriptors
@@ -159,8 +148,8 @@ __device__ __forceinline__ void each(const PointDesc* __restrict__ chunk, uint64
 // one form per loop, into the FP64 sums [slice][template][row][node] that
 // k_dep_gather (or k_dep_finish) interpolates.
 __global__ __launch_bounds__(kDepBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_dep_wide(
-    const PointDesc* __restrict__ desc, const int64_t* __restrict__ offsets, const int32_t* __restrict__ order,
-    GatherArgs a)
+    const PointDesc* __restrict__ desc, const PointKey* __restrict__ keys, const int64_t* __restrict__ offsets,
+    const int32_t* __restrict__ order, GatherArgs a)
 {
     int64_t t;
     int blk;
@@ -180,9 +169,11 @@ __global__ __launch_bounds__(kDepBlock) __attribute__((amdgpu_waves_per_eu(4))) 
         part[c] = 0.0f;
     }
     const PointDesc* __restrict__ td = desc + p0;
+    const PointKey* __restrict__ tk = keys + p0;
     const int np = (int)(p1 - p0);
     const int nch = (np + kChunk - 1) / kChunk;
-    const int c0 = (int)((int64_t)nch * blockIdx.y / gridDim.y), c1 = (int)((int64_t)nch * (blockIdx.y + 1) / gridDim.y);
+    const int c0 = (int)((int64_t)nch * blockIdx.y / gridDim.y);
+    const int c1 = (int)((int64_t)nch * (blockIdx.y + 1) / gridDim.y);
     const int lane = threadIdx.x & 63;
     auto add = [&](const PointDesc& d, auto nodes) {
         constexpr int NODES = decltype(nodes)::value;
@@ -191,12 +182,13 @@ __global__ __launch_bounds__(kDepBlock) __attribute__((amdgpu_waves_per_eu(4))) 
         psf::merged_row<NODES>(d, row, M, L, h);
         psf::gauss_strip<NODES>(d, M, L, h, col0, part);
     };
-    Foot fn = footprint(td, c0 * kChunk + lane, np);
+    PointKey kn = key_of(tk, c0 * kChunk + lane, np);
     for (int ch = c0; ch < c1; ++ch) {
-        const Foot f = fn;
-        fn = footprint(td, (ch + 1) * kChunk + lane, np);           // next chunk's footprints in flight
-        const bool hit = f.f.x <= f.f.y && f.f.z <= row_hi && f.f.w >= row_lo;
-        const uint64_t h1 = __ballot(hit && f.kind == psf::kWide1), h2 = __ballot(hit && f.kind == psf::kWide2);
+        const PointKey k = kn;
+        kn = key_of(tk, (ch + 1) * kChunk + lane, np);              // next chunk's keys in flight
+        const uint32_t cls = k.cls();
+        const bool hit = k.ya() <= row_hi && k.yb() >= row_lo;
+        const uint64_t h1 = __ballot(hit && cls == psf::kClsWide1), h2 = __ballot(hit && cls == psf::kClsWide2);
         if (!(h1 | h2)) continue;
         each(td + ch * kChunk, h1, [&](const PointDesc& d) { add(d, std::integral_constant<int, 1>{}); });
         each(td + ch * kChunk, h2, [&](const PointDesc& d) { add(d, std::integral_constant<int, 2>{}); });
@@ -251,8 +243,8 @@ __device__ inline void finish_cols(const GatherArgs& a, int64_t t, int row, int 
 // the per-point constants fit the registers of five waves per SIMD.
 template <bool kAsym>
 __global__ __launch_bounds__(kDepBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_dep_gather(
-    const PointDesc* __restrict__ desc, const int64_t* __restrict__ offsets, const int32_t* __restrict__ order,
-    GatherArgs a)
+    const PointDesc* __restrict__ desc, const PointKey* __restrict__ keys, const int64_t* __restrict__ offsets,
+    const int32_t* __restrict__ order, GatherArgs a)
 {
     __shared__ double sacc_[kCPT][kDepBlock];
     const LdsAcc sacc{(lds_double*)&sacc_[0][0]};
@@ -285,9 +277,11 @@ __global__ __launch_bounds__(kDepBlock) __attribute__((amdgpu_waves_per_eu(4))) 
     // through it without copies; a bin sums a chunk's points pass by pass, each
     // in point order (deterministic).
     const PointDesc* __restrict__ td = desc + p0;
+    const PointKey* __restrict__ tk = keys + p0;
     const int np = (int)(p1 - p0);
     const int nch = (np + kChunk - 1) / kChunk;
-    const int c0 = (int)((int64_t)nch * blockIdx.y / gridDim.y), c1 = (int)((int64_t)nch * (blockIdx.y + 1) / gridDim.y);
+    const int c0 = (int)((int64_t)nch * blockIdx.y / gridDim.y);
+    const int c1 = (int)((int64_t)nch * (blockIdx.y + 1) / gridDim.y);
     const int lane = threadIdx.x & 63;
     const int wave_id = (int)(threadIdx.x >> 6);
     auto in_rows = [&](const PointDesc& d) { return valid && row >= d.ya && row <= d.yb; };
@@ -345,21 +339,19 @@ __global__ __launch_bounds__(kDepBlock) __attribute__((amdgpu_waves_per_eu(4))) 
             }
         }
     };
-    constexpr int kSecond = kAsym ? psf::kGauss : psf::kGauss2;
-    Foot fn = footprint(td, c0 * kChunk + lane, np);
+    PointKey kn = key_of(tk, c0 * kChunk + lane, np);
     for (int ch = c0; ch < c1; ++ch) {
-        const Foot f = fn;
-        fn = footprint(td, (ch + 1) * kChunk + lane, np);           // next chunk's footprints in flight
-        const bool hit = f.f.x <= f.f.y && f.f.z <= row_hi && f.f.w >= row_lo && f.kind < psf::kWide1;
-        const bool full = f.f.x == 0 && f.f.y == nx - 1;
+        const PointKey k = kn;
+        kn = key_of(tk, (ch + 1) * kChunk + lane, np);              // next chunk's keys in flight
+        const uint32_t cls = k.cls();
+        const bool hit = k.ya() <= row_hi && k.yb() >= row_lo && cls >= psf::kClsOne;
         const uint64_t all = __ballot(hit);
         if (!all) continue;
-        const uint64_t h1 = __ballot(hit && f.kind == psf::kGauss1);
-        const uint64_t h2 = __ballot(hit && full && f.kind == kSecond);
+        const uint64_t h1 = __ballot(hit && cls == psf::kClsOne), h2 = __ballot(hit && cls == psf::kClsSecond);
+        const uint64_t h3 = __ballot(hit && cls == psf::kClsDirect);
         const PointDesc* __restrict__ chunk = td + ch * kChunk;
         each(chunk, h1, [&](const PointDesc& d) { add_common(d, std::integral_constant<int, 1>{}); });
         each(chunk, h2, [&](const PointDesc& d) { add_common(d, std::integral_constant<int, kAsym ? 0 : 2>{}); });
-        const uint64_t h3 = __ballot(hit && f.kind == psf::kDirect);
         each(chunk, all & ~(h1 | h2 | h3), add);
         each(chunk, h3, direct);
 #pragma unroll
@@ -518,8 +510,9 @@ __global__ __launch_bounds__(1024) void k_dep_order(const unsigned long long* __
 // launch is small enough to order in one pass.  Where a launch would leave the
 // chip idle its points are split into slices, whose FP64 sums k_dep_finish
 // adds in order.
-static int launch_gather(sfh_ctx* ctx, const PointDesc* desc, const int64_t* d_offsets, int64_t ntemplates,
-                         int64_t npoints, bool asym, int nx, int ny, float* out32, double* out64, int64_t ld_out)
+static int launch_gather(sfh_ctx* ctx, const PointDesc* desc, const PointKey* keys, const int64_t* d_offsets,
+                         int64_t ntemplates, int64_t npoints, bool asym, int nx, int ny, float* out32, double* out64,
+                         int64_t ld_out)
 {
     GatherArgs a{};
     a.nx = nx;
@@ -574,14 +567,14 @@ static int launch_gather(sfh_ctx* ctx, const PointDesc* desc, const int64_t* d_o
             a.wide = (double*)p;
             TimedLaunch tl(ctx, "deposit_wide");
             hipLaunchKernelGGL(k_dep_wide, dim3((unsigned)(wblk * nt), (unsigned)a.wslices), dim3(kDepBlock), 0,
-                               ctx->stream, desc, offsets, worder, a);
+                               ctx->stream, desc, keys, offsets, worder, a);
         }
         if (int rc = check_launch(ctx, "k_dep_wide")) return rc;
         {
             TimedLaunch tl(ctx, asym ? "deposit_asym" : "deposit_cov");
             const dim3 g((unsigned)grid, (unsigned)ns);
-            if (asym) hipLaunchKernelGGL(k_dep_gather<true>, g, dim3(kDepBlock), 0, ctx->stream, desc, offsets, order, a);
-            else hipLaunchKernelGGL(k_dep_gather<false>, g, dim3(kDepBlock), 0, ctx->stream, desc, offsets, order, a);
+            hipLaunchKernelGGL(asym ? k_dep_gather<true> : k_dep_gather<false>, g, dim3(kDepBlock), 0, ctx->stream,
+                               desc, keys, offsets, order, a);
         }
         if (int rc = check_launch(ctx, "k_dep_gather")) return rc;
         if (ns > 1) {
@@ -615,8 +608,9 @@ static int deposit(sfh_ctx* ctx, const double* colors, const double* mags, const
     SFH_ARG_CHECK(ctx, ld_out >= (int64_t)nx * ny, "ld_out < nx*ny");
     const bool asym = (cov_mult == 0.0) && cmult == nullptr;
     void *pdesc = nullptr, *pcnt = nullptr;
-    if (int rc = scratch(ctx, "dep_desc", (size_t)(npoints_total + 1) * sizeof(PointDesc), &pdesc))
+    if (int rc = scratch(ctx, "dep_desc", (size_t)(npoints_total + 1) * (sizeof(PointDesc) + sizeof(PointKey)), &pdesc))
         return rc;
+    PointKey* keys = (PointKey*)((PointDesc*)pdesc + npoints_total + 1);
     if (int rc = scratch(ctx, "dep_counters", 64, &pcnt)) return rc;
     SFH_HIP_TRY(ctx, hipMemsetAsync(pcnt, 0, 64, ctx->stream));
     unsigned long long* d_pairs = (unsigned long long*)pcnt;
@@ -626,10 +620,10 @@ static int deposit(sfh_ctx* ctx, const double* colors, const double* mags, const
         TimedLaunch tl(ctx, "deposit_prep");
         hipLaunchKernelGGL(k_dep_prep, dim3((unsigned)cdiv(npoints_total, 256)), dim3(256), 0, ctx->stream,
                            colors, mags, cerr, merr, weights, cmult, cov_mult, npoints_total, rx, ry,
-                           asym ? 1 : 0, (PointDesc*)pdesc, d_pairs, d_bad);
+                           asym ? 1 : 0, (PointDesc*)pdesc, keys, d_pairs, d_bad);
     }
     if (int rc = check_launch(ctx, "k_dep_prep")) return rc;
-    if (int rc = launch_gather(ctx, (const PointDesc*)pdesc, d_offsets, ntemplates, npoints_total, asym, nx, ny,
+    if (int rc = launch_gather(ctx, (const PointDesc*)pdesc, keys, d_offsets, ntemplates, npoints_total, asym, nx, ny,
                                out32, out64, ld_out))
         return rc;
     // Non-finite inputs: the reference's round(Int, NaN) throws InexactError.
@@ -645,14 +639,14 @@ static int deposit(sfh_ctx* ctx, const double* colors, const double* mags, const
 
 // The gather of descriptors already built (by the device preparation of
 // partial_cmd_smooth): template t owns desc[koff[t] .. koff[t+1]).
-int deposit_from_desc(sfh_ctx* ctx, const void* desc, const int64_t* d_koff, int64_t ntemplates, int64_t npoints,
-                      bool asym, sfh_range xe, sfh_range ye, float* out32, int64_t ld_out)
+int deposit_from_desc(sfh_ctx* ctx, const void* desc, const void* keys, const int64_t* d_koff, int64_t ntemplates,
+                      int64_t npoints, bool asym, sfh_range xe, sfh_range ye, float* out32, int64_t ld_out)
 {
     if (int rc = validate_ranges(ctx, xe, ye)) return rc;
     const int nx = (int)(xe.length - 1), ny = (int)(ye.length - 1);
     SFH_ARG_CHECK(ctx, ld_out >= (int64_t)nx * ny, "ld_out < nx*ny");
-    return launch_gather(ctx, (const PointDesc*)desc, d_koff, ntemplates, npoints, asym, nx, ny, out32, nullptr,
-                         ld_out);
+    return launch_gather(ctx, (const PointDesc*)desc, (const PointKey*)keys, d_koff, ntemplates, npoints, asym, nx, ny,
+                         out32, nullptr, ld_out);
 }
 
 }  // namespace sfh

@@ -104,6 +104,7 @@ struct Args {
     double* iso;           // 3 x Qtotal magnitudes (roles a, b, y)
     int64_t qtotal;
     psf::PointDesc* desc;  // koff layout
+    psf::PointKey* keys;   // koff layout
     unsigned long long* pairs;
     int* bad;
 };
@@ -320,6 +321,7 @@ __global__ __launch_bounds__(kWG) void k_pcs_desc(Args a)
             }
         }
         a.desc[kbase + k] = d;
+        a.keys[kbase + k] = psf::point_key(d, (int)(a.ex.length - 1), a.cov_mult == 0.0);
     }
     for (int off = 32; off > 0; off >>= 1) cnt += __shfl_xor(cnt, off, 64);
     if ((threadIdx.x & 63) == 0 && cnt) atomicAdd(a.pairs, cnt);
@@ -535,13 +537,15 @@ int sfh_partial_cmd_smooth_batch(sfh_ctx* ctx, int64_t ntemplates, const int64_t
     if (int rc = upload_scratch(ctx, "pcs_koff", koff.data(), koff.size() * sizeof(int64_t), &dk)) return rc;
     if (int rc = scratch(ctx, "pcs_mini", (size_t)(Q + 1) * sizeof(double), &dmini)) return rc;
     if (int rc = scratch(ctx, "pcs_iso", (size_t)(Q + 1) * 3 * sizeof(double), &diso)) return rc;
-    if (int rc = scratch(ctx, "dep_desc", (size_t)(K + 1) * sizeof(psf::PointDesc), &ddesc)) return rc;
+    if (int rc = scratch(ctx, "dep_desc", (size_t)(K + 1) * (sizeof(psf::PointDesc) + sizeof(psf::PointKey)), &ddesc))
+        return rc;
     a.qoff = (const int64_t*)dq;
     a.koff = (const int64_t*)dk;
     a.mini = (double*)dmini;
     a.iso = (double*)diso;
     a.qtotal = Q;
     a.desc = (psf::PointDesc*)ddesc;
+    a.keys = (psf::PointKey*)(a.desc + K + 1);
 
     // 2. resampled masses and magnitudes, 3. kernel point descriptors
     {
@@ -562,7 +566,7 @@ int sfh_partial_cmd_smooth_batch(sfh_ctx* ctx, int64_t ntemplates, const int64_t
         if (int rc = scratch(ctx, "pcs_out", (size_t)nbins * ntemplates * sizeof(float), &p)) return rc;
         dst = (float*)p;
     }
-    if (int rc = deposit_from_desc(ctx, ddesc, (const int64_t*)dk, ntemplates, K, a.cov_mult == 0.0, xedges,
+    if (int rc = deposit_from_desc(ctx, ddesc, a.keys, (const int64_t*)dk, ntemplates, K, a.cov_mult == 0.0, xedges,
                                    yedges, dst, ld))
         return rc;
     unsigned long long pairs = 0;

@@ -99,6 +99,33 @@ struct alignas(16) PointDesc {
     float q[8];             // Gaussian forms: q[j] = 2^-(du (j + 1/2))^2, the strip's column factors
 };
 
+// What the gather reads of every point to find its hits: the rows of its
+// footprint and the class of its evaluation, in 8 bytes.
+enum : uint32_t { kClsNone = 0, kClsWide1, kClsWide2, kClsOne, kClsSecond, kClsRest, kClsDirect };
+struct PointKey {
+    uint32_t a, b;     // ya | low two bits of the class << 30, yb | its high bits << 30
+    __host__ __device__ int ya() const { return (int)(a & 0x3FFFFFFFu); }
+    __host__ __device__ int yb() const { return (int)(b & 0x3FFFFFFFu); }
+    __host__ __device__ uint32_t cls() const { return (a >> 30) | (b >> 30) << 2; }
+};
+
+// The class of a point on a grid of nx columns: kClsOne, one merged node per
+// row; kClsSecond, the other common form (a covariant kernel's two nodes, an
+// asymmetric one of the grid's width with a y factor per row); kClsRest,
+// masked strips.
+__host__ __device__ inline PointKey point_key(const PointDesc& d, int nx, bool asym)
+{
+    if (d.xa > d.xb) return PointKey{1u, 0u};
+    const bool full = d.xa == 0 && d.xb == nx - 1;
+    const uint32_t c = d.kind == kWide1    ? kClsWide1
+                       : d.kind == kWide2  ? kClsWide2
+                       : d.kind == kDirect ? kClsDirect
+                       : d.kind == kGauss1 ? kClsOne
+                       : d.kind == kGauss2 || (asym && full && d.kind == kGauss) ? kClsSecond
+                                                                                 : kClsRest;
+    return PointKey{(uint32_t)d.ya | (c & 3u) << 30, (uint32_t)d.yb | (c >> 2) << 30};
+}
+
 struct Range {
     double first, step;
     int64_t length;
