@@ -35,6 +35,7 @@
 
 namespace sfh {
 
+using psf::PointCounts;
 using psf::PointDesc;
 using psf::PointKey;
 
@@ -72,9 +73,7 @@ __global__ __launch_bounds__(256) void k_dep_prep(
         out[p] = d;
         keys[p] = psf::point_key(d, (int)(ex.length - 1), asym != 0);
     }
-    // wave-level sum of pair counts, one atomic per wave
-    for (int off = 32; off > 0; off >>= 1) cnt += __shfl_xor(cnt, off, 64);
-    if ((threadIdx.x & 63) == 0 && cnt) atomicAdd(pairs, cnt);
+    psf::add_count(pairs, blockIdx.x, cnt);
 }
 
 struct GatherArgs {
@@ -611,29 +610,26 @@ static int deposit(sfh_ctx* ctx, const double* colors, const double* mags, const
     if (int rc = scratch(ctx, "dep_desc", (size_t)(npoints_total + 1) * (sizeof(PointDesc) + sizeof(PointKey)), &pdesc))
         return rc;
     PointKey* keys = (PointKey*)((PointDesc*)pdesc + npoints_total + 1);
-    if (int rc = scratch(ctx, "dep_counters", 64, &pcnt)) return rc;
-    SFH_HIP_TRY(ctx, hipMemsetAsync(pcnt, 0, 64, ctx->stream));
-    unsigned long long* d_pairs = (unsigned long long*)pcnt;
-    int* d_bad = (int*)((char*)pcnt + 16);
+    if (int rc = scratch(ctx, "dep_counters", sizeof(PointCounts), &pcnt)) return rc;
+    SFH_HIP_TRY(ctx, hipMemsetAsync(pcnt, 0, sizeof(PointCounts), ctx->stream));
+    PointCounts* dc = (PointCounts*)pcnt;
     psf::Range rx{xe.first, xe.step, xe.length}, ry{ye.first, ye.step, ye.length};
     if (npoints_total > 0) {
         TimedLaunch tl(ctx, "deposit_prep");
         hipLaunchKernelGGL(k_dep_prep, dim3((unsigned)cdiv(npoints_total, 256)), dim3(256), 0, ctx->stream,
                            colors, mags, cerr, merr, weights, cmult, cov_mult, npoints_total, rx, ry,
-                           asym ? 1 : 0, (PointDesc*)pdesc, keys, d_pairs, d_bad);
+                           asym ? 1 : 0, (PointDesc*)pdesc, keys, dc->pairs, &dc->bad);
     }
     if (int rc = check_launch(ctx, "k_dep_prep")) return rc;
     if (int rc = launch_gather(ctx, (const PointDesc*)pdesc, keys, d_offsets, ntemplates, npoints_total, asym, nx, ny,
                                out32, out64, ld_out))
         return rc;
     // Non-finite inputs: the reference's round(Int, NaN) throws InexactError.
-    int bad = 0;
-    unsigned long long pairs = 0;
-    SFH_HIP_TRY(ctx, hipMemcpyAsync(&bad, d_bad, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-    SFH_HIP_TRY(ctx, hipMemcpyAsync(&pairs, d_pairs, sizeof(pairs), hipMemcpyDeviceToHost, ctx->stream));
+    PointCounts hc;
+    SFH_HIP_TRY(ctx, hipMemcpyAsync(&hc, dc, sizeof(hc), hipMemcpyDeviceToHost, ctx->stream));
     SFH_HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-    if (bad) return set_error(ctx, SFH_ERR_DOMAIN, "non-finite kernel parameter (InexactError in round(Int, ·))");
-    if (pairs_out) *pairs_out = (int64_t)pairs;
+    if (hc.bad) return set_error(ctx, SFH_ERR_DOMAIN, "non-finite kernel parameter (InexactError in round(Int, ·))");
+    if (pairs_out) *pairs_out = hc.total();
     return SFH_OK;
 }
 

@@ -14,11 +14,19 @@
 //                 segment's new masses m_i + j Δm_i / n_i (or m_{i+1}); the
 //                 magnitudes of the three filters involved are interpolated
 //                 linearly on the isochrone's knots, plus the distance modulus.
-//   k_pcs_desc    workgroup per isochrone: the callables at every resampled
-//                 point, the weights (trapezoid of the IMF, completeness of the
-//                 left point), the midpoint series (the range form when every
-//                 step agrees to sqrt(eps), as midpoints(v, true) does) and the
-//                 footprint / evaluation constants of each kernel point.
+//   k_pcs_vals    thread per resampled point: the callables and the IMF there,
+//                 each evaluated once (their powers and exponentials are most
+//                 of the preparation's FP64 work).
+//   k_pcs_desc    thread per kernel point: the weights (trapezoid of the IMF,
+//                 completeness of the left point), the midpoint series (the
+//                 range form when every step agrees to sqrt(eps), as
+//                 midpoints(v, true) does) and the footprint / evaluation
+//                 constants.
+// Both are bound by FP64 latency, so they run as many workgroups as there are
+// points.  With the callables evaluated four times per point inside one
+// workgroup per isochrone they took 0.39 ms for 700 isochrones of 2000 points
+// (1.5M kernel points) and 0.08 ms for 50 of 500; now 0.19 and 0.03 ms (0.12 ms
+// of that gain for 700 from the pair counts' atomics, which all went to one word).
 //
 // FP64 throughout, in the reference's operation order, with no contracted
 // multiply-adds.  Inputs the restatement does not reproduce are refused with
@@ -102,6 +110,7 @@ struct Args {
     psf::Range ex, ey;
     double* mini;          // resampled masses, qoff layout
     double* iso;           // 3 x Qtotal magnitudes (roles a, b, y)
+    double* vals;          // kVals x Qtotal values of the callables (k_pcs_vals)
     int64_t qtotal;
     psf::PointDesc* desc;  // koff layout
     psf::PointKey* keys;   // koff layout
@@ -215,16 +224,14 @@ __global__ __launch_bounds__(kWG) void k_pcs_points(Args a)
     if (flags) atomicOr(a.bad, flags);
 }
 
-// The four midpoint series of resampled point k (bias-shifted colour and y
-// magnitude, colour error, y error: :871-888) and its completeness.
-struct PointVals {
-    double v[4];
-    double compl_;
-};
+// Per resampled point: the four midpoint series (bias-shifted colour and y
+// magnitude, colour error, y error: :871-888), its completeness and the IMF.
+enum : int { kCompl = 4, kPdf = 5, kVals = 6 };
 
-__device__ inline PointVals point_vals(const Args& a, int64_t q)
+__global__ __launch_bounds__(kWG) void k_pcs_vals(Args a)
 {
-    PointVals o;
+    const int64_t q = (int64_t)blockIdx.x * kWG + threadIdx.x;
+    if (q >= a.qtotal) return;
     const double ia = a.iso[q], ib = a.iso[a.qtotal + q], iy = a.iso[2 * a.qtotal + q];
     const double ea = eval(a.err[0], ia), eb = eval(a.err[1], ib), ey = eval(a.err[2], iy);   // :855
     double cerr;
@@ -237,12 +244,9 @@ __device__ inline PointVals point_vals(const Args& a, int64_t q)
     }
     const double ba = ia + eval(a.bias[0], ia), bb = ib + eval(a.bias[1], ib);   // :884
     const double by = iy + eval(a.bias[2], iy);
-    o.v[0] = ba - bb;                               // :885
-    o.v[1] = by;
-    o.v[2] = cerr;
-    o.v[3] = ey;
-    o.compl_ = compl_;
-    return o;
+    const double out[kVals] = {ba - bb, by, cerr, ey, compl_, eval(a.imf, a.mini[q])};        // :885
+#pragma unroll
+    for (int s = 0; s < kVals; ++s) a.vals[s * a.qtotal + q] = out[s];
 }
 
 // Julia's isapprox(x, y) with atol = 0, rtol = sqrt(eps(Float64))
@@ -253,57 +257,60 @@ __device__ inline bool approx(double x, double y)
 
 __global__ __launch_bounds__(kWG) void k_pcs_desc(Args a)
 {
-    __shared__ int ranges[4];
+    __shared__ int ranges;
     const int64_t t = blockIdx.x;
     const int64_t q0 = a.qoff[t], Q = a.qoff[t + 1] - q0;
     const int64_t K = Q - 1;
-    if (K <= 0) return;
-    if (threadIdx.x < 4) ranges[threadIdx.x] = 1;
-    __syncthreads();
+    if (K <= (int64_t)blockIdx.y * kWG) return;
+    auto val = [&](int s, int64_t k) { return a.vals[s * a.qtotal + q0 + k]; };
+    if (threadIdx.x == 0) ranges = 0xF;
     // midpoints(v, true): the range form when every step is approximately the first (:421-428)
-    const PointVals f0 = point_vals(a, q0), f1 = point_vals(a, q0 + 1);
-    const PointVals fl = point_vals(a, q0 + K);
-    double d0[4];
+    double f0[4], d0[4];
 #pragma unroll
-    for (int s = 0; s < 4; ++s) d0[s] = f1.v[s] - f0.v[s];
-    int ok = 0xF;
-    for (int64_t k = threadIdx.x; k < K; k += kWG) {
-        const PointVals u = point_vals(a, q0 + k), w = point_vals(a, q0 + k + 1);
-#pragma unroll
-        for (int s = 0; s < 4; ++s)
-            if (!approx(d0[s], w.v[s] - u.v[s])) ok &= ~(1 << s);
+    for (int s = 0; s < 4; ++s) {
+        f0[s] = val(s, 0);
+        d0[s] = val(s, 1) - f0[s];
     }
-#pragma unroll
-    for (int s = 0; s < 4; ++s)
-        if (!(ok & (1 << s))) atomicAnd(&ranges[s], 0);
     __syncthreads();
-    bool rng[4];
+    for (int64_t k0 = 0; k0 < K; k0 += kWG) {
+        const int64_t k = k0 + threadIdx.x;
+        int ok = 0xF;
+        if (k < K) {
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+                if (!approx(d0[s], val(s, k + 1) - val(s, k))) ok &= ~(1 << s);
+        }
+        if (ok != 0xF) atomicAnd(&ranges, ok);
+        __syncthreads();
+        const int left = ranges;
+        __syncthreads();
+        if (!left) break;                                       // no series is a range
+    }
+    const int rng = ranges;
     double start[4], rstep[4];
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
-        rng[s] = ranges[s] != 0;
-        start[s] = f0.v[s] + d0[s] / 2.0;
-        const double stop = fl.v[s] - d0[s] / 2.0;
+        start[s] = f0[s] + d0[s] / 2.0;
+        const double stop = val(s, K) - d0[s] / 2.0;
         rstep[s] = K > 1 ? (stop - start[s]) / (double)(K - 1) : 0.0;
     }
     const double nm = a.norm[t], mm = a.mean_mass[t];
     const int64_t kbase = a.koff[t];
     int flags = 0;
     unsigned long long cnt = 0;
-    for (int64_t k = threadIdx.x; k < K; k += kWG) {
-        const int64_t q = q0 + k;
-        const PointVals u = point_vals(a, q), w = point_vals(a, q + 1);
+    for (int64_t k = (int64_t)blockIdx.y * kWG + threadIdx.x; k < K; k += (int64_t)gridDim.y * kWG) {
         double mid[4];
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
-            if (rng[s]) mid[s] = K == 1 ? start[s] : start[s] + (double)k * rstep[s];
-            else mid[s] = u.v[s] + (w.v[s] - u.v[s]) / 2.0;       // v[i] + d[i] / 2 :430
+            const double u = val(s, k), w = val(s, k + 1);
+            if (rng >> s & 1) mid[s] = K == 1 ? start[s] : start[s] + (double)k * rstep[s];
+            else mid[s] = u + (w - u) / 2.0;                     // v[i] + d[i] / 2 :430
         }
         // calculate_weights :770-773 (completeness of the left point)
-        const double m0 = a.mini[q], m1 = a.mini[q + 1];
+        const double m0 = a.mini[q0 + k], m1 = a.mini[q0 + k + 1];
         if (!(m1 > m0)) flags |= kBadDuplicate;
-        double wt = (m1 - m0) * (eval(a.imf, m0) + eval(a.imf, m1)) / 2.0;
-        wt = wt * (u.compl_ * nm / mm);
+        double wt = (m1 - m0) * (val(kPdf, k) + val(kPdf, k + 1)) / 2.0;
+        wt = wt * (val(kCompl, k) * nm / mm);
         psf::PointDesc d;
         const bool fin = isfinite(mid[0]) && isfinite(mid[1]) && isfinite(mid[2]) && isfinite(mid[3]) && isfinite(wt);
         if (!fin) {
@@ -323,8 +330,7 @@ __global__ __launch_bounds__(kWG) void k_pcs_desc(Args a)
         a.desc[kbase + k] = d;
         a.keys[kbase + k] = psf::point_key(d, (int)(a.ex.length - 1), a.cov_mult == 0.0);
     }
-    for (int off = 32; off > 0; off >>= 1) cnt += __shfl_xor(cnt, off, 64);
-    if ((threadIdx.x & 63) == 0 && cnt) atomicAdd(a.pairs, cnt);
+    psf::add_count(a.pairs, blockIdx.x * gridDim.y + blockIdx.y, cnt);
     if (flags) atomicOr(a.bad, flags);
 }
 
@@ -508,10 +514,10 @@ int sfh_partial_cmd_smooth_batch(sfh_ctx* ctx, int64_t ntemplates, const int64_t
     a.ey = psf::Range{yedges.first, yedges.step, yedges.length};
     void *pc = nullptr, *pcnt = nullptr;
     if (int rc = scratch(ctx, "pcs_counts", (size_t)ntemplates * sizeof(int64_t), &pc)) return rc;
-    if (int rc = scratch(ctx, "pcs_flags", 64, &pcnt)) return rc;
-    SFH_HIP_TRY(ctx, hipMemsetAsync(pcnt, 0, 64, s));
-    a.pairs = (unsigned long long*)pcnt;
-    a.bad = (int*)((char*)pcnt + 16);
+    if (int rc = scratch(ctx, "pcs_flags", sizeof(psf::PointCounts), &pcnt)) return rc;
+    SFH_HIP_TRY(ctx, hipMemsetAsync(pcnt, 0, sizeof(psf::PointCounts), s));
+    a.pairs = ((psf::PointCounts*)pcnt)->pairs;
+    a.bad = &((psf::PointCounts*)pcnt)->bad;
 
     // 1. resampled point counts
     {
@@ -532,17 +538,19 @@ int sfh_partial_cmd_smooth_batch(sfh_ctx* ctx, int64_t ntemplates, const int64_t
     }
     const int64_t Q = qoff[ntemplates], K = koff[ntemplates];
     SFH_ARG_CHECK(ctx, Q < ((int64_t)1 << 34), "too many resampled points (%lld)", (long long)Q);
-    void *dq = nullptr, *dk = nullptr, *dmini = nullptr, *diso = nullptr, *ddesc = nullptr;
+    void *dq = nullptr, *dk = nullptr, *dmini = nullptr, *diso = nullptr, *dvals = nullptr, *ddesc = nullptr;
     if (int rc = upload_scratch(ctx, "pcs_qoff", qoff.data(), qoff.size() * sizeof(int64_t), &dq)) return rc;
     if (int rc = upload_scratch(ctx, "pcs_koff", koff.data(), koff.size() * sizeof(int64_t), &dk)) return rc;
     if (int rc = scratch(ctx, "pcs_mini", (size_t)(Q + 1) * sizeof(double), &dmini)) return rc;
     if (int rc = scratch(ctx, "pcs_iso", (size_t)(Q + 1) * 3 * sizeof(double), &diso)) return rc;
+    if (int rc = scratch(ctx, "pcs_vals", (size_t)(Q + 1) * kVals * sizeof(double), &dvals)) return rc;
     if (int rc = scratch(ctx, "dep_desc", (size_t)(K + 1) * (sizeof(psf::PointDesc) + sizeof(psf::PointKey)), &ddesc))
         return rc;
     a.qoff = (const int64_t*)dq;
     a.koff = (const int64_t*)dk;
     a.mini = (double*)dmini;
     a.iso = (double*)diso;
+    a.vals = (double*)dvals;
     a.qtotal = Q;
     a.desc = (psf::PointDesc*)ddesc;
     a.keys = (psf::PointKey*)(a.desc + K + 1);
@@ -555,7 +563,9 @@ int sfh_partial_cmd_smooth_batch(sfh_ctx* ctx, int64_t ntemplates, const int64_t
     if (int rc = check_launch(ctx, "k_pcs_points")) return rc;
     {
         TimedLaunch tl(ctx, "pcs_desc");
-        hipLaunchKernelGGL(k_pcs_desc, dim3((unsigned)ntemplates), dim3(kWG), 0, s, a);
+        if (Q > 0) hipLaunchKernelGGL(k_pcs_vals, dim3((unsigned)cdiv(Q, kWG)), dim3(kWG), 0, s, a);
+        const int64_t nsplit = std::min<int64_t>(std::max<int64_t>(cdiv(K, ntemplates * kWG), 1), 1024);
+        hipLaunchKernelGGL(k_pcs_desc, dim3((unsigned)ntemplates, (unsigned)nsplit), dim3(kWG), 0, s, a);
     }
     if (int rc = check_launch(ctx, "k_pcs_desc")) return rc;
     // 4. deposition into the device output (or a staging buffer for `out`)
@@ -569,18 +579,17 @@ int sfh_partial_cmd_smooth_batch(sfh_ctx* ctx, int64_t ntemplates, const int64_t
     if (int rc = deposit_from_desc(ctx, ddesc, a.keys, (const int64_t*)dk, ntemplates, K, a.cov_mult == 0.0, xedges,
                                    yedges, dst, ld))
         return rc;
-    unsigned long long pairs = 0;
-    SFH_HIP_TRY(ctx, hipMemcpyAsync(&bad, a.bad, sizeof(int), hipMemcpyDeviceToHost, s));
-    SFH_HIP_TRY(ctx, hipMemcpyAsync(&pairs, a.pairs, sizeof(pairs), hipMemcpyDeviceToHost, s));
+    psf::PointCounts hc;
+    SFH_HIP_TRY(ctx, hipMemcpyAsync(&hc, pcnt, sizeof(hc), hipMemcpyDeviceToHost, s));
     if (out) {
         SFH_HIP_TRY(ctx, hipMemcpy2DAsync(out, (size_t)nbins * sizeof(float), dst, (size_t)ld * sizeof(float),
                                           (size_t)nbins * sizeof(float), (size_t)ntemplates, hipMemcpyDeviceToHost,
                                           s));
     }
     SFH_HIP_TRY(ctx, hipStreamSynchronize(s));
-    if (bad) return pcs_error(ctx, bad);
+    if (hc.bad) return pcs_error(ctx, hc.bad);
     if (npoints_out) *npoints_out = K;
-    if (pairs_out) *pairs_out = (int64_t)pairs;
+    if (pairs_out) *pairs_out = hc.total();
     return SFH_OK;
 }
 
