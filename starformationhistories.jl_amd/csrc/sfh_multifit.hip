@@ -308,23 +308,39 @@ __device__ inline double block_max(double v, double* red)
 }
 
 // Per-fit reduction of the item partials: negLL (+Inf for an exact zero sum,
-// fitting_base.jl:95) and G.
+// fitting_base.jl:95) and G.  Workgroup (f, w): templates 16 w .. 16 w + 15 of
+// fit f, thread = 16 item slices x 16 templates as k_single_reduce.  Latency
+// bound: one workgroup per fit with a thread per template walked a fit's
+// items (up to some hundred) one load after another, 161 us for 64 fits of
+// 50-700 templates x 5k-60k bins; 9 us with the items spread over 16 threads.
 __global__ __launch_bounds__(kWG) void k_multi_reduce(const FitDesc* __restrict__ fits, const double* __restrict__ ll_part,
                                                       const double* __restrict__ g_part, double* __restrict__ negLL,
                                                       double* __restrict__ G)
 {
+    __shared__ double sh[kWG];
+    __shared__ double red[4];
     const FitDesc fd = fits[blockIdx.x];
-    if (threadIdx.x == 0) {
-        double s = 0.0;
-        for (int64_t i = 0; i < fd.nitems; ++i) s += ll_part[fd.item0 + i];
-        negLL[blockIdx.x] = (s != 0.0) ? -s : INFINITY;
+    const int tt = threadIdx.x & 15, sl = threadIdx.x >> 4;
+    if (blockIdx.y == 0) {
+        double v = 0.0;
+        for (int64_t i = threadIdx.x; i < fd.nitems; i += kWG) v += ll_part[fd.item0 + i];
+        const double s = block_sum(v, red);
+        if (threadIdx.x == 0) negLL[blockIdx.x] = (s != 0.0) ? -s : INFINITY;
     }
-    if (G) {
-        for (int64_t t = threadIdx.x; t < fd.T; t += kWG) {
-            double s = 0.0;
-            for (int64_t i = 0; i < fd.nitems; ++i) s += g_part[fd.poff + i * fd.T + t];
-            G[fd.xoff + t] = s;
-        }
+    const int64_t t = (int64_t)blockIdx.y * 16 + tt;
+    if (!G || (int64_t)blockIdx.y * 16 >= fd.T) return;
+    double v = 0.0;
+    if (t < fd.T) {
+#pragma unroll 8
+        for (int64_t i = sl; i < fd.nitems; i += 16) v += g_part[fd.poff + i * fd.T + t];
+    }
+    sh[threadIdx.x] = v;
+    __syncthreads();
+    if (sl == 0 && t < fd.T) {
+        double g = sh[tt];
+#pragma unroll
+        for (int k = 1; k < 16; ++k) g += sh[16 * k + tt];
+        G[fd.xoff + t] = g;
     }
 }
 
@@ -585,6 +601,7 @@ __global__ __launch_bounds__(kWG) void k_opt_accept(OptParams p)
     // objective and gradient in the transformed variables at the trial point
     if (threadIdx.x == 0) {
         double s = 0.0;
+#pragma unroll 8
         for (int64_t i = 0; i < fd.nitems; ++i) s += p.ll_part[fd.item0 + i];
         sll = (s != 0.0) ? -s : INFINITY;
     }
@@ -592,7 +609,8 @@ __global__ __launch_bounds__(kWG) void k_opt_accept(OptParams p)
     double thsum = 0.0, gd = 0.0;
     for (int t = threadIdx.x; t < T; t += kWG) {
         double G = 0.0;
-        for (int64_t i = 0; i < fd.nitems; ++i) G += p.g_part[fd.poff + i * T + t];
+#pragma unroll 8
+        for (int64_t i = 0; i < fd.nitems; ++i) G += p.g_part[fd.poff + i * T + t];   // loads eight at a time
         const double tt = init ? th[t] : fma(a, d[t], th[t]);
         double v;
         if (p.transform == SFH_FIT_LOG) v = map ? G * x[t] - 1.0 : G * x[t];   // solvers.jl:185-187, 193-195
@@ -1172,8 +1190,8 @@ int fg_device_impl(sfh_multifit* mf, const double* d_X, double eps, double eps_g
     if (int rc = check_launch(ctx, "k_multi_fg")) return rc;
     {
         TimedLaunch tl(ctx, "multifit_reduce");
-        hipLaunchKernelGGL(k_multi_reduce, dim3((unsigned)mf->nfits), dim3(kWG), 0, ctx->stream, mf->d_fits, mf->d_llp,
-                           mf->d_gp, d_negLL, d_G);
+        const dim3 grid((unsigned)mf->nfits, (unsigned)(d_G ? cdiv(mf->maxT, 16) : 1));
+        hipLaunchKernelGGL(k_multi_reduce, grid, dim3(kWG), 0, ctx->stream, mf->d_fits, mf->d_llp, mf->d_gp, d_negLL, d_G);
     }
     return check_launch(ctx, "k_multi_reduce");
 }
