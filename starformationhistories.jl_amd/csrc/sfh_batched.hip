@@ -342,9 +342,11 @@ __device__ inline void wait_vmcnt(int n)
     case 2: __builtin_amdgcn_s_waitcnt(0xF72); break;
     case 3: __builtin_amdgcn_s_waitcnt(0xF73); break;
     case 4: __builtin_amdgcn_s_waitcnt(0xF74); break;
+    case 5: __builtin_amdgcn_s_waitcnt(0xF75); break;
     case 6: __builtin_amdgcn_s_waitcnt(0xF76); break;
     case 8: __builtin_amdgcn_s_waitcnt(0xF78); break;
     case 9: __builtin_amdgcn_s_waitcnt(0xF79); break;
+    case 10: __builtin_amdgcn_s_waitcnt(0xF7A); break;
     case 12: __builtin_amdgcn_s_waitcnt(0xF7C); break;
     default: __builtin_amdgcn_s_waitcnt(0xF70); break;
     }
@@ -391,7 +393,7 @@ __device__ inline void static_for(F&& f)
 // reused by its ~32 resident workgroups.
 struct Swizzle {
     int nrt, nct, gr, gc, nsr, nsc;
-    int xsplit;     // split-K launches: 1-D grid, XCD x runs splits x, x + 8, ... (nsplit % 8 == 0)
+    int xsplit;     // split-K launches: the number of splits; XCD x runs splits x, x + 8, ...
 };
 
 __device__ inline bool swizzle(const Swizzle& s, int64_t id, int* rt, int* ct)
@@ -415,7 +417,7 @@ struct EpiLL {
     double eps_g;            // R clamp: eps(eltype(composite))
     double eps_hi;           // max(eps, eps_g): below it R is recomputed with eps_g
     double* ll_part;         // [row tile][Bpad]
-    uint4* R;                // gradient B operand tiles [kb2][cb][2][64]
+    uint4* R;                // gradient B operand tiles [kb2][cb][2][64], or NULL
     int64_t ncb;             // column blocks (Bpad/32)
     int64_t Bpad;
 };
@@ -479,10 +481,11 @@ __global__ __launch_bounds__(WR * WC * 64, 1) void k_gemm(const uint4* __restric
         const int64_t id = blockIdx.x, tiles = (int64_t)sw.nrt * sw.nct;
         const int64_t local = id >> 3, tile = local % tiles;
         split = (local / tiles) * 8 + (id & 7);
+        if (split >= sw.xsplit) return;         // the grid is padded to whole rounds of 8 splits
         ct = (int)(tile / sw.nrt);
         rt = (int)(tile % sw.nrt);
     } else {
-        split = blockIdx.y;
+        split = 0;
         if (!swizzle(sw, blockIdx.x, &rt, &ct)) return;
     }
     const int64_t kb0 = split * kb_per_split;
@@ -620,6 +623,7 @@ __global__ __launch_bounds__(WR * WC * 64, 1) void k_gemm(const uint4* __restric
                     }
                     rv[i] = r;
                 }
+                if (!el.R) continue;            // log-likelihood only
                 // R fragments: K-blocks 2*rbk (i = 0..7) and 2*rbk+1 (i = 8..15)
 #pragma unroll
                 for (int half = 0; half < 2; ++half) {
@@ -685,28 +689,29 @@ __global__ __launch_bounds__(WR * WC * 64, 1) void k_gemm(const uint4* __restric
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 typedef double f64x2 __attribute__((ext_vector_type(2)));
 
-// Coefficients X (T x B, column-major FP64) -> [kblock][col tile][16 k][128 walkers] FP64.
+// Coefficients X (T x B, column-major FP64) -> [kblock][col tile][16 k][CN walkers] FP64.
 // One workgroup per (kblock, col tile): reads run along the templates (16
 // consecutive t of a walker, 128 bytes), writes along the walkers, through an
 // LDS tile.
+template <int CN>
 __global__ __launch_bounds__(256) void k_prep_x64(const double* __restrict__ X, int64_t T, int64_t B,
                                                   int64_t nct, int64_t nkb, double* __restrict__ out)
 {
-    __shared__ double tile[16][kBN + 1];
+    __shared__ double tile[16][CN + 1];
     const int64_t ct = blockIdx.x % nct, kb = blockIdx.x / nct;
 #pragma unroll
-    for (int j = 0; j < 16 * kBN / 256; ++j) {
+    for (int j = 0; j < 16 * CN / 256; ++j) {
         const int idx = threadIdx.x + 256 * j;
         const int c = idx / 16, k = idx % 16;
-        const int64_t t = kb * 16 + k, w = ct * kBN + c;
+        const int64_t t = kb * 16 + k, w = ct * CN + c;
         tile[k][c] = (t < T && w < B) ? X[w * T + t] : 0.0;
     }
     __syncthreads();
-    double* o = out + (kb * nct + ct) * 16 * kBN;
+    double* o = out + (kb * nct + ct) * 16 * CN;
 #pragma unroll
-    for (int j = 0; j < 16 * kBN / 256; ++j) {
+    for (int j = 0; j < 16 * CN / 256; ++j) {
         const int idx = threadIdx.x + 256 * j;
-        o[idx] = tile[idx / kBN][idx % kBN];
+        o[idx] = tile[idx / CN][idx % CN];
     }
 }
 
@@ -719,25 +724,30 @@ __device__ inline int a_elem(int r, int k)
 }
 
 // Composite on the FP64 matrix cores + the same log-likelihood / R epilogue as
-// k_gemm<LL>.  Workgroup tile 128 bins x 128 walkers, 4 waves of 64 x 64, each
-// wave 4 x 4 v_mfma_f64_16x16x4f64 tiles (lane l: A[row l%16][k l/16],
+// k_gemm<LL>.  Workgroup tile BM bins x CN walkers: 2 x 2 waves of 64 x 64 for
+// CN = 128, 4 x 1 waves of BM / 4 x CN for fewer, each wave TA x TB
+// v_mfma_f64_16x16x4f64 tiles (lane l: A[row l%16][k l/16],
 // B[k l/16][col l%16], D[row l/16 + 4i][col l%16] in accumulator i).  A (FP32 fragment tiles)
 // and X (FP64) K-blocks go global -> registers (two K-blocks ahead, two staging
 // sets) -> one of two LDS stages; the R tile is re-laid out through LDS into the
 // gradient GEMM's fragment tiles.
+template <int CN, int BM>
 __global__ __launch_bounds__(kWG, 1) void k_gemm_f64_ll(const uint4* __restrict__ A_, const double* __restrict__ X,
                                                         int64_t nrb_total, int64_t nct_total, int64_t nkb,
                                                         Swizzle sw, EpiLL el)
 {
-    constexpr int CA = kRB * 2;                 // 8 KiB: FP32 A tile of one K-block (two halves per rowblock)
-    constexpr int CX = 16;                      // 16 KiB: one 128-walker FP64 row per k
+    constexpr int RB = BM / 32;
+    constexpr int CA = RB * 2;                  // 8 or 4 KiB: FP32 A tile of one K-block (two halves per rowblock)
+    constexpr int CX = CN / 8;                  // 16, 8 or 4 KiB: one CN-walker FP64 row per k
+    constexpr int WC = CN == 128 ? 2 : 1, WR = 4 / WC;          // waves along walkers, along bins
+    constexpr int TA = BM / WR / 16, TB = CN / WC / 16;        // a wave's tiles of 16 bins x 16 walkers
     constexpr int STAGE_U4 = (CA + CX) * 64;    // 1536 16-byte words per K-block
-    constexpr int NPER = STAGE_U4 / kWG;        // 6 per thread
-    constexpr int NPA = CA * 64 / kWG;          // the first 2 of them from the A tile
+    constexpr int NPER = STAGE_U4 / kWG;        // 6, 4 or 2 per thread
+    constexpr int NPA = CA * 64 / kWG;          // the first 2 (or 1) of them from the A tile
     static_assert(STAGE_U4 % kWG == 0 && (CA * 64) % kWG == 0, "stage split");
-    // two LDS stages (48 KiB) during the K loop; the 128 x 128 FP32 R tile (64 KiB) afterwards
-    __shared__ u32x4 lds[4096];
-    __shared__ double sLL[kWR][kBN];
+    // two LDS stages (up to 48 KiB) during the K loop; the BM x CN FP32 R tile (up to 64 KiB) afterwards
+    __shared__ u32x4 lds[2 * STAGE_U4 > BM * CN / 4 ? 2 * STAGE_U4 : BM * CN / 4];
+    __shared__ double sLL[WR][CN];
     float* sR = reinterpret_cast<float*>(lds);
 
     int rt, ct;
@@ -745,17 +755,17 @@ __global__ __launch_bounds__(kWG, 1) void k_gemm_f64_ll(const uint4* __restrict_
     const u32x4* A = reinterpret_cast<const u32x4*>(A_);
     const u32x4* Xv = reinterpret_cast<const u32x4*>(X);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wr = wave / kWC, wc = wave % kWC;
+    const int wr = wave / WC, wc = wave % WC;
     const int lr = lane & 15, lk = lane >> 4;
 
-    f64x4 acc[4][4];
+    f64x4 acc[TA][TB];
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
+    for (int a = 0; a < TA; ++a)
 #pragma unroll
-        for (int b = 0; b < 4; ++b) acc[a][b] = f64x4{0.0, 0.0, 0.0, 0.0};
+        for (int b = 0; b < TB; ++b) acc[a][b] = f64x4{0.0, 0.0, 0.0, 0.0};
 
     // element u of a stage: the A tile (contiguous) then the X rows (contiguous)
-    const int64_t a_row0 = (int64_t)rt * kRB * 2 * 64;
+    const int64_t a_row0 = (int64_t)rt * CA * 64;
     const int64_t a_stride = nrb_total * 2 * 64, x_stride = nct_total * CX * 64;
     const u32x4* x0 = Xv + (int64_t)ct * CX * 64;
 #define SFH_GLOAD(kb, R)                                                                         \
@@ -772,27 +782,27 @@ __global__ __launch_bounds__(kWG, 1) void k_gemm_f64_ll(const uint4* __restrict_
         const float* cA = reinterpret_cast<const float*>(lds + st * STAGE_U4);
         const double* cX = reinterpret_cast<const double*>(lds + st * STAGE_U4 + CA * 64);
         // fragments of step ks + 1 are read while step ks's products run
-        float ga[2][4];
-        double fb[2][4];
+        float ga[2][TA];
+        double fb[2][TB];
         auto rd = [&](int ks, int s) {
             const int k = 4 * ks + lk;
 #pragma unroll
-            for (int a = 0; a < 4; ++a) ga[s][a] = cA[a_elem(wr * 64 + a * 16 + lr, k)];
+            for (int a = 0; a < TA; ++a) ga[s][a] = cA[a_elem((wr * TA + a) * 16 + lr, k)];
 #pragma unroll
-            for (int b = 0; b < 4; ++b) fb[s][b] = cX[k * kBN + wc * 64 + b * 16 + lr];
+            for (int b = 0; b < TB; ++b) fb[s][b] = cX[k * CN + (wc * TB + b) * 16 + lr];
         };
         rd(0, 0);
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
             const int s = ks & 1;
             if (ks < 3) rd(ks + 1, s ^ 1);
-            double fa[4];
+            double fa[TA];
 #pragma unroll
-            for (int a = 0; a < 4; ++a) fa[a] = (double)ga[s][a];
+            for (int a = 0; a < TA; ++a) fa[a] = (double)ga[s][a];
 #pragma unroll
-            for (int a = 0; a < 4; ++a)
+            for (int a = 0; a < TA; ++a)
 #pragma unroll
-                for (int b = 0; b < 4; ++b)
+                for (int b = 0; b < TB; ++b)
                     acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[a], fb[s][b], acc[a][b], 0, 0, 0);
         }
     };
@@ -830,48 +840,54 @@ __global__ __launch_bounds__(kWG, 1) void k_gemm_f64_ll(const uint4* __restrict_
     __syncthreads();    // every wave is done with the stages before they become the R tile
 
     // epilogue: LL terms (FP64) and R into LDS
-    double part[4] = {0.0, 0.0, 0.0, 0.0};
+    double part[TB] = {};
 #pragma unroll
-    for (int a = 0; a < 4; ++a) {
+    for (int a = 0; a < TA; ++a) {
 #pragma unroll
-        for (int b = 0; b < 4; ++b) {
-            const int cl = wc * 64 + b * 16 + lr;                 // walker within the tile
-            const int64_t w = (int64_t)ct * kBN + cl;
+        for (int b = 0; b < TB; ++b) {
+            const int cl = (wc * TB + b) * 16 + lr;               // walker within the tile
+            const int64_t w = (int64_t)ct * CN + cl;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const int rl = wr * 64 + a * 16 + lk + 4 * i;     // bin within the tile
-                const int64_t bin = (int64_t)rt * kBM + rl;
+                const int rl = (wr * TA + a) * 16 + lk + 4 * i;   // bin within the tile
+                const int64_t bin = (int64_t)rt * BM + rl;
                 float r = 0.f;
                 if (bin < el.nbins && w < el.B) {
                     const double m = acc[a][b][i];
                     ll_r_term(el, el.data[bin], m, part[b], r);
                 }
-                sR[rl * kBN + cl] = r;
+                sR[rl * CN + cl] = r;
             }
         }
     }
 #pragma unroll
-    for (int b = 0; b < 4; ++b) {
+    for (int b = 0; b < TB; ++b) {
         part[b] += __shfl_xor(part[b], 16, 64);
         part[b] += __shfl_xor(part[b], 32, 64);
-        if (lk == 0) sLL[wr][wc * 64 + b * 16 + lr] = part[b];
+        if (lk == 0) sLL[wr][(wc * TB + b) * 16 + lr] = part[b];
     }
     __syncthreads();
-    for (int k = tid; k < kBN; k += kWG)
-        el.ll_part[(int64_t)rt * el.Bpad + (int64_t)ct * kBN + k] = sLL[0][k] + sLL[1][k];
-    // R fragments: 8 K-blocks x 4 column blocks x 64 lanes per tile
-    for (int item = tid; item < 8 * kCB * 64; item += kWG) {
-        const int lp = item & 63, cbl = (item >> 6) % kCB, kbl = (item >> 6) / kCB;
+    for (int k = tid; k < CN; k += kWG) {
+        double s = sLL[0][k];
+#pragma unroll
+        for (int r = 1; r < WR; ++r) s += sLL[r][k];
+        el.ll_part[(int64_t)rt * el.Bpad + (int64_t)ct * CN + k] = s;
+    }
+    if (!el.R) return;                          // log-likelihood only
+    // R fragments: BM / 16 K-blocks x CN / 32 column blocks x 64 lanes per tile
+    constexpr int CBT = CN / 32;
+    for (int item = tid; item < BM / 16 * CBT * 64; item += kWG) {
+        const int lp = item & 63, cbl = (item >> 6) % CBT, kbl = (item >> 6) / CBT;
         const int cl = cbl * 32 + (lp & 31), hp = lp >> 5;
         uint16_t h0[8], h1[8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
             uint16_t s2[2];
-            split_f32<2>(sR[(kbl * 16 + gperm(hp, j)) * kBN + cl], s2);
+            split_f32<2>(sR[(kbl * 16 + gperm(hp, j)) * CN + cl], s2);
             h0[j] = s2[0];
             h1[j] = s2[1];
         }
-        const int64_t kb2 = (int64_t)rt * 8 + kbl, cb = (int64_t)ct * kCB + cbl;
+        const int64_t kb2 = (int64_t)rt * (BM / 16) + kbl, cb = (int64_t)ct * CBT + cbl;
         uint4* o = el.R + ((kb2 * el.ncb + cb) * 2) * 64 + lp;
         o[0] = pack8(h0);
         o[64] = pack8(h1);
@@ -882,8 +898,14 @@ __global__ __launch_bounds__(kWG, 1) void k_gemm_f64_ll(const uint4* __restrict_
 // for an exact 0, fitting_base.jl:95), 16 walkers x 16 row slices per
 // workgroup (slice s sums rows s, s + 16, ... in order; the slices then add in
 // order).  The rest: G[t + T*b] = sum_split gpart[split][b][t] (the gradient
-// of -logL), one element per thread.
+// of -logL), 64 elements per workgroup x 4 split slices (slice s sums splits
+// s, s + 4, ... in order; the slices then add in order).  One thread per
+// element walked up to 64 splits one load after another: 20 us for 24 walkers
+// of 700 templates, 5 us now.
+// Where there are elements enough to fill the chip without that (SL = 1),
+// one thread per element stays the faster form (30 against 40 us for 4096 walkers).
 constexpr int kFinW = 16, kFinS = 16;
+template <int SL>
 __global__ __launch_bounds__(256) void k_finish(const double* __restrict__ ll_part, int64_t nrt,
                                                 const float* __restrict__ gpart, int nsplit, int64_t T,
                                                 int64_t B, int64_t Bpad, int64_t Tpad2, int64_t nll_blocks,
@@ -908,13 +930,25 @@ __global__ __launch_bounds__(256) void k_finish(const double* __restrict__ ll_pa
         }
         return;
     }
-    const int64_t g = ((int64_t)blockIdx.x - nll_blocks) * 256 + threadIdx.x;
-    if (G && g < T * B) {
+    constexpr int NE = 256 / SL;
+    __shared__ double part[SL][NE];
+    const int e = threadIdx.x % NE, sl = threadIdx.x / NE;
+    const int64_t g = ((int64_t)blockIdx.x - nll_blocks) * NE + e;
+    double s = 0.0;
+    if (g < T * B) {
         const int64_t b = g / T, t = g - b * T;
-        double s = 0.0;
-        for (int k = 0; k < nsplit; ++k) s += (double)gpart[((int64_t)k * Bpad + b) * Tpad2 + t];
-        G[g] = s;
+        const float* p = gpart + b * Tpad2 + t;
+#pragma unroll 8
+        for (int k = sl; k < nsplit; k += SL) s += (double)p[k * Bpad * Tpad2];
     }
+    if constexpr (SL > 1) {
+        part[sl][e] = s;
+        __syncthreads();
+        if (sl > 0) return;
+#pragma unroll
+        for (int k = 1; k < SL; ++k) s += part[k][e];
+    }
+    if (g < T * B) G[g] = s;
 }
 
 }  // namespace bat
@@ -1031,22 +1065,29 @@ static int fg_batched_impl(sfh_ctx* ctx, const sfh_templates* tpl, const sfh_dat
     BatchedOperands* ops = nullptr;
     if (int rc = get_operands(ctx, tpl, mode, &ops)) return rc;
     const int64_t N = tpl->nbins, T = tpl->ntemplates;
-    const int64_t Bpad = cdiv(B, kBN) * kBN;
-    const int64_t nrb1 = ops->npad / 32, nkb1 = ops->tpad1 / 16, ncb = Bpad / 32, nct = Bpad / kBN;
-    const int64_t nkb2 = ops->npad / 16, nrt1 = ops->npad / kBM;
+    // walkers per composite tile: 128, or for few of them a narrower FP64 tile (a
+    // tile's walkers past B are matrix-core work for nothing: 24 walkers of 700
+    // templates x 60,000 bins took 200 us in 128-wide tiles, 65 us in 128 x 32 and
+    // 62 us in 64 x 32 ones, whose 938 workgroups balance better)
+    const int cn = mode == F64 && B <= 32 ? 32 : mode == F64 && B <= 64 ? 64 : kBN;
+    const int64_t Bpad = cdiv(B, cn) * cn;
+    const int64_t nrb1 = ops->npad / 32, nkb1 = ops->tpad1 / 16, ncb = Bpad / 32, nct = Bpad / cn;
+    const int64_t nkb2 = ops->npad / 16, nrt1 = ops->npad / (cn == 32 ? 64 : kBM);
 
     void *px = nullptr, *pr = nullptr, *pll = nullptr, *pg = nullptr;
-    const size_t xbytes = mode == F64 ? (size_t)nkb1 * nct * 16 * kBN * sizeof(double)
+    const size_t xbytes = mode == F64 ? (size_t)nkb1 * nct * 16 * cn * sizeof(double)
                                       : (size_t)nkb1 * ncb * 2 * 64 * sizeof(uint4);
     if (int rc = scratch(ctx, "bat_x", xbytes, &px)) return rc;
-    if (int rc = scratch(ctx, "bat_r", (size_t)nkb2 * ncb * 2 * 64 * sizeof(uint4), &pr)) return rc;
+    if (d_G)
+        if (int rc = scratch(ctx, "bat_r", (size_t)nkb2 * ncb * 2 * 64 * sizeof(uint4), &pr)) return rc;
     if (int rc = scratch(ctx, "bat_ll", (size_t)nrt1 * Bpad * sizeof(double), &pll)) return rc;
 
     {
         TimedLaunch tl(ctx, "batched_prep_x");
         if (mode == F64) {
-            hipLaunchKernelGGL(k_prep_x64, dim3((unsigned)(nkb1 * nct)), dim3(256), 0, ctx->stream, d_X, T, B, nct,
-                               nkb1, (double*)px);
+            hipLaunchKernelGGL(cn == 32 ? k_prep_x64<32> : cn == 64 ? k_prep_x64<64> : k_prep_x64<128>,
+                               dim3((unsigned)(nkb1 * nct)), dim3(256), 0, ctx->stream, d_X, T, B, nct, nkb1,
+                               (double*)px);
         } else {
             const int64_t n = nkb1 * ncb * 64;
             const dim3 grid((unsigned)cdiv(n, 256));
@@ -1064,10 +1105,11 @@ static int fg_batched_impl(sfh_ctx* ctx, const sfh_templates* tpl, const sfh_dat
         EpiLL el{data->d_data, N, B, eps, eps_g, eps > eps_g ? eps : eps_g, (double*)pll, (uint4*)pr, ncb, Bpad};
         EpiGrad eg{};
         const dim3 grid(swizzle_grid(sw), 1);
+        const auto f64 = cn == 32 ? k_gemm_f64_ll<32, 64> : cn == 64 ? k_gemm_f64_ll<64, kBM> : k_gemm_f64_ll<kBN, kBM>;
         TimedLaunch tl(ctx, "batched_composite_ll");
         if (mode == F64)
-            hipLaunchKernelGGL(k_gemm_f64_ll, grid, dim3(kWG), 0, ctx->stream, ops->a1[0], (const double*)px, nrb1,
-                               nct, nkb1, sw, el);
+            hipLaunchKernelGGL(f64, grid, dim3(kWG), 0, ctx->stream, ops->a1[0], (const double*)px, nrb1, nct, nkb1, sw,
+                               el);
         else if (mode == FP32)
             hipLaunchKernelGGL((k_gemm<FP32, true>), grid, dim3(kWG), 0, ctx->stream, ops->a1[0], (const uint4*)px,
                                nrb1, ncb, nkb1, nkb1, sw, el, eg);
@@ -1081,16 +1123,21 @@ static int fg_batched_impl(sfh_ctx* ctx, const sfh_templates* tpl, const sfh_dat
     if (d_G) {
         // 256 x 128 tiles (4 x 2 waves), one 512-thread workgroup per CU; the
         // bins are split so the workgroups fill whole waves of the 256 CUs
-        constexpr int GWR = 4, GWC = 2, GRB = kTR * GWR, GCB = kTC * GWC;
+        // (for 64 walkers or fewer 256 x 64 tiles of 4 x 1 waves: bound by one read
+        // of the templates, 34 us at the copy rate; 56 -> 40 us for 24 walkers)
+        constexpr int GWR = 4, GRB = kTR * GWR;
+        const bool narrow = ncb <= kTC;
+        const int gwc = narrow ? 1 : 2, GCB = kTC * gwc;
         const int64_t nrb2 = ops->tpad2 / 32;
         const int nrt = (int)cdiv(nrb2, GRB), nct2 = (int)cdiv(ncb, GCB);
         const int64_t tiles = (int64_t)nrt * nct2;
         int best = 1;
         double best_cost = 1e300;
-        for (int ns = 1; ns <= 64 && ns <= std::max<int64_t>(1, nkb2 / 32); ++ns) {
-            const int64_t wg = tiles * ns;
-            const double waves = (double)cdiv(wg, 256);
-            // time ~ waves of workgroups x K-blocks per workgroup
+        const int most = narrow ? 128 : 64;
+        for (int ns = 1; ns <= most && ns <= std::max<int64_t>(1, nkb2 / 32); ++ns) {
+            // time ~ rounds of workgroups on an XCD's 32 CUs x K-blocks per workgroup
+            // (XCD x runs splits x, x + 8, ...)
+            const double waves = (double)cdiv(tiles * cdiv(ns, 8), 32);
             const double cost = waves * (double)cdiv(nkb2, ns);
             if (cost < best_cost * 0.999) {
                 best_cost = cost;
@@ -1100,27 +1147,27 @@ static int fg_batched_impl(sfh_ctx* ctx, const sfh_templates* tpl, const sfh_dat
         const int64_t kps = cdiv(nkb2, best);
         nsplit = (int)cdiv(nkb2, kps);
         if (int rc = scratch(ctx, "bat_g", (size_t)nsplit * Bpad * ops->tpad2 * sizeof(float), &pg)) return rc;
-        Swizzle sw = make_swizzle(nrt, nct2, nrt, std::max(1, 8 / nrt));
-        dim3 grid(swizzle_grid(sw), (unsigned)nsplit);
-        if (nsplit % 8 == 0) {
-            sw.xsplit = 1;
-            grid = dim3((unsigned)(tiles * nsplit), 1);
-        }
+        // whole splits per XCD, also where the launch has few tiles (a patch
+        // of tiles per XCD would leave all of them to one XCD)
+        Swizzle sw{};
+        sw.nrt = nrt;
+        sw.nct = nct2;
+        sw.xsplit = nsplit;
+        const dim3 grid((unsigned)(tiles * cdiv(nsplit, 8) * 8));
         EpiLL el{};
         EpiGrad eg{(float*)pg, Bpad, ops->tpad2};
         TimedLaunch tl(ctx, "batched_gradient");
-        if (mode == FP32)
-            hipLaunchKernelGGL((k_gemm<GRAD_FP32, false, GWR, GWC>), grid, dim3(GWR * GWC * 64), 0, ctx->stream,
-                               ops->a2[1], (const uint4*)pr, nrb2, ncb, kps, nkb2, sw, el, eg);
-        else
-            hipLaunchKernelGGL((k_gemm<GRAD_BF16, false, GWR, GWC>), grid, dim3(GWR * GWC * 64), 0, ctx->stream,
-                               ops->a2[0], (const uint4*)pr, nrb2, ncb, kps, nkb2, sw, el, eg);
+        const auto kernel = mode == FP32 ? (narrow ? k_gemm<GRAD_FP32, false, GWR, 1> : k_gemm<GRAD_FP32, false, GWR, 2>)
+                                         : (narrow ? k_gemm<GRAD_BF16, false, GWR, 1> : k_gemm<GRAD_BF16, false, GWR, 2>);
+        hipLaunchKernelGGL(kernel, grid, dim3(GWR * gwc * 64), 0, ctx->stream, ops->a2[mode == FP32 ? 1 : 0],
+                           (const uint4*)pr, nrb2, ncb, kps, nkb2, sw, el, eg);
         if (int rc = check_launch(ctx, "gradient GEMM")) return rc;
     }
     {
-        const int64_t nll = cdiv(B, kFinW), ng = d_G ? cdiv(T * B, 256) : 0;
+        const bool few = T * B <= (int64_t)1 << 18;
+        const int64_t nll = cdiv(B, kFinW), ng = d_G ? cdiv(T * B, few ? 64 : 256) : 0;
         TimedLaunch tl(ctx, "batched_finish");
-        hipLaunchKernelGGL(k_finish, dim3((unsigned)(nll + ng)), dim3(256), 0, ctx->stream, (const double*)pll, nrt1,
+        hipLaunchKernelGGL(few ? k_finish<4> : k_finish<1>, dim3((unsigned)(nll + ng)), dim3(256), 0, ctx->stream, (const double*)pll, nrt1,
                            (const float*)pg, nsplit, T, B, Bpad, ops->tpad2, nll, d_negLL, d_G);
     }
     return check_launch(ctx, "k_finish");
