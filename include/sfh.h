@@ -571,6 +571,15 @@ int sfh_nn_conv_t_dinput(sfh_ctx* ctx, int dtype, const float* d, int64_t B, int
  * parity class per launch plane, the im2col operand gathered as it is read. */
 int sfh_nn_conv_t_fwd(sfh_ctx* ctx, int dtype, const void* in, int64_t B, int64_t Hi, int64_t Wi, int64_t C,
                       const void* w, const float* bias, float* pre, void* aout);
+/* aout of sfh_nn_conv_t_fwd alone (predictions do not read pre). */
+int sfh_nn_conv_t_act(sfh_ctx* ctx, int dtype, const void* in, int64_t B, int64_t Hi, int64_t Wi, int64_t C,
+                      const void* w, const float* bias, void* aout);
+/* sfh_nn_conv_t_fwd followed by sfh_nn_conv1_fwd with SiLU between them, the
+ * decoder's last two layers: out (B x 4Hi x 4Wi) with w1 (16 x 32) and bmap as
+ * in sfh_nn_conv1_fwd; pre (may be NULL) receives the 32-channel tensor between
+ * them before its activation.  BF16: one kernel, FP32 sums in another order. */
+int sfh_nn_conv_t_out(sfh_ctx* ctx, int dtype, const void* in, int64_t B, int64_t Hi, int64_t Wi, int64_t C,
+                      const void* w, const float* bias, const float* w1, const float* bmap, float* pre, float* out);
 /* Weight gradient of that transposed convolution with 32 input and 32 output
  * channels: dK (16 x 32 rows of 32, row tap 32 + co, FP32) = sum over input
  * pixels p of im2col(d)[p][tap 32 + co] act(pre[p][ci]) (act 0: identity, 1:

@@ -1193,9 +1193,161 @@ __global__ __launch_bounds__(kWG) void k_conv_fwd(const T* __restrict__ in, uint
             if (qb < 0) continue;
             const int64_t q = qb + r;
             const float v = acc[a][i] + bv;
-            pre[q] = v;
+            if (pre) pre[q] = v;
             if (aout) aout[q] = from_f32<T>(v * sigmoid(v));
         }
+}
+
+// ------------------------------ last two layers of the decoder in one kernel
+
+// The last 32-channel transposed convolution (bias, SiLU) and the
+// single-channel output layer on its result: out (B x 4Hi x 4Wi) from in (BF16,
+// B x Hi x Wi x 32), the 32-channel tensor between them (B x 2Hi x 2Wi) in
+// registers.  pre, when given, receives it before the activation (what the
+// backward reads).
+//
+// A workgroup makes one tile of kT2Y x kT2X middle pixels and their 2x-scaled
+// outputs.  The tile's inputs are staged in LDS (80 bytes per pixel, so a wave's
+// 16-byte fragment reads are conflict-free); wave = output parity class (py, px) of
+// the first layer (its four taps' weights in registers), whose pixels of the
+// tile plus a one-pixel halo it takes 16 at a time:
+//   D[co][pixel] = sum_(tap, ci) w[tap][co][ci] in[pixel + tap][ci]  (16x16x32 BF16
+//     MFMA, two halves of co; lane l: pixel l % 16, channels 4 (l / 16) + i),
+//   tv[tap][pixel] = sum_co w1[tap][co] SiLU(D + bias)[co][pixel]   (16x16x4 FP32
+//     MFMA: k-step i takes channel 4 g + i of lane group g, so the activated
+//     accumulators are the operand as they stand),
+// tv goes to LDS, and each output adds its four taps.  As two kernels the
+// middle tensor's 2 MB per image were written and read once more, which
+// bounded both: 450 us for 256 images of 52 x 76, 170 us in one kernel (76 for
+// 32 images, 32 with pre written).  What bounds it now is the sum of its VALU
+// work (two quarter-rate operations per activation) and its matrix products,
+// over 1.47 times the tile's pixels (halo and rounding up to 16); taller tiles
+// (12, 18, 26 rows: 1.31, 1.26, 1.17 times) measured 164, 176 and 264 us, for
+// fewer workgroups per CU.
+//
+// SiLU with the hardware reciprocal and one Newton step (within 1 ulp, as the
+// IEEE division, at a third of its instructions: the activations of the halo
+// included are this kernel's VALU work).  1 + exp(-x) is kept finite, where
+// the step is defined; below x = -87 the result is under 1e-36 either way.
+__device__ inline float silu_rcp(float x)
+{
+    const float d = 1.f + fminf(__expf(-x), 0x1p126f);
+    float r = __builtin_amdgcn_rcpf(d);
+    r = fmaf(fmaf(-d, r, 1.f), r, r);
+    return x * r;
+}
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8v __attribute__((ext_vector_type(8)));
+constexpr int kT2Y = 8, kT2X = 38;                             // middle pixels of a tile (both even)
+constexpr int kT2RY = kT2Y + 2, kT2RX = kT2X + 2;              // with the halo
+constexpr int kT2IY = kT2Y / 2 + 2, kT2IX = kT2X / 2 + 2;      // input pixels
+__global__ __launch_bounds__(kWG) void k_conv_out(const uint16_t* __restrict__ in, uint32_t img_bytes, int Hi, int Wi,
+                                                  const uint16_t* __restrict__ w, const float* __restrict__ bias,
+                                                  const float* __restrict__ w1, const float* __restrict__ bmap,
+                                                  int tilesx, int tilesy, float* __restrict__ pre,
+                                                  float* __restrict__ out)
+{
+    constexpr int C = 32, NI = kT2IY * kT2IX, NR = kT2RY * kT2RX;
+    constexpr int CX = kT2RX / 2, NC = CX * (kT2RY / 2);       // one class's pixels: CX per row
+    __shared__ u32x4 sin[NI * 5];
+    __shared__ float tv[16][NR + 1];
+    const int H = 2 * Hi, W = 2 * Wi;
+    const int tx = blockIdx.x % tilesx, ty = (blockIdx.x / tilesx) % tilesy;
+    const int64_t b = blockIdx.x / (tilesx * tilesy);
+    const int y0 = ty * kT2Y, x0 = tx * kT2X;                  // first middle pixel
+    // inputs (y0 / 2 - 1 + r, x0 / 2 - 1 + c); zeros outside the image
+    const __amdgpu_buffer_rsrc_t rs = tensor_rsrc(in + b * Hi * (int64_t)Wi * C, img_bytes);
+    for (int i = threadIdx.x; i < NI * 4; i += kWG) {
+        const int p = i >> 2, q = i & 3;
+        const int y = y0 / 2 - 1 + p / kT2IX, x = x0 / 2 - 1 + p % kT2IX;
+        const bool ok = y >= 0 && y < Hi && x >= 0 && x < Wi;
+        sin[p * 5 + q] = buf_load16(rs, ok ? (uint32_t)(((y * Wi + x) * C + 8 * q) * 2) : kNoRow);
+    }
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int n = lane & 15, g = lane >> 4;
+    const int py = wave >> 1, px = wave & 1;
+    const int ky0 = (py + 1) & 1, kx0 = (px + 1) & 1;
+    // weights of the class's taps j = 2 dy + dx, both halves of co
+    u32x4 wa[4][2];
+    int toff[4];                                               // the taps' input pixels relative to (ry, rx)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int ky = ky0 + 2 * (j >> 1), kx = kx0 + 2 * (j & 1);
+#pragma unroll
+        for (int hf = 0; hf < 2; ++hf)
+            wa[j][hf] = *reinterpret_cast<const u32x4*>(w + ((ky * 4 + kx) * C + 16 * hf + n) * C + 8 * g);
+        // class pixel (ry, rx) is middle pixel (2 y + py, 2 x + px) with y = y0 / 2 -
+        // py + ry (the halo row above belongs to py = 1), input row y +
+        // (py + 1 - ky) / 2, i.e. row ry + 1 - py + (py + 1 - ky) / 2 of the staged ones
+        toff[j] = (1 - py + (py + 1 - ky) / 2) * kT2IX + (1 - px + (px + 1 - kx) / 2);
+    }
+    float wk[8], bv[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const int c = 16 * (i >> 2) + 4 * g + (i & 3);
+        wk[i] = w1[n * C + c];
+        bv[i] = bias ? bias[c] : 0.f;
+    }
+    __syncthreads();
+#pragma unroll 1
+    for (int p0 = 0; p0 < NC; p0 += 16) {
+        const int p = p0 + n < NC ? p0 + n : NC - 1;           // pixels past the last repeat it
+        const int ry = p / CX, rx = p - ry * CX;
+        const u32x4* sp = sin + (ry * kT2IX + rx) * 5 + g;
+        f32x4 acc[2] = {f32x4{bv[0], bv[1], bv[2], bv[3]}, f32x4{bv[4], bv[5], bv[6], bv[7]}};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const bf16x8v x = __builtin_bit_cast(bf16x8v, sp[toff[j] * 5]);
+#pragma unroll
+            for (int hf = 0; hf < 2; ++hf)
+                acc[hf] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8v, wa[j][hf]), x, acc[hf], 0, 0, 0);
+        }
+        const int Yr = 2 * ry + 1 - py, Xr = 2 * rx + 1 - px;  // row and column in the haloed tile
+        const int Y = y0 - 1 + Yr, X = x0 - 1 + Xr;
+        const bool inside = Y >= 0 && Y < H && X >= 0 && X < W;
+        if (pre && inside && Yr >= 1 && Yr <= kT2Y && Xr >= 1 && Xr <= kT2X && p0 + n < NC) {
+            float* o = pre + ((b * H + Y) * (int64_t)W + X) * C + 4 * g;
+            *reinterpret_cast<f32x4*>(o) = acc[0];
+            *reinterpret_cast<f32x4*>(o + 16) = acc[1];
+        }
+        f32x4 t = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const float v = acc[i >> 2][i & 3];
+            t = __builtin_amdgcn_mfma_f32_16x16x4f32(wk[i], silu_rcp(v), t, 0, 0, 0);
+        }
+        // lane holds taps 4 g + i of its pixel
+        if (p0 + n < NC) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) tv[4 * g + i][Yr * kT2RX + Xr] = inside ? t[i] : 0.f;
+        }
+    }
+    __syncthreads();
+    // the 2 x 2 outputs (2Y + a, 2X + c) of every middle pixel of the tile: taps
+    // ky = 1, 3 of rows Y, Y - 1 for a = 0, ky = 0, 2 of rows Y + 1, Y for a = 1
+    // (outside the image: zeros), columns alike
+    const int W2 = 2 * W;
+    for (int q = threadIdx.x; q < kT2Y * kT2X; q += kWG) {
+        const int my = q / kT2X, mx = q - my * kT2X;
+        const int Y = y0 + my, X = x0 + mx;
+        if (Y >= H || X >= W) continue;
+        const int e = (my + 1) * kT2RX + mx + 1;
+        const int o = 2 * Y * W2 + 2 * X;
+        float* po = out + b * 4 * H * (int64_t)W + o;
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                float sum = bmap ? bmap[o + a * W2 + c] : 0.f;
+#pragma unroll
+                for (int dy = 0; dy < 2; ++dy)
+#pragma unroll
+                    for (int dx = 0; dx < 2; ++dx)
+                        sum += tv[(1 - a + 2 * dy) * 4 + 1 - c + 2 * dx][e + (a - dy) * kT2RX + c - dx];
+                po[a * W2 + c] = sum;
+            }
+    }
 }
 
 // ------------------------------------ transposed-convolution weight gradient
@@ -1840,6 +1992,34 @@ static bool conv1_direct(int64_t B, int64_t H, int64_t W, int64_t Ci, const floa
            B * H * W * kC1Ci < ((int64_t)1 << 40) && B * cdiv(H, kC1TY) * cdiv(W, kC1TX) < ((int64_t)1 << 31);
 }
 
+// The 32-channel transposed convolution's launches (pre or aout may be NULL).
+static int conv_t_fwd(sfh_ctx* ctx, int dtype, const void* in, int64_t B, int64_t Hi, int64_t Wi, int64_t C,
+                      const void* w, const float* bias, float* pre, void* aout)
+{
+    const int64_t P = B * Hi * Wi;
+    if (P == 0) return SFH_OK;
+    // batch chunks whose input images span less than 2^31 bytes (the gathers'
+    // 32-bit buffer offsets); images are independent, so chunking is exact
+    const int64_t esz = dtype == 0 ? 2 : 4, img = Hi * Wi * C;
+    const int64_t nb = std::max<int64_t>(1, (((int64_t)1 << 31) - 1) / (img * esz));
+    for (int64_t b0 = 0; b0 < B; b0 += nb) {
+        const int64_t bn = std::min(nb, B - b0), Pc = bn * Hi * Wi;
+        const uint32_t nbytes = (uint32_t)(bn * img * esz);
+        const int64_t oo = b0 * 4 * img;    // output image offset (2Hi x 2Wi x C)
+        const dim3 grid((unsigned)cdiv(Pc, 256), 1, 4);
+        if (dtype == 0)
+            hipLaunchKernelGGL(k_conv_fwd<uint16_t>, grid, dim3(kWG), 0, ctx->stream, (const uint16_t*)in + b0 * img,
+                               nbytes, (int)bn, (int)Hi, (int)Wi, 1.0 / (double)Wi, 1.0 / (double)Hi,
+                               (const uint16_t*)w, bias, pre ? pre + oo : nullptr, aout ? (uint16_t*)aout + oo : nullptr);
+        else
+            hipLaunchKernelGGL(k_conv_fwd<float>, grid, dim3(kWG), 0, ctx->stream, (const float*)in + b0 * img, nbytes,
+                               (int)bn, (int)Hi, (int)Wi, 1.0 / (double)Wi, 1.0 / (double)Hi, (const float*)w, bias,
+                               pre ? pre + oo : nullptr, aout ? (float*)aout + oo : nullptr);
+        if (int rc = check_launch(ctx, "k_conv_fwd")) return rc;
+    }
+    return SFH_OK;
+}
+
 extern "C" {
 
 int sfh_nn_gemm_nt(sfh_ctx* ctx, int dtype, const void* A, int64_t lda, const void* B, int64_t ldb, float* C,
@@ -2256,27 +2436,45 @@ int sfh_nn_conv_t_fwd(sfh_ctx* ctx, int dtype, const void* in, int64_t B, int64_
                            4 * Hi * Wi * C < ((int64_t)1 << 31),
                   "sfh_nn_conv_t_fwd: 32 channels, 16-byte aligned in and w, B Hi Wi < 2^31, one input image "
                   "under 2 GiB");
+    return conv_t_fwd(ctx, dtype, in, B, Hi, Wi, C, w, bias, pre, aout);
+}
+
+int sfh_nn_conv_t_act(sfh_ctx* ctx, int dtype, const void* in, int64_t B, int64_t Hi, int64_t Wi, int64_t C,
+                      const void* w, const float* bias, void* aout)
+{
+    SFH_NN_BEGIN(ctx);
+    const int64_t P = B * Hi * Wi;
+    SFH_ARG_CHECK(ctx, in && w && aout && (dtype == 0 || dtype == 1) && C == 32 && B >= 0 && Hi >= 1 && Wi >= 1 &&
+                           aligned16(in) && aligned16(w) && P < ((int64_t)1 << 31) &&
+                           4 * Hi * Wi * C < ((int64_t)1 << 31),
+                  "sfh_nn_conv_t_act: 32 channels, 16-byte aligned in and w, B Hi Wi < 2^31, one input image "
+                  "under 2 GiB");
+    return conv_t_fwd(ctx, dtype, in, B, Hi, Wi, C, w, bias, nullptr, aout);
+}
+
+int sfh_nn_conv_t_out(sfh_ctx* ctx, int dtype, const void* in, int64_t B, int64_t Hi, int64_t Wi, int64_t C,
+                      const void* w, const float* bias, const float* w1, const float* bmap, float* pre, float* out)
+{
+    SFH_NN_BEGIN(ctx);
+    const int64_t P = B * Hi * Wi;
+    SFH_ARG_CHECK(ctx, in && w && w1 && out && (dtype == 0 || dtype == 1) && C == 32 && B >= 0 && Hi >= 1 && Wi >= 1 &&
+                           aligned16(in) && aligned16(w) && aligned16(pre) && P < ((int64_t)1 << 29) &&
+                           4 * Hi * Wi * C * 4 < ((int64_t)1 << 31),
+                  "sfh_nn_conv_t_out: 32 channels, 16-byte aligned in, w and pre, B Hi Wi < 2^29, one middle image "
+                  "under 2 GiB");
     if (P == 0) return SFH_OK;
-    // batch chunks whose input images span less than 2^31 bytes (the gathers'
-    // 32-bit buffer offsets); images are independent, so chunking is exact
-    const int64_t esz = dtype == 0 ? 2 : 4, img = Hi * Wi * C;
-    const int64_t nb = std::max<int64_t>(1, (((int64_t)1 << 31) - 1) / (img * esz));
-    for (int64_t b0 = 0; b0 < B; b0 += nb) {
-        const int64_t bn = std::min(nb, B - b0), Pc = bn * Hi * Wi;
-        const uint32_t nbytes = (uint32_t)(bn * img * esz);
-        const int64_t oo = b0 * 4 * img;    // output image offset (2Hi x 2Wi x C)
-        const dim3 grid((unsigned)cdiv(Pc, 256), 1, 4);
-        if (dtype == 0)
-            hipLaunchKernelGGL(k_conv_fwd<uint16_t>, grid, dim3(kWG), 0, ctx->stream, (const uint16_t*)in + b0 * img,
-                               nbytes, (int)bn, (int)Hi, (int)Wi, 1.0 / (double)Wi, 1.0 / (double)Hi,
-                               (const uint16_t*)w, bias, pre + oo, aout ? (uint16_t*)aout + oo : nullptr);
-        else
-            hipLaunchKernelGGL(k_conv_fwd<float>, grid, dim3(kWG), 0, ctx->stream, (const float*)in + b0 * img, nbytes,
-                               (int)bn, (int)Hi, (int)Wi, 1.0 / (double)Wi, 1.0 / (double)Hi, (const float*)w, bias,
-                               pre + oo, aout ? (float*)aout + oo : nullptr);
-        if (int rc = check_launch(ctx, "k_conv_fwd")) return rc;
+    const int64_t tx = cdiv(2 * Wi, kT2X), ty = cdiv(2 * Hi, kT2Y);
+    if (dtype == 0 && B * tx * ty < ((int64_t)1 << 31)) {
+        hipLaunchKernelGGL(k_conv_out, dim3((unsigned)(B * tx * ty)), dim3(kWG), 0, ctx->stream, (const uint16_t*)in,
+                           (uint32_t)(Hi * Wi * C * 2), (int)Hi, (int)Wi, (const uint16_t*)w, bias, w1, bmap, (int)tx,
+                           (int)ty, pre, out);
+        return check_launch(ctx, "k_conv_out");
     }
-    return SFH_OK;
+    void* p = pre;
+    if (!p)
+        if (int rc = scratch(ctx, "nn_conv_out_pre", (size_t)P * 4 * C * sizeof(float), &p)) return rc;
+    if (int rc = sfh_nn_conv_t_fwd(ctx, dtype, in, B, Hi, Wi, C, w, bias, (float*)p, nullptr)) return rc;
+    return sfh_nn_conv1_fwd(ctx, (const float*)p, B, 2 * Hi, 2 * Wi, C, w1, bmap, 1, out);
 }
 
 int sfh_nn_conv_t_dweight(sfh_ctx* ctx, int dtype, const float* d, const float* pre, int act, int64_t B, int64_t Hi,

@@ -203,6 +203,9 @@ class TemplateSurrogate:
         """Network output for a batch of physical parameters (B x 4): a torch
         FP32 tensor B x 208 x 304 (log-template; rows < 200, columns < 300 are
         the Hess diagram).  raw=True: params are already scaled to [-1, 1]."""
+        return self._forward(params, raw, True, True)
+
+    def _forward(self, params, raw, keep, refresh):
         x = np.asarray(params, dtype=np.float32) if raw else scale_params(params)
         x = np.atleast_2d(x)
         B = x.shape[0]
@@ -212,15 +215,19 @@ class TemplateSurrogate:
         x16[:, :4] = x
         self.x0f[:B * 16].copy_(self.torch.from_numpy(x16.ravel()))
         self.torch.cuda.synchronize()
-        self._forward_device(B)
+        self._forward_device(B, keep, refresh)
         self.ctx.synchronize()
         return self.out[:B * OUT_H * OUT_W].view(B, OUT_H, OUT_W)
 
-    def _forward_device(self, B):
+    def _forward_device(self, B, keep=True, refresh=True):
         """The network on the scaled inputs already in x0f (B x 16), queued on
-        the context's stream."""
+        the context's stream.  keep: with what a backward reads of the decoder
+        (predictions leave it out); refresh: with the low-precision weight
+        copies made first."""
         v = self.views
-        self._refresh_weights()
+        self.kept = keep
+        if refresh:
+            self._refresh_weights()
         self._bias_act(self.x0f, 16, None, B, 16, IDENT, None, self.x0, 16)
         # MLP
         self._linear(self.x0, 16, self.w["W0"], 16, B, HID0, 16, v["b0"], self.pre0, self.a0, HID0, self.a0T)
@@ -228,18 +235,18 @@ class TemplateSurrogate:
         self._linear(self.a1, HID1, self.w["W2"], HID1, B, LAT, HID1, v["b2"], self.pre2, self.a2, LAT)
         # decoder
         H, W = H0, W0
-        ins = (self.a2, self.a3, self.a4)
-        pres = (self.pre3, self.pre4, self.pre5)
-        outs = (self.a3, self.a4, None)
-        for li, (K, cb) in enumerate((("K1", "c1"), ("K2", "c2"), ("K3", "c3"))):
-            # pre-activation (+ bias) and, but for the last layer, its SiLU in one kernel
-            self._c(self.lib.sfh_nn_conv_t_fwd(self.ctx.handle, self.dt, ins[li].data_ptr(), B, H, W, CH,
-                                               self.w[K].data_ptr(), v[cb].data_ptr(), pres[li].data_ptr(),
-                                               outs[li].data_ptr() if outs[li] is not None else None))
+        for K, cb, a_in, pre, a_out in (("K1", "c1", self.a2, self.pre3, self.a3),
+                                        ("K2", "c2", self.a3, self.pre4, self.a4)):
+            # pre-activation (+ bias) and its SiLU in one kernel
+            args = (self.ctx.handle, self.dt, a_in.data_ptr(), B, H, W, CH, self.w[K].data_ptr(), v[cb].data_ptr())
+            self._c(self.lib.sfh_nn_conv_t_fwd(*args, pre.data_ptr(), a_out.data_ptr()) if keep else
+                    self.lib.sfh_nn_conv_t_act(*args, a_out.data_ptr()))
             H, W = 2 * H, 2 * W
-        # single-channel output layer on SiLU(pre5), the activation applied inside
-        self._c(self.lib.sfh_nn_conv1_fwd(self.ctx.handle, self.pre5.data_ptr(), B, H, W, CH, v["w4"].data_ptr(),
-                                          v["bmap"].data_ptr(), SILU, self.out.data_ptr()))
+        # the last 32-channel layer and the single-channel output layer
+        self._c(self.lib.sfh_nn_conv_t_out(self.ctx.handle, self.dt, self.a4.data_ptr(), B, H, W, CH,
+                                           self.w["K3"].data_ptr(), v["c3"].data_ptr(), v["w4"].data_ptr(),
+                                           v["bmap"].data_ptr(), self.pre5.data_ptr() if keep else None,
+                                           self.out.data_ptr()))
 
     # ---------------------------------------------------------- backward
     def backward(self, target):
@@ -249,6 +256,8 @@ class TemplateSurrogate:
         B = self.B
         t = target.contiguous().view(-1)
         self.torch.cuda.synchronize()
+        if not self.kept:                        # the last forward was a prediction's
+            self._forward_device(B)
         loss = C.c_float()
         self._c(self.lib.sfh_nn_mse(self.ctx.handle, self.out.data_ptr(), t.data_ptr(), None, B, OUT_H, OUT_W,
                                     CROP_H, CROP_W, self.dout.data_ptr(), C.byref(loss), None))
@@ -446,7 +455,7 @@ class TemplateSurrogate:
             out = self.torch.empty((n, nx * ny), dtype=self.torch.float32, device=self.dev)
         for b0 in range(0, n, batch):
             b1 = min(n, b0 + batch)
-            y = self.forward(p[b0:b1])
+            y = self._forward(p[b0:b1], False, False, b0 == 0)     # one set of weight copies per call
             self._c(self.lib.sfh_nn_log_template(self.ctx.handle, y.data_ptr(), b1 - b0, OUT_H, OUT_W, nx, ny,
                                                  LOG_EPS, LOG_OFFSET, LOG_SCALE, out[b0].data_ptr(),
                                                  out.stride(0)))
