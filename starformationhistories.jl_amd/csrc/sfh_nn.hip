@@ -1350,6 +1350,83 @@ __global__ __launch_bounds__(kWG) void k_conv_out(const uint16_t* __restrict__ i
     }
 }
 
+// Forward of one 32-channel layer (BF16): a workgroup's tile of kT1Y x kT1X
+// outputs as in k_conv_out above -- inputs staged in LDS, wave = parity class
+// with its weights in registers, 16 pixels at a time, lane l holding four
+// channels of pixel l % 16, so that outputs leave as 16-byte (pre) and 8-byte
+// (aout) stores.  The gathering form (k_conv_fwd, kept for FP32 operands) reads
+// every input four times through L2 and stores two bytes per lane.
+constexpr int kT1Y = 4, kT1X = 38;
+constexpr int kT1IY = kT1Y / 2 + 2, kT1IX = kT1X / 2 + 2;
+__global__ __launch_bounds__(kWG) void k_conv_mid(const uint16_t* __restrict__ in, uint32_t img_bytes, int Hi, int Wi,
+                                                  const uint16_t* __restrict__ w, const float* __restrict__ bias,
+                                                  int tilesx, int tilesy, float* __restrict__ pre,
+                                                  uint16_t* __restrict__ aout)
+{
+    constexpr int C = 32, NI = kT1IY * kT1IX, CX = kT1X / 2, NC = CX * (kT1Y / 2);
+    __shared__ u32x4 sin[NI * 5];
+    const int H = 2 * Hi, W = 2 * Wi;
+    const int tx = blockIdx.x % tilesx, ty = (blockIdx.x / tilesx) % tilesy;
+    const int64_t b = blockIdx.x / (tilesx * tilesy);
+    const int y0 = ty * (kT1Y / 2), x0 = tx * (kT1X / 2);      // first input pixel
+    const __amdgpu_buffer_rsrc_t rs = tensor_rsrc(in + b * Hi * (int64_t)Wi * C, img_bytes);
+    for (int i = threadIdx.x; i < NI * 4; i += kWG) {
+        const int p = i >> 2, q = i & 3;
+        const int y = y0 - 1 + p / kT1IX, x = x0 - 1 + p % kT1IX;
+        const bool ok = y >= 0 && y < Hi && x >= 0 && x < Wi;
+        sin[p * 5 + q] = buf_load16(rs, ok ? (uint32_t)(((y * Wi + x) * C + 8 * q) * 2) : kNoRow);
+    }
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int n = lane & 15, g = lane >> 4;
+    const int py = wave >> 1, px = wave & 1;
+    const int ky0 = (py + 1) & 1, kx0 = (px + 1) & 1;
+    u32x4 wa[4][2];
+    int toff[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int ky = ky0 + 2 * (j >> 1), kx = kx0 + 2 * (j & 1);
+#pragma unroll
+        for (int hf = 0; hf < 2; ++hf)
+            wa[j][hf] = *reinterpret_cast<const u32x4*>(w + ((ky * 4 + kx) * C + 16 * hf + n) * C + 8 * g);
+        toff[j] = (1 + (py + 1 - ky) / 2) * kT1IX + 1 + (px + 1 - kx) / 2;
+    }
+    f32x4 bv[2] = {};
+    if (bias) {
+#pragma unroll
+        for (int hf = 0; hf < 2; ++hf)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) bv[hf][i] = bias[16 * hf + 4 * g + i];
+    }
+    __syncthreads();
+#pragma unroll 1
+    for (int p0 = 0; p0 < NC; p0 += 16) {
+        const int p = p0 + n < NC ? p0 + n : NC - 1;
+        const int ry = p / CX, rx = p - ry * CX;
+        const u32x4* sp = sin + (ry * kT1IX + rx) * 5 + g;
+        f32x4 acc[2] = {bv[0], bv[1]};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const bf16x8v x = __builtin_bit_cast(bf16x8v, sp[toff[j] * 5]);
+#pragma unroll
+            for (int hf = 0; hf < 2; ++hf)
+                acc[hf] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8v, wa[j][hf]), x, acc[hf], 0, 0, 0);
+        }
+        const int Y = 2 * (y0 + ry) + py, X = 2 * (x0 + rx) + px;
+        if (p0 + n >= NC || Y >= H || X >= W) continue;
+        const int64_t q = ((b * H + Y) * (int64_t)W + X) * C + 4 * g;
+#pragma unroll
+        for (int hf = 0; hf < 2; ++hf) {
+            if (pre) *reinterpret_cast<f32x4*>(pre + q + 16 * hf) = acc[hf];
+            if (aout) {
+                uint32_t h[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) h[i] = to_bf16(silu_rcp(acc[hf][i]));
+                *reinterpret_cast<uint2*>(aout + q + 16 * hf) = make_uint2(h[0] | h[1] << 16, h[2] | h[3] << 16);
+            }
+        }
+    }
+}
+
 // ------------------------------------ transposed-convolution weight gradient
 
 // Partial weight gradients of a stride-2, 4x4, padding-1 transposed
@@ -2007,7 +2084,13 @@ static int conv_t_fwd(sfh_ctx* ctx, int dtype, const void* in, int64_t B, int64_
         const uint32_t nbytes = (uint32_t)(bn * img * esz);
         const int64_t oo = b0 * 4 * img;    // output image offset (2Hi x 2Wi x C)
         const dim3 grid((unsigned)cdiv(Pc, 256), 1, 4);
-        if (dtype == 0)
+        const int64_t tx = cdiv(2 * Wi, kT1X), ty = cdiv(2 * Hi, kT1Y);
+        // whole 16-byte pre and 8-byte aout stores; otherwise the gathering form
+        if (dtype == 0 && aligned16(pre) && ((uintptr_t)aout & 7u) == 0 && bn * tx * ty < ((int64_t)1 << 31))
+            hipLaunchKernelGGL(k_conv_mid, dim3((unsigned)(bn * tx * ty)), dim3(kWG), 0, ctx->stream,
+                               (const uint16_t*)in + b0 * img, (uint32_t)(img * 2), (int)Hi, (int)Wi, (const uint16_t*)w,
+                               bias, (int)tx, (int)ty, pre ? pre + oo : nullptr, aout ? (uint16_t*)aout + oo : nullptr);
+        else if (dtype == 0)
             hipLaunchKernelGGL(k_conv_fwd<uint16_t>, grid, dim3(kWG), 0, ctx->stream, (const uint16_t*)in + b0 * img,
                                nbytes, (int)bn, (int)Hi, (int)Wi, 1.0 / (double)Wi, 1.0 / (double)Hi,
                                (const uint16_t*)w, bias, pre ? pre + oo : nullptr, aout ? (uint16_t*)aout + oo : nullptr);
