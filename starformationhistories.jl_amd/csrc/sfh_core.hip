@@ -56,7 +56,13 @@ int scratch(sfh_ctx* ctx, const char* name, size_t bytes, void** out)
             b.bytes = 0;
         }
         size_t want = bytes < 256 ? 256 : bytes;
-        if (hipMalloc(&b.ptr, want) != hipSuccess) {
+        hipError_t e = hipMalloc(&b.ptr, want);
+        if (e != hipSuccess && ctx->pool_bytes > 0) {
+            (void)hipGetLastError();
+            pool_clear(ctx);
+            e = hipMalloc(&b.ptr, want);
+        }
+        if (e != hipSuccess) {
             b.ptr = nullptr;
             return set_error(ctx, SFH_ERR_ALLOC, "hipMalloc(%zu) for scratch '%s' failed", want, name);
         }
@@ -64,6 +70,51 @@ int scratch(sfh_ctx* ctx, const char* name, size_t bytes, void** out)
     }
     *out = b.ptr;
     return SFH_OK;
+}
+
+void pool_clear(sfh_ctx* ctx)
+{
+    for (DevBuf& b : ctx->pool) (void)hipFree(b.ptr);     // waits for the work on them
+    ctx->pool.clear();
+    ctx->pool_bytes = 0;
+}
+
+int pool_get(sfh_ctx* ctx, size_t bytes, DevBuf* out)
+{
+    if (bytes < 256) bytes = 256;
+    size_t best = ctx->pool.size();
+    for (size_t i = 0; i < ctx->pool.size(); ++i) {
+        const size_t have = ctx->pool[i].bytes;
+        if (have >= bytes && have / 2 <= bytes && (best == ctx->pool.size() || have < ctx->pool[best].bytes)) best = i;
+    }
+    if (best < ctx->pool.size()) {
+        *out = ctx->pool[best];
+        ctx->pool_bytes -= out->bytes;
+        ctx->pool.erase(ctx->pool.begin() + (ptrdiff_t)best);
+        return SFH_OK;
+    }
+    // an eighth more than asked for, so that the next catalogue of about this size fits
+    const size_t want = bytes + bytes / 8;
+    out->bytes = want;
+    if (hipMalloc(&out->ptr, want) == hipSuccess) return SFH_OK;
+    (void)hipGetLastError();
+    pool_clear(ctx);
+    out->bytes = bytes;
+    if (hipMalloc(&out->ptr, bytes) == hipSuccess) return SFH_OK;
+    (void)hipGetLastError();
+    *out = DevBuf{};
+    return set_error(ctx, SFH_ERR_ALLOC, "hipMalloc(%zu) failed", bytes);
+}
+
+void pool_put(sfh_ctx* ctx, DevBuf* b)
+{
+    if (b->ptr && ctx->pool_bytes + b->bytes <= kPoolBytes && ctx->pool.size() < ctx->pool.capacity()) {
+        ctx->pool.push_back(*b);
+        ctx->pool_bytes += b->bytes;
+    } else if (b->ptr) {
+        (void)hipFree(b->ptr);
+    }
+    *b = DevBuf{};
 }
 
 int pinned(sfh_ctx* ctx, size_t bytes, void** out)
@@ -477,6 +528,7 @@ int sfh_ctx_create(int device, void* stream, sfh_ctx** out)
         g_create_error = "noalloc_init: hipGetSymbolAddress of the static fg! buffer failed";
         return rc;
     }
+    c->pool.reserve(kPoolBuffers);
     *out = c;
     return SFH_OK;
 }
@@ -490,6 +542,7 @@ static void ctx_teardown(sfh_ctx* ctx)
         resolve_timing(ctx);
         for (auto& kv : ctx->scratch)
             if (kv.second.ptr) hipFree(kv.second.ptr);
+        pool_clear(ctx);
         for (hipEvent_t e : ctx->event_pool) hipEventDestroy(e);
         if (ctx->pinned) hipHostFree(ctx->pinned);
         if (ctx->own_stream) hipStreamDestroy(ctx->stream);

@@ -28,6 +28,7 @@ struct sfh_catalog {
     double* d_masses = nullptr;   // n x nstars
     double* d_mags = nullptr;     // n x nfilters
     int64_t* d_index = nullptr;   // system index, or index of the input star
+    sfh::DevBuf bufs[3];          // their memory, from the context's pool
 };
 
 namespace sfh {
@@ -388,28 +389,34 @@ int catalog_reserve(sfh_catalog* c, int64_t need)
     sfh_ctx* ctx = c->ctx;
     if (need <= c->cap) return SFH_OK;
     const int64_t cap = std::max<int64_t>(need, c->cap + c->cap / 2 + 1024);
-    double *m = nullptr, *g = nullptr;
-    int64_t* ix = nullptr;
-    if (c->nstars > 0) SFH_HIP_TRY(ctx, hipMalloc(&m, (size_t)cap * c->nstars * sizeof(double)));
-    SFH_HIP_TRY(ctx, hipMalloc(&g, (size_t)cap * std::max(c->nfilters, 1) * sizeof(double)));
-    SFH_HIP_TRY(ctx, hipMalloc(&ix, (size_t)cap * sizeof(int64_t)));
-    if (c->n > 0) {
-        if (m) SFH_HIP_TRY(ctx, hipMemcpyAsync(m, c->d_masses, (size_t)c->n * c->nstars * sizeof(double),
-                                               hipMemcpyDeviceToDevice, ctx->stream));
-        SFH_HIP_TRY(ctx, hipMemcpyAsync(g, c->d_mags, (size_t)c->n * c->nfilters * sizeof(double),
-                                        hipMemcpyDeviceToDevice, ctx->stream));
-        SFH_HIP_TRY(ctx, hipMemcpyAsync(ix, c->d_index, (size_t)c->n * sizeof(int64_t), hipMemcpyDeviceToDevice,
-                                        ctx->stream));
+    DevBuf old[3] = {c->bufs[0], c->bufs[1], c->bufs[2]}, bufs[3];
+    const size_t bytes[3] = {(size_t)cap * c->nstars * sizeof(double),
+                             (size_t)cap * std::max(c->nfilters, 1) * sizeof(double), (size_t)cap * sizeof(int64_t)};
+    const size_t used[3] = {(size_t)c->n * c->nstars * sizeof(double), (size_t)c->n * c->nfilters * sizeof(double),
+                            (size_t)c->n * sizeof(int64_t)};
+    int rc = SFH_OK;
+    for (int k = c->nstars > 0 ? 0 : 1; k < 3 && !rc; ++k) {
+        rc = pool_get(ctx, bytes[k], &bufs[k]);
+        if (!rc && used[k] > 0 &&
+            hipMemcpyAsync(bufs[k].ptr, old[k].ptr, used[k], hipMemcpyDeviceToDevice, ctx->stream) != hipSuccess)
+            rc = set_error(ctx, SFH_ERR_DEVICE, "catalogue copy failed");
     }
-    SFH_HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-    hipFree(c->d_masses);
-    hipFree(c->d_mags);
-    hipFree(c->d_index);
-    c->d_masses = m;
-    c->d_mags = g;
-    c->d_index = ix;
+    for (int k = 0; k < 3; ++k) {
+        if (!rc) c->bufs[k] = bufs[k];
+        pool_put(ctx, rc ? &bufs[k] : &old[k]);
+    }
+    if (rc) return rc;
+    c->d_masses = (double*)c->bufs[0].ptr;
+    c->d_mags = (double*)c->bufs[1].ptr;
+    c->d_index = (int64_t*)c->bufs[2].ptr;
     c->cap = cap;
     return SFH_OK;
+}
+
+void catalog_release(sfh_catalog* c)
+{
+    for (DevBuf& b : c->bufs) pool_put(c->ctx, &b);
+    delete c;
 }
 
 // Append the kept entries among the first n of a staged batch to c.
@@ -541,10 +548,7 @@ int sfh_generate_stars(sfh_ctx* ctx, int64_t npoints, const double* mini, int32_
     c->nstars = a.nst;
     c->nfilters = nfilters;
     auto fail = [&](int rc) {
-        hipFree(c->d_masses);
-        hipFree(c->d_mags);
-        hipFree(c->d_index);
-        delete c;
+        catalog_release(c);
         return rc;
     };
 
@@ -639,12 +643,12 @@ int sfh_catalog_from_host(sfh_ctx* ctx, int64_t n, int32_t nfilters, const doubl
     c->nfilters = nfilters;
     int rc = catalog_reserve(c, std::max<int64_t>(n, 1));
     if (!rc && n > 0 &&
-        hipMemcpy(c->d_mags, mags, (size_t)n * nfilters * sizeof(double), hipMemcpyHostToDevice) != hipSuccess)
+        (hipMemcpyAsync(c->d_mags, mags, (size_t)n * nfilters * sizeof(double), hipMemcpyHostToDevice, ctx->stream) !=
+             hipSuccess ||
+         hipStreamSynchronize(ctx->stream) != hipSuccess))
         rc = set_error(ctx, SFH_ERR_DEVICE, "sfh_catalog_from_host: copy failed");
     if (rc) {
-        hipFree(c->d_mags);
-        hipFree(c->d_index);
-        delete c;
+        catalog_release(c);
         return rc;
     }
     c->n = n;
@@ -719,11 +723,7 @@ int sfh_catalog_destroy(sfh_catalog* c)
     {
         std::lock_guard<std::recursive_mutex> g(ctx->mu);
         hipSetDevice(ctx->device);
-        hipStreamSynchronize(ctx->stream);
-        hipFree(c->d_masses);
-        hipFree(c->d_mags);
-        hipFree(c->d_index);
-        delete c;
+        catalog_release(c);
     }
     ctx_release(ctx);
     return SFH_OK;
@@ -781,9 +781,7 @@ int sfh_model_cmd(sfh_ctx* ctx, const sfh_catalog* in, const sfh_table* err, con
         int rc = check_launch(ctx, "k_observe");
         if (!rc) rc = compact_append(c, d_keep, n, nullptr, d_out, 0);
         if (rc) {
-            hipFree(c->d_mags);
-            hipFree(c->d_index);
-            delete c;
+            catalog_release(c);
             return rc;
         }
     }
