@@ -1084,6 +1084,85 @@ __global__ __launch_bounds__(kWG) void k_conv_dinput(const float* __restrict__ d
         }
 }
 
+// The same gradient for 32 input and output channels in BF16, from tiles: a
+// workgroup takes kDIY x kDIX input pixels (six rows of half the network's
+// 38-pixel-wide maps, 114 of its 4 waves' 128 columns), stages their window of
+// d in LDS once, rounded to BF16, and every wave multiplies 32 pixels by all
+// taps in the K order of the gathering form, whose results it repeats to the
+// bit.  80 bytes per window pixel and even and odd columns apart, so that the
+// 16-byte reads of neighbouring pixels (every other window column) spread over
+// the banks.  The weights are the A operand, so a lane's accumulators are four
+// quadruples of one pixel's channels: 16-byte stores.  The gathering form reads
+// each gradient four times (once per input pixel of its window) from L2 and
+// converts it four times, and needed slices of the taps and their sum where
+// its 256-pixel tiles were few: 42.9, 12.0 and 12.0 us (and two sums of 4.8)
+// for 32 images of 52 x 76, 26 x 38 and 13 x 19 pixels; %TIMES% from tiles.
+// Bound by the reads of d (1.23 times its size with the window's rim) and the
+// stores.
+constexpr int kDIY = 6, kDIX = 19;
+constexpr int kDIWY = 2 * kDIY + 2, kDIHX = kDIX + 1, kDIWX = 2 * kDIHX;    // window rows, half columns, columns
+__global__ __launch_bounds__(kWG) void k_conv_dinput_tile(const float* __restrict__ d, uint32_t img_bytes, int Hi,
+                                                          int Wi, const uint16_t* __restrict__ wT, int64_t ldw,
+                                                          int tilesx, int tilesy, float* __restrict__ out, int64_t ldo)
+{
+    constexpr int C = 32, NP = kDIWY * kDIWX, NPX = kDIY * kDIX, NS = C;
+    static_assert(NPX <= 128, "one 32-pixel group per wave");
+    __shared__ u32x4 win[NP * 5];
+    const int H2 = 2 * Hi, W2 = 2 * Wi;
+    const int tx = blockIdx.x % tilesx, ty = (blockIdx.x / tilesx) % tilesy;
+    const int64_t b = blockIdx.x / (tilesx * tilesy);
+    const int y0 = ty * kDIY, x0 = tx * kDIX;
+    const __amdgpu_buffer_rsrc_t rs = tensor_rsrc(d + b * H2 * (int64_t)W2 * C, img_bytes);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int r = lane & 31, h = lane >> 5;
+    const uint16_t* pw = wT + r * ldw + 8 * h;
+    constexpr int NR = 16;      // weight fragments in flight
+    Frag<uint16_t> fw[NR];
+#pragma unroll
+    for (int s = 0; s < NR; ++s) load_frag_raw(pw + 16 * s, fw[s]);
+    constexpr int U = 3;        // 32-byte loads of a thread in flight
+#pragma unroll 1
+    for (int i0 = threadIdx.x; i0 < NP * 4; i0 += U * kWG) {
+        f4 lo[U], hi[U];
+        int to[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int i = i0 + u * kWG, p = i >> 2, q = i & 3;
+            const int wy = p / kDIWX, wx = p - wy * kDIWX;
+            const int Y = 2 * y0 - 1 + wy, X = 2 * x0 - 1 + wx;
+            const bool ok = p < NP && Y >= 0 && Y < H2 && X >= 0 && X < W2;
+            const uint32_t off = ok ? (uint32_t)((Y * W2 + X) * C + 8 * q) * 4u : kNoRow;
+            lo[u] = __builtin_bit_cast(f4, buf_load16(rs, off));
+            hi[u] = __builtin_bit_cast(f4, buf_load16(rs, off + 16));
+            to[u] = p < NP ? (wy * kDIWX + (wx & 1) * kDIHX + (wx >> 1)) * 5 + q : -1;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            Frag<uint16_t> f;
+            to_frag(lo[u], hi[u], f);
+            if (to[u] >= 0) win[to[u]] = f.v;
+        }
+    }
+    __syncthreads();
+    const int e = wave * 32 + r, ec = e < NPX ? e : NPX - 1;
+    const int ry = ec / kDIX, rx = ec - ry * kDIX;
+    const u32x4* pv = win + (2 * ry * kDIWX + rx) * 5 + h;
+    f32x16 acc = {};
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+        const int tap = s >> 1, ky = tap >> 2, kx = tap & 3;
+        Frag<uint16_t> f;
+        f.v = pv[(ky * kDIWX + (kx & 1) * kDIHX + (kx >> 1)) * 5 + (s & 1) * 2];
+        acc = mma(fw[s % NR], f, acc);
+        if (s + NR < NS) load_frag_raw(pw + 16 * (s + NR), fw[s % NR]);
+    }
+    if (e >= NPX || y0 + ry >= Hi || x0 + rx >= Wi) return;
+    float* po = out + ((b * Hi + y0 + ry) * (int64_t)Wi + x0 + rx) * ldo + 4 * h;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+        *reinterpret_cast<f4*>(po + 8 * q) = f4{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
+}
+
 // out[0..n) = v (a kernel, so that the call can sit in a captured graph)
 __global__ __launch_bounds__(kWG) void k_fill(float* __restrict__ out, int64_t n, float v)
 {
@@ -2465,6 +2544,16 @@ int sfh_nn_conv_t_dinput(sfh_ctx* ctx, int dtype, const float* d, int64_t B, int
                   "sfh_nn_conv_t_dinput: Co 8, 16 or 32, ldw >= 16 Co (a multiple of 8), ldo >= Ci, "
                   "16-byte aligned d and wT, B Hi Wi < 2^31, one gradient image under 2 GiB");
     if (P == 0) return SFH_OK;
+    // BF16, 32 x 32 channels and 16-byte stores: tiles (76.5 -> 48.9 us over the
+    // decoder's three layers, k_conv_dinput_tile); the gathering form for the
+    // channel counts, FP32 operands and row strides that the tiles don't take
+    const int64_t tx = cdiv(Wi, kDIX), ty = cdiv(Hi, kDIY);
+    if (dtype == 0 && Co == 32 && Ci == 32 && ldo % 4 == 0 && aligned16(out) && B * tx * ty < ((int64_t)1 << 31)) {
+        hipLaunchKernelGGL(k_conv_dinput_tile, dim3((unsigned)(B * tx * ty)), dim3(kWG), 0, ctx->stream, d,
+                           (uint32_t)(16 * Hi * Wi * Co), (int)Hi, (int)Wi, (const uint16_t*)wT, ldw, (int)tx, (int)ty,
+                           out, ldo);
+        return check_launch(ctx, "k_conv_dinput_tile");
+    }
     const double iw = 1.0 / (double)Wi, ih = 1.0 / (double)Hi;
     // batch chunks whose gradient images span less than 2^31 bytes (the gathers'
     // 32-bit buffer offsets); images are independent, so chunking is exact
