@@ -14,8 +14,10 @@
 //             din = dcols W,  dW = dcols^T in                          (GEMMs)
 // and that composition is kept as entry points; the training path runs
 // each line as one product whose operands are gathered as they are loaded
-// (k_conv_fwd by output parity class, k_conv_dinput, k_conv_dweight), so no
-// column matrix is written.  The single-channel output layer works on the
+// (in BF16 from tiles staged in LDS: k_conv_mid, k_conv_out with the output
+// layer, k_conv_dinput_tile; k_conv_fwd by output parity class and k_conv_dinput
+// gather for the other types and channel counts; k_conv_dweight), so no column
+// matrix is written.  The single-channel output layer works on the
 // pixel grid with 16 x 16 x 4 FP32 MFMA tap sums (k_conv1_*).  Activations are
 // channels-last (pixel-major, channel fastest) and weight rows tap-major
 // ((ky*4 + kx)*Co + co), so the gathers move runs of Co consecutive floats.
@@ -682,13 +684,26 @@ __device__ inline void chan_part32(f4 s, f4* red, float* __restrict__ part)
 // walk the blocks grid-stride.  With part non-null, also the workgroup's
 // channel sums of din: per lane over its rows, then the four lane groups with
 // shuffles and the waves through LDS, in a fixed order, into part[wg][c].
+//
+// With DW also the weight gradient's partials dwpart[wg][tap 32 + c] = sum over
+// the workgroup's pixels of window(p)[tap] act(in[p][c]): a lane's four
+// activations of a block (pixels 4 (l / 16) + r, channel l % 16) are, r by r, the B
+// operand of 16 x 16 x 4 products over pixels as they stand, and the A operand is
+// the window of the same pixels at tap l % 16, off the lines just read.  As two
+// kernels (k_conv1_dw below, kept for a weight gradient alone) the 32-channel
+// tensor was read twice: 29.4 + 22.7 us for 32 images of 104 x 152, 36.0 in one
+// (and 4.8 for a second pass over the partials), 24 training steps 11.06 ->
+// 10.68 ms.
+template <bool DW>
 __global__ __launch_bounds__(kWG) void k_conv1_din(const float* __restrict__ dout, uint32_t dout_bytes,
                                                    const float* __restrict__ in, int B, int H, int W, double inv_w,
                                                    double inv_h, const float* __restrict__ w, int act,
-                                                   float* __restrict__ din, float* __restrict__ part)
+                                                   float* __restrict__ din, float* __restrict__ part,
+                                                   float* __restrict__ dwpart)
 {
     constexpr int NWV = kWG / 64;
     __shared__ float red[NWV][kC1Ci];
+    __shared__ float redw[DW ? NWV : 1][DW ? 16 * kC1Ci : 1];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int mt = lane & 15, mk = lane >> 4;
     const int64_t P = (int64_t)B * H * W, nblk = (P + 15) / 16;
@@ -701,6 +716,7 @@ __global__ __launch_bounds__(kWG) void k_conv1_din(const float* __restrict__ dou
         wb1[ks] = w[(4 * ks + mk) * kC1Ci + 16 + mt];
     }
     float cs0 = 0.f, cs1 = 0.f;
+    f4 dw0 = {0.f, 0.f, 0.f, 0.f}, dw1 = {0.f, 0.f, 0.f, 0.f};
     for (int64_t bi = (int64_t)blockIdx.x * NWV + wave; bi < nblk; bi += (int64_t)gridDim.x * NWV) {
         const int64_t pa = bi * 16 + mt, pq = pa < P ? pa : P - 1;
         const int64_t rr = udiv31(pq, W, inv_w), b = udiv31(rr, H, inv_h);
@@ -719,8 +735,27 @@ __global__ __launch_bounds__(kWG) void k_conv1_din(const float* __restrict__ dou
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int64_t pd = bi * 16 + 4 * mk + r, pc = pd < P ? pd : P - 1;
-            x0[r] = act == 1 ? in[pc * kC1Ci + mt] : 0.f;
-            x1[r] = act == 1 ? in[pc * kC1Ci + 16 + mt] : 0.f;
+            x0[r] = DW || act == 1 ? in[pc * kC1Ci + mt] : 0.f;
+            x1[r] = DW || act == 1 ? in[pc * kC1Ci + 16 + mt] : 0.f;
+        }
+        // the window at tap mt of the same pixels (pixel 4 mk is lane 4 mk's)
+        float aw[4];
+        if constexpr (DW) {
+            int xw = __shfl(x, 4 * mk, 64), yw = __shfl(y, 4 * mk, 64), bw = __shfl((int)b, 4 * mk, 64);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int Y = 2 * yw - 1 + (mt >> 2), Xw = 2 * xw - 1 + (mt & 3);
+                const bool ok = bi * 16 + 4 * mk + r < P && Y >= 0 && Y < H2 && Xw >= 0 && Xw < W2;
+                aw[r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                                      rs, ok ? (uint32_t)(((bw * H2 + Y) * W2 + Xw) * 4) : kNoRow, 0, 0));
+                if (++xw == W) {
+                    xw = 0;
+                    if (++yw == H) {
+                        yw = 0;
+                        ++bw;
+                    }
+                }
+            }
         }
         f4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -732,10 +767,16 @@ __global__ __launch_bounds__(kWG) void k_conv1_din(const float* __restrict__ dou
         for (int r = 0; r < 4; ++r) {
             const int64_t pd = bi * 16 + 4 * mk + r;
             float v0 = acc0[r], v1 = acc1[r];
+            float s0 = 1.f, s1 = 1.f;
             if (act == 1) {
-                const float s0 = sigmoid(x0[r]), s1 = sigmoid(x1[r]);
+                s0 = sigmoid(x0[r]);
+                s1 = sigmoid(x1[r]);
                 v0 *= s0 * (1.f + x0[r] * (1.f - s0));
                 v1 *= s1 * (1.f + x1[r] * (1.f - s1));
+            }
+            if constexpr (DW) {
+                dw0 = __builtin_amdgcn_mfma_f32_16x16x4f32(aw[r], x0[r] * s0, dw0, 0, 0, 0);
+                dw1 = __builtin_amdgcn_mfma_f32_16x16x4f32(aw[r], x1[r] * s1, dw1, 0, 0, 0);
             }
             if (pd < P) {
                 din[pd * kC1Ci + mt] = v0;
@@ -760,6 +801,21 @@ __global__ __launch_bounds__(kWG) void k_conv1_din(const float* __restrict__ dou
 #pragma unroll
             for (int k = 1; k < NWV; ++k) t += red[k][threadIdx.x];
             part[(int64_t)blockIdx.x * kC1Ci + threadIdx.x] = t;
+        }
+    }
+    if constexpr (DW) {
+        // lane holds taps 4 mk .. 4 mk + 3 of channels mt and 16 + mt
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            redw[wave][(4 * mk + r) * kC1Ci + mt] = dw0[r];
+            redw[wave][(4 * mk + r) * kC1Ci + 16 + mt] = dw1[r];
+        }
+        __syncthreads();
+        for (int i = threadIdx.x; i < 16 * kC1Ci; i += kWG) {
+            float t = redw[0][i];
+#pragma unroll
+            for (int k = 1; k < NWV; ++k) t += redw[k][i];
+            dwpart[(int64_t)blockIdx.x * 16 * kC1Ci + i] = t;
         }
     }
 }
@@ -1095,8 +1151,9 @@ __global__ __launch_bounds__(kWG) void k_conv_dinput(const float* __restrict__ d
 // quadruples of one pixel's channels: 16-byte stores.  The gathering form reads
 // each gradient four times (once per input pixel of its window) from L2 and
 // converts it four times, and needed slices of the taps and their sum where
-// its 256-pixel tiles were few: 42.9, 12.0 and 12.0 us (and two sums of 4.8)
-// for 32 images of 52 x 76, 26 x 38 and 13 x 19 pixels; %TIMES% from tiles.
+// its 256-pixel tiles were few: 42.9, 12.0 and 12.0 us and two sums of 4.8 for
+// 32 images of 52 x 76, 26 x 38 and 13 x 19 pixels, 76.5 together; 48.9 from
+// tiles.
 // Bound by the reads of d (1.23 times its size with the window's rim) and the
 // stores.
 constexpr int kDIY = 6, kDIX = 19;
@@ -2459,21 +2516,30 @@ int sfh_nn_conv1_bwd(sfh_ctx* ctx, const float* dout, const float* in, int64_t B
     void* p = nullptr;
     if ((din || dw) && conv1_direct(B, H, W, Ci, (dw || act) ? in : nullptr, din ? w : nullptr, din)) {
         if (din) {
-            const int64_t nwg = chan_grid(P);
+            // with the weight gradient, fewer workgroups (four per CU on 256): each
+            // writes its 16 x 32 partial
+            const int64_t nwg = dw ? std::min<int64_t>(chan_grid(P), 1024) : chan_grid(P);
             void* cp = nullptr;
             if (dsum)
                 if (int rc = scratch(ctx, "nn_chan_part", (size_t)nwg * 32 * sizeof(float), &cp)) return rc;
-            hipLaunchKernelGGL(k_conv1_din, dim3((unsigned)nwg), dim3(kWG), 0, ctx->stream, dout, (uint32_t)(P * 16),
-                               in, (int)B, (int)H, (int)W, 1.0 / (double)W, 1.0 / (double)H, w, act, din,
-                               (float*)cp);
+            if (dw)
+                if (int rc = scratch(ctx, "nn_conv1_dw", (size_t)nwg * 16 * kC1Ci * sizeof(float), &p)) return rc;
+            const auto kernel = dw ? k_conv1_din<true> : k_conv1_din<false>;
+            hipLaunchKernelGGL(kernel, dim3((unsigned)nwg), dim3(kWG), 0, ctx->stream, dout, (uint32_t)(P * 16), in,
+                               (int)B, (int)H, (int)W, 1.0 / (double)W, 1.0 / (double)H, w, act, din, (float*)cp,
+                               (float*)p);
             if (int rc = check_launch(ctx, "k_conv1_din")) return rc;
+            if (dw)
+                if (int rc = colsum(ctx, (const float*)p, 16 * kC1Ci, nwg, 16 * kC1Ci, 1.f, 0.f, dw, 16 * kC1Ci,
+                                    16 * kC1Ci, "nn_conv1_dw_sum"))
+                    return rc;
             if (dsum) {
                 hipLaunchKernelGGL(k_chan_final32, dim3(1), dim3(kChanFinWG), 0, ctx->stream, (const float*)cp, nwg,
                                    dsum);
                 if (int rc = check_launch(ctx, "k_chan_final32")) return rc;
             }
         }
-        if (dw) {
+        if (dw && !din) {
             // one partial per workgroup (at most 256: a single-pass column sum)
             int64_t nwg = std::min<int64_t>(256, cdiv(P, kC1DwWG / 8));
             const int64_t per = cdiv(P, nwg);
