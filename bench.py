@@ -436,7 +436,7 @@ def binaries_bench(sfh, ctx, args):
     T = sfh.binary_hess_batch(model, isos, errs, 1, (0, 1), imf, comp, None, edges, **kw)
     batch_s = time.time() - t0
     pk, _ = ctx.kernel_stats("binary_pairs")
-    dk, _ = ctx.kernel_stats("deposit_cov")
+    dk = sum(ctx.kernel_stats(k)[0] for k in ("deposit_wide", "deposit_cov"))
     ctx.set_timing(False)
     n = len(isos)
     t0 = time.time()
@@ -625,34 +625,34 @@ def templates_bench(sfh, torch, ctx, O, args, ncpu):
     for _ in range(nrep):
         out = sfh.partial_cmd_smooth_batch(isos, errs, 1, (0, 1), imf, comps, ctx=ctx, **kw)
     ctx.synchronize()
-    kern = {k: ctx.kernel_stats(k) for k in ("pcs_count", "pcs_points", "pcs_desc", "deposit_order", "deposit_cov")}
+    kern = {k: ctx.kernel_stats(k) for k in ("pcs_count", "pcs_points", "pcs_desc", "deposit_order", "deposit_wide",
+                                             "deposit_cov")}
     ctx.set_timing(False)
     kms = {k: v[0] / max(v[1], 1) for k, v in kern.items()}
-    dep_ms = kms["deposit_cov"]
+    dep_ms = kms["deposit_wide"] + kms["deposit_cov"]
     prep_ms = kms["pcs_count"] + kms["pcs_points"] + kms["pcs_desc"] + kms["deposit_order"]
     pairs_per_s = pairs / (dep_ms * 1e-3)
-    # VALU instructions per pair of the gather's dominant path (the Gaussian
-    # form over a full-width row strip of 16 bins, 94% of the pairs): per GL
-    # node and bin one FMA and one recurrence multiply (6 per pair), plus the
-    # strip's set-up amortised over its 16 bins (139 VALU instructions per
-    # strip in the compiled kernel).  The published peak counts two wave64
-    # instructions per 4 cycles per SIMD; what FP32 code of the strip's mix
-    # (an FMA reading a scalar register, a two-register multiply) reaches is
+    # VALU instructions of the two gathers over these templates, counted by the
+    # hardware (SQ_INSTS_VALU, wave64: 6.4e8 of k_dep_wide, 9.65e8 of
+    # k_dep_gather, for 2.83e10 pairs; deterministic for these inputs): what the
+    # kernels execute, inactive lanes included.  The published peak counts two
+    # wave64 instructions per 4 cycles per SIMD; what FP32 code of the strip's
+    # mix (an FMA reading a scalar register, a two-register multiply) reaches is
     # measured in the same run by the library's issue-rate probe.
-    inst_per_strip = 139.0
-    ops_per_pair = inst_per_strip / 16.0
+    ops_per_pair = (6.4e8 + 9.65e8) * 64 / 2.83e10
     achieved = pairs_per_s * ops_per_pair
     issue = ctx.valu_issue_rate()
-    roof = {"bound": "valu", "kernel": "k_dep_gather<false>", "achieved": achieved / 1e12, "peak": VALU_PEAK / 1e12,
+    roof = {"bound": "valu", "kernel": "k_dep_wide + k_dep_gather<false>", "achieved": achieved / 1e12,
+            "peak": VALU_PEAK / 1e12,
             "unit": "T VALU lane-instructions/s", "frac": achieved / VALU_PEAK, "traffic": None,
             "measured_issue_rate": issue / 1e12, "frac_of_measured_issue_rate": achieved / issue,
             "peak_note": "peak: the published FP32 vector rate (157.3 TFLOP/s = 78.6 T FMA lane-ops/s), two VALU "
                          "instructions per 4 cycles per SIMD from two waves (no packed FP32 in this build); "
                          "measured_issue_rate: the rate independent streams of the strip's instruction mix reach "
                          "on this device in this run (sfh_probe_valu_issue, four waves per SIMD)",
-            "algorithmic": f"{ops_per_pair:g} VALU instructions per (point, bin) pair (the Gaussian-form strip: "
-                           f"3 GL nodes x (accumulate FMA + recurrence multiply) per bin, plus the strip's set-up "
-                           f"of 5 exp2 and 44 other instructions over 16 bins) x {pairs:.4g} pairs per launch; "
+            "algorithmic": f"{ops_per_pair:.3g} VALU lane-instructions per (point, bin) pair, the hardware's count of "
+                           f"both gathers on this workload (wide kernels on every fourth column, rows of one or two "
+                           f"merged Gauss-Legendre nodes) x {pairs:.4g} pairs per launch; "
                            f"peak = 256 CUs x 4 SIMDs x 32 lanes x 2.4 GHz lane-instructions/s"}
     # the same templates through the host (NumPy) preparation, for comparison
     t0 = time.time()
