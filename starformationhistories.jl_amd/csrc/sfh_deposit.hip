@@ -26,7 +26,10 @@
 // one node, 22% in rows of two): 7.5 ms with three nodes per row and every
 // column evaluated, 6.0 ms with the nodes merged, 4.0 ms (1.76 wide + 2.23)
 // with the wide kernels on a quarter of their columns and the accumulators
-// reached by LDS instead of flat accesses (VGPRs 112 -> 89).
+// reached by LDS instead of flat accesses (VGPRs 112 -> 89), 3.4 ms with the
+// kernels of 0.026 <= e < 0.2 in the sum form, 2.8 ms with the wide gather's
+// FP64 sums in registers and its workgroups by cost, 2.7 ms (1.13 + 1.59) with
+// 8-byte keys for the hit search.
 #include "sfh_internal.h"
 #include "sfh_psf.h"
 
@@ -146,6 +149,8 @@ __device__ __forceinline__ void each(const PointDesc* __restrict__ chunk, uint64
 // kStep-th column: the gather below with 16 nodes of one row per thread and
 // one form per loop, into the FP64 sums [slice][template][row][node] that
 // k_dep_gather (or k_dep_finish) interpolates.
+// VALU bound: 6.4e8 wave instructions for 700 templates, 94% of their lanes
+// active, 4.0 cycles each per SIMD; 1.13 ms (1.76 with the FP64 sums in LDS).
 __global__ __launch_bounds__(kDepBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_dep_wide(
     const PointDesc* __restrict__ desc, const PointKey* __restrict__ keys, const int64_t* __restrict__ offsets,
     const int32_t* __restrict__ order, GatherArgs a)
@@ -239,7 +244,10 @@ __device__ inline void finish_cols(const GatherArgs& a, int64_t t, int row, int 
 
 // The FP64 accumulators live in LDS (16 per thread, 32 KiB per workgroup: five
 // workgroups per CU), touched once per 64 points, so that the FP32 strip and
-// the per-point constants fit the registers of five waves per SIMD.
+// the per-point constants fit the registers of five waves per SIMD (the sums
+// in registers measured the same: 1577 against 1576 us for 700 templates).
+// VALU bound: 9.65e8 wave instructions, 57% of their lanes active (the short
+// footprints of the sum and erf-difference forms), 3.7 cycles each per SIMD.
 template <bool kAsym>
 __global__ __launch_bounds__(kDepBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_dep_gather(
     const PointDesc* __restrict__ desc, const PointKey* __restrict__ keys, const int64_t* __restrict__ offsets,
