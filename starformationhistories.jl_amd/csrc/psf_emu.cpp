@@ -8,7 +8,7 @@
 // add each bin straight into FP64.  Lets the CPU test-suite check the FP32
 // formulation and the footprint index math against the FP64 oracle without a
 // GPU.
-#include "../../starformationhistories.jl_amd/csrc/sfh_psf.h"
+#include "sfh_psf.h"
 
 #include <cstring>
 #include <vector>
