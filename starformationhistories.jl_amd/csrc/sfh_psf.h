@@ -51,6 +51,8 @@ constexpr float kGaussEps = 0.026f;   // the Gaussian form below this half width
 // h^2 (1 + 2 g^2), h = half row height / sigma_y
 constexpr double kOneNodeEta = 0.00135;
 constexpr double kTwoNodeEta = 0.03;
+// ... and where the strips' multipliers 2^(+-2 m du) stay finite (gauss_strip)
+constexpr double kMaxLogB = 120.0;
 // Wide kernels (merged Gaussian forms whose footprint spans the grid's width)
 // are evaluated on every kStep-th column only, and the sum over all of them is
 // interpolated to the columns between with kTaps-point Lagrange weights
@@ -91,9 +93,8 @@ struct alignas(16) PointDesc {
                             // nodes' x shifts g t -+ s3; kSum: the outer Gaussians' x shifts
                             // -+ s3 and the middle one's amplitude s1 over theirs
     int32_t kind;
-    float gf, gfi;          // kGauss, covariant, and kGauss2: 2^(2 v du) and its inverse, v the x
-                            // distance of a row's outer nodes from its middle (g ey, or s3): the
-                            // nodes' strip multipliers relative to the middle's
+    float gf, gfi;          // kGauss2: 2^(2 s3 du) and its inverse, the nodes' strip multipliers
+                            // relative to the middle's
     int32_t terms;          // kGauss: 1; kSum: 2 or 3 Gaussians
     int32_t pad0;
     float q[8];             // Gaussian forms: q[j] = 2^-(du (j + 1/2))^2, the strip's column factors
@@ -229,10 +230,9 @@ __host__ __device__ constexpr InterpWeights interp_weights()
     return t;
 }
 
-// The strip constants of a Gaussian form with column step du and the rows'
-// outer nodes a coordinate distance v from the middle, from the rounded
-// values that the kernel uses (gauss_strip).
-__host__ __device__ inline void set_strip(PointDesc* d, double v)
+// The column factors of a Gaussian form's strips, from the rounded step du that
+// the kernel uses (gauss_strip).
+__host__ __device__ inline void set_strip(PointDesc* d)
 {
     // (j + 3/2)^2 - (j + 1/2)^2 = 2 (j + 1): two exp2 and products in FP64 instead
     // of an exp2 per column (they were most of a descriptor's cost)
@@ -243,9 +243,6 @@ __host__ __device__ inline void set_strip(PointDesc* d, double v)
         q *= p;
         p *= w;
     }
-    const double r = exp2(2.0 * v * du);
-    d->gf = (float)r;
-    d->gfi = (float)(1.0 / r);
 }
 
 // The x coordinates of a merged Gaussian form (ax, du: scaled), whose footprint
@@ -261,12 +258,15 @@ __host__ __device__ inline void set_merged_x(PointDesc* d, int32_t kind, double 
     }
     d->ax = (float)ax;
     d->du = (float)du;
-    set_strip(d, (double)d->s3);
+    set_strip(d);
+    const double r = exp2(2.0 * (double)d->s3 * (double)d->du);
+    d->gf = (float)r;
+    d->gfi = (float)(1.0 / r);
 }
 
 // A covariant kernel in the Gaussian form with its rows' Gauss-Legendre nodes
 // merged (only for a footprint that spans the grid's width); false where the
-// row is too high for that (the three nodes stay).
+// row is too high for that, or its shear too large (the three nodes stay).
 // Around a row centre t, phi = t^2/2 + gam (u + g t)^2 (gam = 1 - b) has the
 // t-derivative s = k2 t + 2 gam g u, k2 = 1 + 2 gam g^2, and the three nodes at
 // t, t +- dl (dl = xi hy / sy) sum exactly to
@@ -302,6 +302,11 @@ __host__ __device__ inline bool set_row_nodes(PointDesc* d, double ax, double du
         lam = bd * (k2 - 2.0 * gam * g * g1);
         pre *= 0.5 * exp(A * v * v);
     }
+    // |2 m du| over every strip: m reaches the rows' shear, the nodes' shift and the
+    // x range of the columns (and of up to eight strips' width past them)
+    const double tm = fmax(fabs((double)d->ay), fabs((double)d->ay + (double)(d->yb - d->ya) * (double)d->dv));
+    const double span = fabs(ax) + (double)(nx + 8 * kCPT) * fabs(du);
+    if (!(2.0 * kStep * fabs(du) * scale * scale * (fabs(g1) * tm + fabs(v) + span) <= kMaxLogB)) return false;
     d->pref = (float)((double)d->pref * pre);
     d->g = (float)(g1 * scale);
     d->s1 = (float)(-rho * kLog2e);
@@ -341,7 +346,7 @@ __host__ __device__ inline void set_sum(PointDesc* d, double ax, double du, doub
     d->ax = (float)(ax * scale);
     d->du = (float)(du * scale);
     d->g = (float)(g * scale);
-    set_strip(d, (double)d->g * (double)d->ey);
+    set_strip(d);
 }
 
 // The form of a point with x coordinate ax of its first column, column step du
@@ -381,7 +386,7 @@ __host__ __device__ inline void set_x_form(PointDesc* d, double ax, double du, b
     d->ax = (float)(ax * scale);
     d->du = (float)(du * scale);
     d->g = (float)(g * scale);
-    set_strip(d, (double)d->g * (double)d->ey);
+    set_strip(d);
 }
 
 // Covariant kernel centred at (x0, y0) (real units) -- addstar! :366-408.
@@ -486,6 +491,15 @@ __host__ __device__ inline float fast_exp2(float x)
     return __builtin_amdgcn_exp2f(x);
 #else
     return std::exp2(x);
+#endif
+}
+
+__host__ __device__ inline float clamp126(float x)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_fmed3f(x, -126.0f, 126.0f);
+#else
+    return fminf(fmaxf(x, -126.0f), 126.0f);
 #endif
 }
 
@@ -630,15 +644,22 @@ __host__ __device__ __forceinline__ void static_for(F&& f)
 // With m the x coordinate midway between columns 7 and 8 and s = c - 7.5,
 //   (m + s du)^2 = m^2 + 2 s m du + s^2 du^2,
 // so E(8 + j) = P B^j q[j] and E(7 - j) = P B^-(j+1) q[j], P = 2^-(m^2 + m du),
-// B = 2^(-2 m du), q[j] = 2^-(du (j + 1/2))^2 (prepared per point).  For the
-// three GL nodes (m_k - m_1 = -+g ey) the outer nodes' B are the middle node's
-// times 2^(+-2 g ey du) (prepared per point), so a row takes 5 exp2 (3 for the
-// asymmetric kernel) instead of one per node and column (an exp2 takes two
-// VALU issue slots, an FMA or multiply one), and a column costs one FMA and
-// one multiply per node.  The multiplier's rounding grows over at most 8
-// steps.  The Gaussian form has du < 0.064 (half bin width e < 0.026), so B
-// stays within [2^-2, 2^2] for |m| < 15.  Each column adds the nodes in order
-// k = 0, 1, 2.
+// B = 2^(-2 m du), q[j] = 2^-(du (j + 1/2))^2 (prepared per point).  A row takes
+// three exp2 per node instead of one per node and column (an exp2 takes two
+// VALU issue slots, an FMA or multiply one), and a column costs one FMA and one
+// multiply per node.  Each column adds the nodes in order k = 0, 1, 2.
+//
+// B and 1/B have to stay finite: where a far strip's P has underflowed to 0, a
+// product with an infinite one would be a NaN.  Without shear |m| stays within
+// the footprint's 5.3 standard deviations and a strip, and the merged nodes'
+// |2 m du| is bounded at the preparation (kMaxLogB, set_row_nodes).  The three GL
+// nodes' m holds the rows' shear g t, which has no bound, so their exponent is
+// clamped to +-126: du < 0.5 (half bin width e < 0.2), so |m| > 126 where the
+// clamp acts, and P is 0 there, and stays 0.  Their B are computed node by node:
+// a node's B is used where its own |m| is small, and as the middle node's B times
+// a prepared 2^(2 g ey du) it would carry the rounding of an exponent as large as
+// the nodes' distance (1e-5 of the peak in rows much higher than the kernel).
+// The two merged nodes lie within 0.1 of each other and share one.
 template <int NODES>
 __host__ __device__ __forceinline__ void gauss_strip(const PointDesc& d, const float* M, const float* L,
                                                      const float* h, int col0, float* part)
@@ -647,31 +668,26 @@ __host__ __device__ __forceinline__ void gauss_strip(const PointDesc& d, const f
     static_assert(NODES >= 1 && NODES <= 3, "one node, two merged ones or three GL nodes");
     const float base = fmaf((float)(col0 - d.xa), d.du, d.ax);
     const float du = d.du;
-    float pf[NODES], B[NODES], Bi[NODES];
-    float m0 = 0.0f;                       // the coordinate whose B is computed: the nodes' middle
+    float m[NODES], pf[NODES], B[NODES], Bi[NODES];
 #pragma unroll
     for (int k = 0; k < NODES; ++k) {
-        const float m = fmaf(7.5f, du, base + h[k]);
-        pf[k] = M[k] * fast_exp2(L[k] - m * (m + du));
-        if (NODES == 2 || k == NODES / 2) m0 += NODES == 2 ? 0.5f * m : m;
+        m[k] = fmaf(7.5f, du, base + h[k]);
+        pf[k] = M[k] * fast_exp2(L[k] - m[k] * (m[k] + du));
     }
-    const float md2 = 2.0f * m0 * du;
-    const float Bm = fast_exp2(-md2), Bmi = fast_exp2(md2);
-    if constexpr (NODES == 1) {
-        B[0] = Bm;
-        Bi[0] = Bmi;
-    } else if constexpr (NODES == 2) {
+    if constexpr (NODES == 2) {
+        const float md2 = (m[0] + m[1]) * du;
+        const float Bm = fast_exp2(-md2), Bmi = fast_exp2(md2);
         B[0] = Bm * d.gf;
         Bi[0] = Bmi * d.gfi;
         B[1] = Bm * d.gfi;
         Bi[1] = Bmi * d.gf;
     } else {
-        B[1] = Bm;
-        Bi[1] = Bmi;
-        B[0] = B[1] * d.gf;
-        Bi[0] = Bi[1] * d.gfi;
-        B[2] = B[1] * d.gfi;
-        Bi[2] = Bi[1] * d.gf;
+#pragma unroll
+        for (int k = 0; k < NODES; ++k) {
+            const float md2 = NODES == 3 ? clamp126(2.0f * m[k] * du) : 2.0f * m[k] * du;
+            B[k] = fast_exp2(-md2);
+            Bi[k] = fast_exp2(md2);
+        }
     }
 #pragma unroll
     for (int k = 0; k < NODES; ++k) {

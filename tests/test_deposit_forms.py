@@ -44,6 +44,75 @@ def test_single_kernels_of_every_width(sfh, emu, O, nx, ny, cov_mult):
     assert worst <= TOL, worst
 
 
+# few high rows, fine columns, and kernels of about two columns much higher than wide
+STEEP = [(200, 300, 2.0, 34.0, 1, None), (200, 300, 2.0, 40.0, 1, None), (200, 300, 1.78, 30.0, -1, None),
+         (1000, 300, 1.8, 30.0, 1, None), (300, 5, 1.96, 3.357, -1, None), (300, 5, 2.45, 5.29, 1, None)]
+
+
+def _sheared():
+    """(nx, ny, sigma_x in columns, sigma_y / sigma_x, cov_mult, cmult): sigma_x
+    across every change of form, sigma_y / sigma_x from 1/100 to 100, grids of few
+    high rows and of fine columns, and the shears of correlations close to 1."""
+    rng = np.random.default_rng(5)
+    for nx, ny in ((200, 300), (300, 5), (1000, 4), (75, 100), (28, 40)):
+        for sxc in np.geomspace(1.5, 0.6 * nx, 24):
+            for ratio in np.geomspace(0.01, 100.0, 9) * rng.uniform(0.8, 1.25):
+                yield nx, ny, sxc, ratio, 1, None
+                yield nx, ny, sxc, ratio, -1, None
+                r = 1.0 - 10.0 ** rng.uniform(-5.0, 0.0)
+                yield nx, ny, sxc, ratio, 1, rng.choice([-1, 1]) * r / np.sqrt(1.0 - r * r) / ratio
+                yield nx, ny, sxc, ratio, 1, rng.normal() * 10.0 ** rng.uniform(-1.0, 1.0)
+    yield from STEEP
+
+
+def _check_sheared(sfh, O, case, evaluate):
+    """A kernel next to a row's middle node (between the nodes a kernel much
+    narrower than a row has no part on the grid): finite, and within the
+    coordinates' rounding.  With T the largest row coordinate |t| of the
+    footprint, a row's t is off by dt = 3 2^-24 T and a column's a = u + g t by
+    |g| dt and its own 3 2^-24 |u|, |u| < 8.  A value exp(-t^2 / 2 - a^2) is off
+    by t dt + 2 a da of itself; relative to the peak's (at t_p, a_p) the factor
+    2 a exp(a_p^2 - a^2) is below 2 (a_p + 0.43)."""
+    nx, ny, sxc, ratio, cov_mult, cm = case
+    ex, ey = sfh.edges_range(-0.5, 2.5, nx + 1), sfh.edges_range(18.0, 30.0, ny + 1)
+    x, y, sx = 1.0 + 0.3 * ex.step, 18.0 + (ny // 2 + 0.51) * ey.step, sxc * ex.step
+    sy = ratio * sx
+    p = [np.array([v]) for v in (x, y, sx, sy, 1.0)]
+    cmult = None if cm is None else np.array([cm])
+    ref, _ = O.bin_cmd_smooth(*p[:4], cov_mult, p[4], oracle_range(O, ex), oracle_range(O, ey), cmult=cmult)
+    mat = evaluate(p, cov_mult, ex, ey, cmult)
+    assert np.isfinite(mat).all(), case
+    peak = ref.max()
+    if peak < 1e-9:            # a ridge that misses the bins: the oracle's own erf differences are noise
+        return
+    eps = 2.0 ** -24
+    t = (18.0 + (np.arange(ny)[:, None] + 0.5 + 0.387 * np.array([-1, 0, 1])) * ey.step - y) / sy
+    T = np.abs(t[np.abs(np.arange(ny) - ny // 2) <= max(1, round(5.0 * sy / ey.step)) + 1]).max()
+    g = (cov_mult if cm is None else cm) * ratio / np.sqrt(2.0)
+    col, row = np.unravel_index(ref.argmax(), ref.shape)
+    a = np.abs((-0.5 + (col + 0.5) * ex.step - x) / (np.sqrt(2.0) * sx) + g * t[row])
+    k = np.argmin(0.5 * t[row] ** 2 + a ** 2)
+    dt = 3.0 * eps * T
+    tol = TOL + abs(t[row, k]) * dt + 2.0 * (a[k] + 0.43) * (abs(g) * dt + 3.0 * eps * 8.0)
+    worst = np.max(np.abs(mat - ref)) / peak
+    assert worst <= tol, (worst, tol, case)
+
+
+def test_sheared_kernels(sfh, emu, O):
+    """The shift g t of a row's columns moves its ridge far out of the strips,
+    whose products have to stay finite."""
+    for case in _sheared():
+        _check_sheared(sfh, O, case, lambda p, cov_mult, ex, ey, cmult: _emu(
+            emu, O, *p, cov_mult, oracle_range(O, ex), oracle_range(O, ey), cmult=cmult)[0])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", STEEP)
+def test_sheared_kernels_on_the_device(sfh, gpu_ctx, O, case):
+    _check_sheared(sfh, O, case, lambda p, cov_mult, ex, ey, cmult: sfh.bin_cmd_smooth(
+        *p[:4], cov_mult, weights=p[4], edges=(ex, ey)).weights)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("nx,ny,n", [(200, 300, 1), (200, 300, 1500), (201, 77, 65), (33, 40, 63), (29, 41, 64),
                                      (28, 17, 129), (17, 5, 40), (16, 9, 300), (3, 2, 10), (1, 2, 5)])
