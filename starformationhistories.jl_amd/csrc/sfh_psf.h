@@ -16,7 +16,8 @@
 //                with t_k = (y_j + xi_k hy - y0)/sy (3-point Gauss-Legendre, :303-304),
 //                g = c sy / (sqrt(2) sx)  (the reference's Δx = dx + c Δy, :328);
 //   asymmetric : A/4 * D(u_i, ex) * D(v_j, ey)  (:203-204; the two sign flips cancel).
-// For e < kSumEps, D is evaluated without the erf-difference cancellation as
+// For e < kSumEps (kSumEpsAsym for asymmetric kernels), D is evaluated without the
+// erf-difference cancellation as
 //   D = (4 e / sqrt(pi)) <exp(-(u+s)^2)>, the mean over |s| < e:
 // e < 0.026, the Gaussian form: the mean is exp(-u^2) S(u^2), S(w) =
 //   sum_n H_2n(sqrt w) e^2n / (2n+1)! = s0 exp(b w) (1 + O(b^2 w^2)), b = s1 / s0
@@ -28,7 +29,10 @@
 //   the sums.  On the 700-template workload 97% of the pairs take this form.
 // 0.026 <= e < kSumEps, the sum form: the mean as two Gaussians (e < kPairEps),
 //   whose first wrong term of ln is 3e-5 (2 u e)^6, at most 2.6e-3 e^6 of the
-//   peak, or three, with 1.4e-7 (2 u e)^8, at most 1.7e-4 e^8 (set_sum).
+//   peak, or three, with 1.4e-7 (2 u e)^8, at most 1.7e-4 e^8 (set_sum).  Relative
+//   to the local value at |u| = 3.7, where a kernel is 1e-6 of its peak, that is
+//   1.4e-7 (two) and 5e-8 (three, e = 0.12); at e = 0.2 it would be 3.2e-6, and
+//   a template's worst bin above 1e-6 of its maximum 4e-6 off instead of 1.6e-6.
 // Both run in scaled coordinates a = u sqrt(log2 e) times the square root of
 // their Gaussian's own factor, so a Gaussian is one hardware exp2 of -a^2.
 #pragma once
@@ -44,13 +48,17 @@ namespace psf {
 
 constexpr float kSeriesEps = 0.1f;    // an asymmetric kernel's y factor as a series below this half height
 constexpr float kPairEps = 0.055f;    // x: the sum form's two Gaussians below this half width, three above
-constexpr float kSumEps = 0.2f;       // the sum form below, erf differences above
+constexpr float kSumEps = 0.12f;      // the sum form below, erf differences above: covariant kernels ...
+constexpr float kSumEpsAsym = 0.1f;   // ... and asymmetric ones
 constexpr float kGaussEps = 0.026f;   // the Gaussian form below this half width
 // Covariant kernels in the Gaussian form: the row's three Gauss-Legendre nodes
 // merged into one node or two (set_row_nodes) up to these values of
-// h^2 (1 + 2 g^2), h = half row height / sigma_y
+// h^2 (1 + 2 g^2), h = half row height / sigma_y.  Two nodes up to 0.03 keep the
+// peak's error as small, but put templates' worst bin above 1e-6 of the maximum
+// at 2.7e-6 instead of the three nodes' 2.5e-6 (0.018: 2.5e-6); 700 templates of
+// 200 x 300 bins take 3.81 ms up to 0.03, 3.86 up to 0.018, 4.02 up to 0.01.
 constexpr double kOneNodeEta = 0.00135;
-constexpr double kTwoNodeEta = 0.03;
+constexpr double kTwoNodeEta = 0.018;
 // ... and where the strips' multipliers 2^(+-2 m du) stay finite (gauss_strip)
 constexpr double kMaxLogB = 120.0;
 // Wide kernels (merged Gaussian forms whose footprint spans the grid's width)
@@ -89,9 +97,9 @@ struct alignas(16) PointDesc {
     float dv;     // t (or v) step per row
     float ey;     // covariant: GL node offset xi*hy/sy; asymmetric: half row width in v
     float pref;   // amplitude prefactor (see header), with the series form factors
-    float s1, s2, s3;       // kGauss1 / kGauss2: a row's y weight 2^(s1 t^2 +- s2 t) and the
-                            // nodes' x shifts g t -+ s3; kSum: the outer Gaussians' x shifts
-                            // -+ s3 and the middle one's amplitude s1 over theirs
+    float s1, s2, s3;       // a row's y weight, kGauss1: 2^(s1 t^2 + s2 t^4), kGauss2: 2^(s1 t^2 +-
+                            // s2 t) and the nodes' x shifts g t -+ s3; kSum: the outer Gaussians' x
+                            // shifts -+ s3 and the middle one's amplitude s1 over theirs
     int32_t kind;
     float gf, gfi;          // kGauss2: 2^(2 s3 du) and its inverse, the nodes' strip multipliers
                             // relative to the middle's
@@ -280,7 +288,7 @@ __host__ __device__ inline void set_merged_x(PointDesc* d, int32_t kind, double 
 // Two nodes: F = exp(al x^2) cosh(be x) with the x^2 and x^4 terms of ln F
 // (be^4 = (3 p^2 - p) / 2, al = p/2 - be^2/2): two Gaussians with the shifts
 // g' t -+ v.  Its first dropped term, 2.9e-4 x^6, is at most 6.6e-4 eta^3 =
-// 1.8e-8 of the peak for eta < 0.03.
+// 3.9e-9 of the peak for eta < 0.018.
 __host__ __device__ inline bool set_row_nodes(PointDesc* d, double ax, double du, double gam, double g, int nx)
 {
     const double dl = (double)d->ey, k2 = 1.0 + 2.0 * gam * g * g;
@@ -310,7 +318,7 @@ __host__ __device__ inline bool set_row_nodes(PointDesc* d, double ax, double du
     d->pref = (float)((double)d->pref * pre);
     d->g = (float)(g1 * scale);
     d->s1 = (float)(-rho * kLog2e);
-    d->s2 = (float)(lam * kLog2e);
+    d->s2 = (float)(lam * kLog2e);        // (0 for one node)
     d->s3 = (float)(v * scale);
     set_merged_x(d, one ? kGauss1 : kGauss2, ax * scale, du * scale, nx);
     return true;
@@ -352,11 +360,13 @@ __host__ __device__ inline void set_sum(PointDesc* d, double ax, double du, doub
 // The form of a point with x coordinate ax of its first column, column step du
 // and half width d->ex (in u) on a grid of nx columns.  cov: a covariant
 // kernel of shear g; else an asymmetric one, whose y factor joins a merged
-// Gaussian form (one node, no shear) where it has the Gaussian form itself.
+// Gaussian form (one node, no shear) where it has the Gaussian form itself, with
+// the next term of its ln S, -(4/45) e^4 v^4, in the row's weight (without it the
+// RMS error of a template's bins was 1.8e-7 instead of 1.5e-7).
 __host__ __device__ inline void set_x_form(PointDesc* d, double ax, double du, bool cov, double g, int nx)
 {
     const float e = d->ex;
-    if (!(e < kSumEps)) {
+    if (!(e < (cov ? kSumEps : kSumEpsAsym))) {
         d->kind = kDirect;
         d->ax = (float)ax;
         d->du = (float)du;
@@ -380,6 +390,8 @@ __host__ __device__ inline void set_x_form(PointDesc* d, double ax, double du, b
         const Series y = series_coeffs(d->ey);
         d->pref = (float)((double)d->pref * (double)y.s0);
         d->s1 = (float)(-(1.0 - (double)y.s1 / (double)y.s0) * kLog2e);
+        const double ey2 = (double)d->ey * (double)d->ey;
+        d->s2 = (float)(-4.0 / 45.0 * ey2 * ey2 * kLog2e);
         set_merged_x(d, kGauss1, ax * scale, du * scale, nx);
         return;
     }
@@ -467,7 +479,7 @@ __host__ __device__ inline int64_t prep_asymmetric(double col, double mag, doubl
     d.dv = (float)(1.0 / s2y);
     d.ey = (float)(0.5 / s2y);
     double pref = A / 4.0;
-    if (d.ex < kSumEps) pref *= 4.0 * (0.5 / s2x) / 1.7724538509055160;
+    if (d.ex < kSumEpsAsym) pref *= 4.0 * (0.5 / s2x) / 1.7724538509055160;
     if (d.ey < kSeriesEps) pref *= 4.0 * (0.5 / s2y) / 1.7724538509055160;
     d.pref = (float)pref;
     // evaluate at i + 1/2 :361
@@ -607,7 +619,7 @@ __host__ __device__ inline void merged_row(const PointDesc& d, int row, float* M
     const float t = fmaf((float)(row - d.ya), d.dv, d.ay);
     if constexpr (NODES == 1) {
         M[0] = d.pref;
-        L[0] = d.s1 * t * t;
+        L[0] = fmaf(d.s2, t * t, d.s1) * (t * t);
         h[0] = d.g * t;
     } else {
         M[0] = M[1] = d.pref;
@@ -654,7 +666,7 @@ __host__ __device__ __forceinline__ void static_for(F&& f)
 // the footprint's 5.3 standard deviations and a strip, and the merged nodes'
 // |2 m du| is bounded at the preparation (kMaxLogB, set_row_nodes).  The three GL
 // nodes' m holds the rows' shear g t, which has no bound, so their exponent is
-// clamped to +-126: du < 0.5 (half bin width e < 0.2), so |m| > 126 where the
+// clamped to +-126: du < 0.3 (half bin width e < 0.12), so |m| > 200 where the
 // clamp acts, and P is 0 there, and stays 0.  Their B are computed node by node:
 // a node's B is used where its own |m| is small, and as the middle node's B times
 // a prepared 2^(2 g ey du) it would carry the rounding of an exponent as large as

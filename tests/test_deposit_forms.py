@@ -44,6 +44,28 @@ def test_single_kernels_of_every_width(sfh, emu, O, nx, ny, cov_mult):
     assert worst <= TOL, worst
 
 
+@pytest.mark.parametrize("kind,bound", [("asym", 2.2e-6), ("cov", 3.3e-6), ("corr", 3.3e-6)])
+def test_tails_of_templates(sfh, emu, O, kind, bound):
+    """Every bin above 1e-6 of a template's maximum.  A kernel's value there is 2^-20
+    of its peak: two roundings of an exponent of 20 (20 ln 2 2^-24 = 8e-7), and of
+    its coordinates |a| < 3.7 (2 |a| da, da = 2^-25 |a| for each of two in the
+    asymmetric kernel, 1.6e-6, and of three with the shear, 2.4e-6).  What the forms
+    leave out is below that."""
+    from sfh_amd import synth
+    edges = synth.edges_200x300()
+    ex, ey = oracle_range(O, edges[0]), oracle_range(O, edges[1])
+    for la, mh, seed in ((6.74, -2.5, 100), (8.16, -1.14, 105), (8.72, -0.23, 107), (9.86, 0.0, 111)):
+        sp, cm = synth.template_points(synth.TemplateSpec(la, mh, seed), 1200, edges, 120.0,
+                                       correlation=0.6 if kind == "corr" else None)
+        p = (sp.colors, sp.mags, sp.color_err, sp.mag_err, sp.weights)
+        cov_mult, cm = 0 if kind == "asym" else 1, cm if kind == "corr" else None
+        ref, _ = O.bin_cmd_smooth(*p[:4], cov_mult, p[4], ex, ey, cmult=cm, nthreads=8)
+        mat, _ = _emu(emu, O, *p, cov_mult, ex, ey, cmult=cm)
+        big = ref > 1e-6 * ref.max()
+        worst = np.max(np.abs(mat[big] - ref[big]) / ref[big])
+        assert worst <= bound, (worst, la, mh, seed)
+
+
 # few high rows, fine columns, and kernels of about two columns much higher than wide
 STEEP = [(200, 300, 2.0, 34.0, 1, None), (200, 300, 2.0, 40.0, 1, None), (200, 300, 1.78, 30.0, -1, None),
          (1000, 300, 1.8, 30.0, 1, None), (300, 5, 1.96, 3.357, -1, None), (300, 5, 2.45, 5.29, 1, None)]
