@@ -306,13 +306,15 @@ __global__ __launch_bounds__(kDepBlock) __attribute__((amdgpu_waves_per_eu(4))) 
         if (!in_rows(d) || col0 > d.xb || col0 + kCPT - 1 < d.xa) return;
         psf::add_point<!kAsym>(d, row, col0, part);
     };
-    // A point in the erf-difference form (a kernel so narrow that its footprint
-    // is at most 37 columns wide) with the whole wave cooperating, instead of
-    // strip code in which only the few lanes whose strips meet the footprint
-    // would work: segments of 16, 32 or 64 lanes take one of the point's rows
-    // inside this wave's strips each, lane l of a segment footprint column
-    // xa + l; lanes 0 .. nc evaluate erfc at their column's left edge (its sign
-    // that of the edge) and a column's right edge is the next lane's.  Each
+    // A point in the erf-difference form (a kernel narrower than 3 columns, 3.6
+    // in the asymmetric case: a footprint of 45 or 37 columns at most) with the
+    // whole wave cooperating, instead of strip code in which only the few lanes
+    // whose strips meet the footprint would work: segments of 16, 32 or 64 lanes
+    // take one of the point's rows inside this wave's strips each, lane l of a
+    // segment footprint column xa + l; lanes 0 .. nc evaluate erfc at their
+    // column's left edge (its sign that of the edge) and a column's right edge is
+    // the next lane's.  A wider footprint (edges so far from 0 that adding steps
+    // to them rounds) is taken in blocks of a segment's columns.  Each
     // bin's value (nodes summed in order, in FP32) is added to its owner's
     // FP64 accumulator in LDS: the bins are distinct, so no two lanes write one
     // word, and the owner's own flush comes later in program order.
@@ -320,10 +322,11 @@ __global__ __launch_bounds__(kDepBlock) __attribute__((amdgpu_waves_per_eu(4))) 
         constexpr int NODES = kAsym ? 1 : 3;
         const int nc = d.xb - d.xa + 1;
         const int lw = nc < 16 ? 4 : nc < 32 ? 5 : 6;          // nc + 1 edges per segment
-        const int l = lane & ((1 << lw) - 1);
+        const int ls = lane & ((1 << lw) - 1), wide = (1 << lw) - 1;
         const int r0 = d.ya > row_lo ? d.ya : row_lo, r1 = d.yb < row_hi ? d.yb : row_hi;
+        for (int cb = 0; cb < nc; cb += wide)
         for (int rp = r0; rp <= r1; rp += 64 >> lw) {
-            const int r = rp + (lane >> lw);
+            const int l = cb + ls, r = rp + (lane >> lw);
             float W[3], h[3] = {0.0f, 0.0f, 0.0f};
             if constexpr (kAsym) W[0] = d.pref * psf::y_factor(fmaf((float)(r - d.ya), d.dv, d.ay), d.ey);
             else psf::cov_row(d, r, W, h);
@@ -336,7 +339,7 @@ __global__ __launch_bounds__(kDepBlock) __attribute__((amdgpu_waves_per_eu(4))) 
                     __builtin_amdgcn_update_dpp(0, __float_as_int(e), 0x130, 0xf, 0xf, false));
                 v = fmaf(W[k], psf::erf_diff(e, e1), v);
             }
-            if (l < nc && r <= r1) {
+            if (l < nc && ls < wide && r <= r1) {
                 const int col = d.xa + l;
                 const int o = r * ncg + col / kCPT - wslot;
                 if (o >= 0 && o < 64) {

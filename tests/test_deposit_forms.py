@@ -2,6 +2,8 @@
 wide kernels on every fourth column with interpolation between, launches whose
 points are split into slices -- against the FP64 oracle, at the sizes where
 their dispatch changes."""
+from types import SimpleNamespace
+
 import numpy as np
 import pytest
 
@@ -147,6 +149,31 @@ def test_one_template(sfh, gpu_ctx, O, nx, ny, n, cov_mult):
     ref, _ = O.bin_cmd_smooth(*p[:4], cov_mult, p[4], oracle_range(O, ex), oracle_range(O, ey))
     h = sfh.bin_cmd_smooth(*p[:4], cov_mult, weights=p[4], edges=(ex, ey))
     assert np.max(np.abs(h.weights - ref)) <= TOL * np.max(np.abs(ref))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("xo", [33, 35, 37])
+def test_wide_footprint_of_erf_differences(sfh, gpu_ctx, emu, O, xo):
+    """Edges so far from 0 that adding steps to them rounds to multiples of 64
+    steps: the columns come out wider than the step that the footprint is counted
+    in, so an erf-difference kernel's footprint spans 2 xo + 1 > 63 columns, which
+    the shear's ridge crosses from end to end.  Against the host build, which
+    takes a footprint column by column (the oracle rounds every column's
+    coordinate, which here moves columns by half a width)."""
+    first = 2.0 ** 58
+    ex, ey = sfh.Range(first, 1.0, 401), sfh.edges_range(18.0, 21.0, 41)
+    q = SimpleNamespace(cov_mult=1)
+    sx = (2.0 * xo - 0.5) / 15.0                        # round(15 sx / 2) = xo
+    for x in (128, 192, 256):
+        xa, xb = x + 1 - xo, x + 1 + xo
+        step = ((first + (xb - 0.5)) - (first + (xa - 0.5))) / (xb - xa)
+        assert xb - xa + 1 > 63 and step / (2.0 * np.sqrt(2.0) * sx) > 0.12
+        q.colors, q.mags, q.color_err, q.mag_err, q.weights = p = [np.array([v]) for v in (first + x, 19.5, sx, 0.2, 1.0)]
+        for c in (100.0, -100.0):
+            ref, _ = _emu(emu, O, *p, 1, oracle_range(O, ex), oracle_range(O, ey), cmult=np.array([c]))
+            assert ref[xa - 1:xb].max(axis=1).min() > 1e-4 * ref.max()
+            h = sfh.deposit_batch(sfh.PointBatch([q], (ex, ey), cmult_list=[np.array([c])])).cpu().numpy()
+            assert np.max(np.abs(h[0] - ref.ravel(order="F"))) <= TOL * ref.max(), (x, c)
 
 
 @pytest.mark.gpu
