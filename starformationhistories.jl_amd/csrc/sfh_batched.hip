@@ -992,8 +992,8 @@ static int get_operands(sfh_ctx* ctx, const sfh_templates* tpl, int mode, Batche
         o.npad = cdiv(N, kBM) * kBM;
         o.tpad1 = std::max<int64_t>(cdiv(T, 16), 2) * 16;   // >= 2 K-blocks: the FP64 composite's loop runs in pairs
         o.tpad2 = cdiv(T, kBM) * kBM;
-        SFH_HIP_TRY(ctx, hipMalloc(&o.ex, (size_t)T * sizeof(int32_t)));
-        SFH_HIP_TRY(ctx, hipMalloc(&o.ex0, (size_t)T * sizeof(int32_t)));
+        SFH_HIP_TRY(ctx, device_alloc(ctx, &o.ex, (size_t)T * sizeof(int32_t)));
+        SFH_HIP_TRY(ctx, device_alloc(ctx, &o.ex0, (size_t)T * sizeof(int32_t)));
         SFH_HIP_TRY(ctx, hipMemsetAsync(o.ex0, 0, (size_t)T * sizeof(int32_t), ctx->stream));
         hipLaunchKernelGGL(k_template_exp, dim3((unsigned)T), dim3(256), 0, ctx->stream, tpl->d_models, ld, N, o.ex);
         if (int rc = check_launch(ctx, "k_template_exp")) return rc;
@@ -1002,7 +1002,7 @@ static int get_operands(sfh_ctx* ctx, const sfh_templates* tpl, int mode, Batche
     const int ai = mode == BF16X2 ? 1 : 0;
     if (!o.a1[ai]) {
         const size_t bytes = (size_t)nkb1 * nrb1 * 2 * 64 * sizeof(uint4);
-        if (hipMalloc(&o.a1[ai], bytes) != hipSuccess) {
+        if (device_alloc(ctx, &o.a1[ai], bytes) != hipSuccess) {
             o.a1[ai] = nullptr;
             return set_error(ctx, SFH_ERR_ALLOC, "hipMalloc(%zu) for composite operand failed", bytes);
         }
@@ -1018,7 +1018,7 @@ static int get_operands(sfh_ctx* ctx, const sfh_templates* tpl, int mode, Batche
     if (!o.a2[gi]) {
         const int64_t nrb2 = o.tpad2 / 32, nkb2 = o.npad / 16;
         const size_t bytes = (size_t)nkb2 * nrb2 * 2 * 64 * sizeof(uint4);
-        if (hipMalloc(&o.a2[gi], bytes) != hipSuccess) {
+        if (device_alloc(ctx, &o.a2[gi], bytes) != hipSuccess) {
             o.a2[gi] = nullptr;
             return set_error(ctx, SFH_ERR_ALLOC, "hipMalloc(%zu) for gradient operand failed", bytes);
         }

@@ -22,6 +22,7 @@
 // All reductions are in FP64 and in a fixed order (bitwise reproducible).
 #include "sfh_internal.h"
 
+#include <algorithm>
 #include <cmath>
 #include <cstdarg>
 #include <cstring>
@@ -56,64 +57,82 @@ int scratch(sfh_ctx* ctx, const char* name, size_t bytes, void** out)
             b.bytes = 0;
         }
         size_t want = bytes < 256 ? 256 : bytes;
-        hipError_t e = hipMalloc(&b.ptr, want);
-        if (e != hipSuccess && ctx->pool_bytes > 0) {
-            (void)hipGetLastError();
-            pool_clear(ctx);
-            e = hipMalloc(&b.ptr, want);
-        }
-        if (e != hipSuccess) {
-            b.ptr = nullptr;
+        if (device_alloc(ctx, &b.ptr, want) != hipSuccess)
             return set_error(ctx, SFH_ERR_ALLOC, "hipMalloc(%zu) for scratch '%s' failed", want, name);
-        }
         b.bytes = want;
     }
     *out = b.ptr;
     return SFH_OK;
 }
 
+// The contexts alive.  Lock order: g_ctxs_mu, then a context's pool_mu; neither
+// is held while a context's own lock is waited for.
+static std::mutex g_ctxs_mu;
+static std::vector<sfh_ctx*>& g_ctxs = *new std::vector<sfh_ctx*>;     // outlives every context
+
 void pool_clear(sfh_ctx* ctx)
 {
-    for (DevBuf& b : ctx->pool) (void)hipFree(b.ptr);     // waits for the work on them
-    ctx->pool.clear();
-    ctx->pool_bytes = 0;
+    std::lock_guard<std::mutex> g(ctx->pool_mu);
+    for (size_t i = 0; i < ctx->pool_n; ++i) (void)hipFree(ctx->pool[i].ptr);     // waits for the work on them
+    ctx->pool_n = ctx->pool_bytes = 0;
+}
+
+hipError_t device_alloc(sfh_ctx* ctx, void** out, size_t bytes)
+{
+    hipError_t e = hipMalloc(out, bytes);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        {
+            std::lock_guard<std::mutex> g(g_ctxs_mu);
+            for (sfh_ctx* c : g_ctxs)
+                if (c->device == ctx->device) pool_clear(c);
+        }
+        e = hipMalloc(out, bytes);
+    }
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        *out = nullptr;
+    }
+    return e;
 }
 
 int pool_get(sfh_ctx* ctx, size_t bytes, DevBuf* out)
 {
     if (bytes < 256) bytes = 256;
-    size_t best = ctx->pool.size();
-    for (size_t i = 0; i < ctx->pool.size(); ++i) {
-        const size_t have = ctx->pool[i].bytes;
-        if (have >= bytes && have / 2 <= bytes && (best == ctx->pool.size() || have < ctx->pool[best].bytes)) best = i;
-    }
-    if (best < ctx->pool.size()) {
-        *out = ctx->pool[best];
-        ctx->pool_bytes -= out->bytes;
-        ctx->pool.erase(ctx->pool.begin() + (ptrdiff_t)best);
-        return SFH_OK;
+    {
+        std::lock_guard<std::mutex> g(ctx->pool_mu);
+        size_t best = ctx->pool_n;
+        for (size_t i = 0; i < ctx->pool_n; ++i) {
+            const size_t have = ctx->pool[i].bytes;
+            if (have >= bytes && have / 2 <= bytes && (best == ctx->pool_n || have < ctx->pool[best].bytes)) best = i;
+        }
+        if (best < ctx->pool_n) {
+            *out = ctx->pool[best];
+            ctx->pool_bytes -= out->bytes;
+            ctx->pool[best] = ctx->pool[--ctx->pool_n];
+            return SFH_OK;
+        }
     }
     // an eighth more than asked for, so that the next catalogue of about this size fits
-    const size_t want = bytes + bytes / 8;
-    out->bytes = want;
-    if (hipMalloc(&out->ptr, want) == hipSuccess) return SFH_OK;
-    (void)hipGetLastError();
-    pool_clear(ctx);
+    out->bytes = bytes + bytes / 8;
+    if (device_alloc(ctx, &out->ptr, out->bytes) == hipSuccess) return SFH_OK;
     out->bytes = bytes;
-    if (hipMalloc(&out->ptr, bytes) == hipSuccess) return SFH_OK;
-    (void)hipGetLastError();
+    if (device_alloc(ctx, &out->ptr, bytes) == hipSuccess) return SFH_OK;
     *out = DevBuf{};
     return set_error(ctx, SFH_ERR_ALLOC, "hipMalloc(%zu) failed", bytes);
 }
 
 void pool_put(sfh_ctx* ctx, DevBuf* b)
 {
-    if (b->ptr && ctx->pool_bytes + b->bytes <= kPoolBytes && ctx->pool.size() < ctx->pool.capacity()) {
-        ctx->pool.push_back(*b);
-        ctx->pool_bytes += b->bytes;
-    } else if (b->ptr) {
-        (void)hipFree(b->ptr);
+    {
+        std::lock_guard<std::mutex> g(ctx->pool_mu);
+        if (b->ptr && ctx->pool_bytes + b->bytes <= kPoolBytes && ctx->pool_n < kPoolBuffers) {
+            ctx->pool[ctx->pool_n++] = *b;
+            ctx->pool_bytes += b->bytes;
+            *b = DevBuf{};
+        }
     }
+    if (b->ptr) (void)hipFree(b->ptr);
     *b = DevBuf{};
 }
 
@@ -528,13 +547,20 @@ int sfh_ctx_create(int device, void* stream, sfh_ctx** out)
         g_create_error = "noalloc_init: hipGetSymbolAddress of the static fg! buffer failed";
         return rc;
     }
-    c->pool.reserve(kPoolBuffers);
+    {
+        std::lock_guard<std::mutex> g(g_ctxs_mu);
+        g_ctxs.push_back(c);
+    }
     *out = c;
     return SFH_OK;
 }
 
 static void ctx_teardown(sfh_ctx* ctx)
 {
+    {
+        std::lock_guard<std::mutex> g(g_ctxs_mu);
+        g_ctxs.erase(std::find(g_ctxs.begin(), g_ctxs.end(), ctx));
+    }
     {
         std::lock_guard<std::recursive_mutex> g(ctx->mu);
         hipSetDevice(ctx->device);
@@ -769,7 +795,7 @@ static int templates_make(sfh_ctx* ctx, const float* src, bool src_device, int64
     t->ctx = ctx;
     t->nbins = nbins;
     t->ntemplates = ntemplates;
-    if (hipMalloc(&t->d_models, (size_t)ld * ntemplates * sizeof(float)) != hipSuccess) {
+    if (device_alloc(ctx, &t->d_models, (size_t)ld * ntemplates * sizeof(float)) != hipSuccess) {
         delete t;
         return set_error(ctx, SFH_ERR_ALLOC, "hipMalloc for %lld x %lld templates failed",
                          (long long)ld, (long long)ntemplates);
@@ -848,7 +874,7 @@ static int data_make(sfh_ctx* ctx, const double* src, bool dev, int64_t nbins, s
     sfh_data* d = new sfh_data();
     d->ctx = ctx;
     d->nbins = nbins;
-    if (hipMalloc(&d->d_data, (size_t)nbins * sizeof(double)) != hipSuccess) {
+    if (device_alloc(ctx, &d->d_data, (size_t)nbins * sizeof(double)) != hipSuccess) {
         delete d;
         return set_error(ctx, SFH_ERR_ALLOC, "hipMalloc for data failed");
     }
@@ -1099,7 +1125,7 @@ int sfh_buffer_alloc(sfh_ctx* ctx, int64_t bytes, void** d_ptr)
     SFH_ARG_CHECK(ctx, d_ptr && bytes >= 0, "sfh_buffer_alloc: bad arguments");
     *d_ptr = nullptr;
     void* p = nullptr;
-    if (hipMalloc(&p, (size_t)(bytes > 0 ? bytes : 1)) != hipSuccess)
+    if (device_alloc(ctx, &p, (size_t)(bytes > 0 ? bytes : 1)) != hipSuccess)
         return set_error(ctx, SFH_ERR_ALLOC, "hipMalloc(%lld) failed", (long long)bytes);
     *d_ptr = p;
     return SFH_OK;

@@ -22,6 +22,9 @@ struct DevBuf {
     size_t bytes = 0;
 };
 
+// What a context's pool holds at most (pool_put).
+constexpr size_t kPoolBytes = (size_t)1 << 30, kPoolBuffers = 64;
+
 struct KernelStat {
     double total_ms = 0.0;
     int64_t launches = 0;
@@ -46,9 +49,11 @@ struct sfh_ctx {
     std::vector<hipEvent_t> event_pool;
     // named scratch buffers
     std::map<std::string, sfh::DevBuf> scratch;
-    // buffers of destroyed catalogues, for the next ones (pool_get / pool_put)
-    std::vector<sfh::DevBuf> pool;
-    size_t pool_bytes = 0;
+    // buffers of destroyed catalogues, for the next ones (pool_get / pool_put),
+    // under a lock of their own: any context's allocation may give them back
+    std::mutex pool_mu;
+    sfh::DevBuf pool[sfh::kPoolBuffers];
+    size_t pool_n = 0, pool_bytes = 0;
     // small pinned host staging buffer
     void* pinned = nullptr;
     size_t pinned_bytes = 0;
@@ -97,15 +102,26 @@ int bind(sfh_ctx* ctx);
 
 // Grow-only named scratch buffer.
 int scratch(sfh_ctx* ctx, const char* name, size_t bytes, void** out);
+// hipMalloc on the context's device, for every allocation of the library: where
+// it fails, the pools of all contexts on that device are given back and it is
+// tried once more.
+hipError_t device_alloc(sfh_ctx* ctx, void** out, size_t bytes);
+template <typename T>
+hipError_t device_alloc(sfh_ctx* ctx, T** out, size_t bytes)
+{
+    void* p = nullptr;
+    const hipError_t e = device_alloc(ctx, &p, bytes);
+    *out = (T*)p;
+    return e;
+}
 // Device buffers that outlive one call but not their handle (catalogues).  A
 // buffer put back is handed out again to a request that fills at least half
 // of it; every use is on the context's stream, so the order there is all the
 // waiting a new owner needs.  At most kPoolBytes in kPoolBuffers are held; the
-// rest, and all of them with the context or when an allocation fails, go back
-// to the device.
+// rest, and all of them with the context or when an allocation of the library
+// fails (device_alloc), go back to the device.
 // (hipFree unmaps: 0.8 ms for the 100 MB of a 2.7M-system catalogue, and
 // hipMalloc about half of that again; a sample-observe-bin pass 2.49 -> 1.09 ms.)
-constexpr size_t kPoolBytes = (size_t)1 << 30, kPoolBuffers = 64;
 int pool_get(sfh_ctx* ctx, size_t bytes, DevBuf* out);
 void pool_put(sfh_ctx* ctx, DevBuf* b);
 void pool_clear(sfh_ctx* ctx);

@@ -1144,14 +1144,14 @@ int build_items(sfh_multifit* mf)
         if (mf->d_llp) (void)hipFree(mf->d_llp);
         mf->d_items = nullptr;
         mf->d_llp = nullptr;
-        SFH_HIP_TRY(ctx, hipMalloc(&mf->d_items, mf->nitems * sizeof(Item)));
-        SFH_HIP_TRY(ctx, hipMalloc(&mf->d_llp, mf->nitems * sizeof(double)));
+        SFH_HIP_TRY(ctx, device_alloc(ctx, &mf->d_items, mf->nitems * sizeof(Item)));
+        SFH_HIP_TRY(ctx, device_alloc(ctx, &mf->d_llp, mf->nitems * sizeof(double)));
         mf->items_cap = mf->nitems;
     }
     if (poff > mf->gp_cap) {
         if (mf->d_gp) (void)hipFree(mf->d_gp);
         mf->d_gp = nullptr;
-        SFH_HIP_TRY(ctx, hipMalloc(&mf->d_gp, poff * sizeof(double)));
+        SFH_HIP_TRY(ctx, device_alloc(ctx, &mf->d_gp, poff * sizeof(double)));
         mf->gp_cap = poff;
     }
     SFH_HIP_TRY(ctx, hipMemcpyAsync(mf->d_items, items.data(), mf->nitems * sizeof(Item), hipMemcpyHostToDevice,
@@ -1200,7 +1200,7 @@ template <typename T>
 int ensure(sfh_ctx* ctx, T** p, size_t count)
 {
     if (*p) return SFH_OK;
-    SFH_HIP_TRY(ctx, hipMalloc((void**)p, std::max<size_t>(count, 1) * sizeof(T)));
+    SFH_HIP_TRY(ctx, device_alloc(ctx, p, std::max<size_t>(count, 1) * sizeof(T)));
     return SFH_OK;
 }
 
@@ -1261,7 +1261,7 @@ int sfh_multifit_create(sfh_ctx* ctx, int64_t nfits, const sfh_templates* const*
     int rc = SFH_OK;
     int32_t* d_colfit = nullptr;
     do {
-        if (hipMalloc(&mf->d_blocked, blocked_elems * sizeof(float)) != hipSuccess) {
+        if (device_alloc(ctx, &mf->d_blocked, blocked_elems * sizeof(float)) != hipSuccess) {
             rc = set_error(ctx, SFH_ERR_ALLOC, "sfh_multifit_create: blocked template copy (%lld floats) failed",
                            (long long)blocked_elems);
             break;
@@ -1275,10 +1275,10 @@ int sfh_multifit_create(sfh_ctx* ctx, int64_t nfits, const sfh_templates* const*
                                ctx->stream, fd.C, fd.ld, fd.T, nblk, mf->d_blocked + boff[f]);
         }
         if ((rc = check_launch(ctx, "k_block_copy"))) break;
-        if (hipMalloc(&mf->d_fits, nfits * sizeof(FitDesc)) != hipSuccess ||
-            hipMalloc(&mf->d_V, (size_t)NVEC * mf->sumT * sizeof(double)) != hipSuccess ||
-            hipMalloc(&mf->d_nsum, nfits * sizeof(double)) != hipSuccess ||
-            hipMalloc(&d_colfit, mf->sumT * sizeof(int32_t)) != hipSuccess) {
+        if (device_alloc(ctx, &mf->d_fits, nfits * sizeof(FitDesc)) != hipSuccess ||
+            device_alloc(ctx, &mf->d_V, (size_t)NVEC * mf->sumT * sizeof(double)) != hipSuccess ||
+            device_alloc(ctx, &mf->d_nsum, nfits * sizeof(double)) != hipSuccess ||
+            device_alloc(ctx, &d_colfit, mf->sumT * sizeof(int32_t)) != hipSuccess) {
             rc = set_error(ctx, SFH_ERR_ALLOC, "sfh_multifit_create: device allocation failed");
             break;
         }

@@ -65,3 +65,41 @@ def test_two_threads(sfh, gpu_ctx):
     [t.start() for t in ts]
     [t.join() for t in ts]
     assert not bad
+
+
+def test_failed_allocations_give_the_pools_back(sfh, gpu_ctx):
+    """An allocation that does not fit, of any kind and in any context, first
+    empties the pools of all contexts.  The sizes are refused by the runtime at
+    once (petabytes), so nothing is filled up."""
+    import ctypes
+
+    import torch
+
+    def buffer(ctx):
+        p = ctypes.c_void_p()
+        ctx.check(ctx.lib.sfh_buffer_alloc(ctx.handle, 1 << 50, ctypes.byref(p)))
+
+    def templates(ctx):
+        sfh.HIPTemplates(ctx=ctx, device_ptr=x.data_ptr(), shape=(1 << 30, 1 << 18))
+
+    def data(ctx):
+        sfh.HIPData(ctx=ctx, device_ptr=x.data_ptr(), nbins=1 << 47)
+
+    x = torch.zeros(16, dtype=torch.float64, device="cuda")
+    a, b = sfh.Context(0), sfh.Context(0)
+    r, obs = _population(sfh, a, 4e5, 3)                # sizes the scratch buffers
+    obs.close()
+    for alloc in (buffer, templates, data):
+        for ctx in (a, b):
+            again, obs = _population(sfh, a, 4e5, 3)
+            assert _same(again, r)
+            obs.close()
+            free = torch.cuda.mem_get_info()[0]
+            with pytest.raises(sfh.DeviceError):
+                alloc(ctx)
+            assert torch.cuda.mem_get_info()[0] >= free + (10 << 20)
+    again, obs = _population(sfh, a, 4e5, 3)            # and the contexts go on working
+    assert _same(again, r)
+    obs.close()
+    a.close()
+    b.close()
