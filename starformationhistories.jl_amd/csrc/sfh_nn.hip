@@ -1363,14 +1363,13 @@ __global__ __launch_bounds__(kWG) void k_conv_fwd(const T* __restrict__ in, uint
 //
 // SiLU with the hardware reciprocal and one Newton step (within 1 ulp, as the
 // IEEE division, at a third of its instructions: the activations of the halo
-// included are this kernel's VALU work).  1 + exp(-x) is kept finite, where
-// the step is defined; below x = -87 the result is under 1e-36 either way.
+// included are this kernel's VALU work).  The step takes a finite denominator;
+// the reciprocal itself takes 1 + exp(-x) as it is, 0 for an infinite one, so
+// that below x = -89 the result is 0 however large |x| (between, under 1e-36).
 __device__ inline float silu_rcp(float x)
 {
-    const float d = 1.f + fminf(__expf(-x), 0x1p126f);
-    float r = __builtin_amdgcn_rcpf(d);
-    r = fmaf(fmaf(-d, r, 1.f), r, r);
-    return x * r;
+    const float d = 1.f + __expf(-x), r = __builtin_amdgcn_rcpf(d);
+    return x * fmaf(fmaf(-fminf(d, 0x1p126f), r, 1.f), r, r);
 }
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
