@@ -29,3 +29,20 @@ def test_few_walkers_against_oracle(sfh, O, gpu_ctx, N, T, B, precision, tol_ll)
         # so each of the two products by 2^-16
         q = data / (models.astype(np.float64) @ X[:, b])
         assert np.all(np.abs(G[:, b] - ref_G) <= 2.0 ** -16 * (models.T.astype(np.float64) @ (np.abs(1 - q) + q)))
+
+
+@pytest.mark.parametrize("N,T,B", [(100, 50, 500), (700, 300, 257), (1500, 40, 300), (3000, 600, 130), (4200, 257, 385),
+                                   (9000, 20, 140)])
+@pytest.mark.parametrize("precision", ["f64", "bf16x2", "fp32"])
+def test_every_split_and_tile_is_summed_once(sfh, gpu_ctx, N, T, B, precision):
+    """The gradient's bins in 1, 1, 2, 5, 8 and more splits over the XCDs: every
+    walker and template against FP64 products, within the bound above."""
+    from sfh_amd import synth
+    models = synth.synthetic_templates(N, T, seed=T)
+    x = np.random.default_rng(B).uniform(100, 1000, T)
+    data = synth.poisson_data(models.astype(np.float64) @ x, seed=3)
+    X = synth.walkers(x, B, 0.2, seed=4)
+    _, G = sfh.fg_batched(X, sfh.HIPTemplates(models), data, precision=precision)
+    C = models.astype(np.float64)
+    q = data[:, None] / (C @ X)
+    assert np.all(np.abs(G - C.T @ (1 - q)) <= 2.0 ** -16 * (C.T @ (np.abs(1 - q) + q)))
