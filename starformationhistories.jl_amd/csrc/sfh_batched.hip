@@ -1126,7 +1126,8 @@ static int fg_batched_impl(sfh_ctx* ctx, const sfh_templates* tpl, const sfh_dat
     if (d_G) {
         // 256 x 128 tiles (4 x 2 waves), one 512-thread workgroup per CU; the
         // bins are split so the workgroups fill whole waves of the 256 CUs
-        // (for 64 walkers or fewer 256 x 64 tiles of 4 x 1 waves: bound by one read
+        // (for 64 walkers or fewer, in the FP64 form, whose composite alone has tiles
+        // of fewer than 128, 256 x 64 tiles of 4 x 1 waves: bound by one read
         // of the templates, 34 us at the copy rate; 56 -> 40 us for 24 walkers)
         constexpr int GWR = 4, GRB = kTR * GWR;
         const bool narrow = ncb <= kTC;
@@ -1157,8 +1158,9 @@ static int fg_batched_impl(sfh_ctx* ctx, const sfh_templates* tpl, const sfh_dat
         EpiLL el{};
         EpiGrad eg{(float*)pg, Bpad, ops->tpad2};
         TimedLaunch tl(ctx, "batched_gradient");
-        const auto kernel = mode == FP32 ? (narrow ? k_gemm<GRAD_FP32, false, GWR, 1> : k_gemm<GRAD_FP32, false, GWR, 2>)
-                                         : (narrow ? k_gemm<GRAD_BF16, false, GWR, 1> : k_gemm<GRAD_BF16, false, GWR, 2>);
+        const auto kernel = mode == FP32 ? k_gemm<GRAD_FP32, false, GWR, 2>
+                            : narrow     ? k_gemm<GRAD_BF16, false, GWR, 1>
+                                         : k_gemm<GRAD_BF16, false, GWR, 2>;
         hipLaunchKernelGGL(kernel, grid, dim3(GWR * gwc * 64), 0, ctx->stream, ops->a2[mode == FP32 ? 1 : 0],
                            (const uint4*)pr, nrb2, ncb, kps, nkb2, sw, el, eg);
         if (int rc = check_launch(ctx, "gradient GEMM")) return rc;
