@@ -16,6 +16,7 @@ the FP64 oracle and the oracle timed on the host cores are reported beside it.
 from __future__ import annotations
 
 import argparse
+import hashlib
 import json
 import os
 import sys
@@ -591,6 +592,23 @@ def _fill_bench(S, torch, ctx, O, args, ncpu, net, la, mh, nstars, exact_rate):
 VALU_PEAK = 256 * 4 * 32 * 2.4e9
 
 
+def deposit_counters(npoints, pairs):
+    """The gathers' hardware counters (profiles/deposit_counters.json), or None
+    where they were taken of other kernels (the sources' hash) or templates."""
+    try:
+        with open(os.path.join(ROOT, "profiles", "deposit_counters.json")) as f:
+            c = json.load(f)
+    except OSError:
+        return None
+    h = hashlib.sha256()
+    for name in ("sfh_psf.h", "sfh_deposit.hip"):
+        with open(os.path.join(ROOT, "starformationhistories.jl_amd", "csrc", name), "rb") as f:
+            h.update(f.read())
+    if (c["kernel_points"], c["pairs"], c["sources_sha256"]) != (npoints, pairs, h.hexdigest()):
+        return None
+    return c["kernels"]
+
+
 def templates_bench(sfh, torch, ctx, O, args, ncpu):
     """The 700-template workload (70 ages x 10 metallicities, 2000-point
     isochrones, 200 x 300 grid, IMF 0.08-120 Msun, colour-magnitude
@@ -632,28 +650,31 @@ def templates_bench(sfh, torch, ctx, O, args, ncpu):
     dep_ms = kms["deposit_wide"] + kms["deposit_cov"]
     prep_ms = kms["pcs_count"] + kms["pcs_points"] + kms["pcs_desc"] + kms["deposit_order"]
     pairs_per_s = pairs / (dep_ms * 1e-3)
-    # VALU instructions of the two gathers over these templates, counted by the
-    # hardware (SQ_INSTS_VALU, wave64: 6.4e8 of k_dep_wide, 9.65e8 of
-    # k_dep_gather, for 2.83e10 pairs; deterministic for these inputs): what the
-    # kernels execute, inactive lanes included.  The published peak counts two
-    # wave64 instructions per 4 cycles per SIMD; what FP32 code of the strip's
-    # mix (an FMA reading a scalar register, a two-register multiply) reaches is
-    # measured in the same run by the library's issue-rate probe.
-    ops_per_pair = (6.4e8 + 9.65e8) * 64 / 2.83e10
-    achieved = pairs_per_s * ops_per_pair
+    # What the two gathers execute: the hardware's counts of a profiled run of
+    # this workload, used where they belong to this build and these templates.
+    # The published peak counts two wave64 instructions per 4 cycles per SIMD;
+    # what FP32 code of the strip's mix (an FMA reading a scalar register, a
+    # two-register multiply) reaches is measured in the same run by the
+    # library's issue-rate probe.
     issue = ctx.valu_issue_rate()
-    roof = {"bound": "valu", "kernel": "k_dep_wide + k_dep_gather<false>", "achieved": achieved / 1e12,
-            "peak": VALU_PEAK / 1e12,
-            "unit": "T VALU lane-instructions/s", "frac": achieved / VALU_PEAK, "traffic": None,
-            "measured_issue_rate": issue / 1e12, "frac_of_measured_issue_rate": achieved / issue,
+    cnt = deposit_counters(npts, pairs)
+    executed = sum(k["SQ_INSTS_VALU"] * 64 for k in cnt.values()) / (dep_ms * 1e-3) if cnt else None
+    active = sum(k["SQ_THREAD_CYCLES_VALU"] for k in cnt.values()) / (dep_ms * 1e-3) if cnt else None
+    roof = {"bound": "valu", "kernel": "k_dep_wide + k_dep_gather<false>",
+            "achieved": executed / 1e12 if cnt else None, "achieved_active_lanes": active / 1e12 if cnt else None,
+            "peak": VALU_PEAK / 1e12, "unit": "T VALU lane-instructions/s",
+            "frac": executed / VALU_PEAK if cnt else None, "frac_active_lanes": active / VALU_PEAK if cnt else None,
+            "traffic": None, "measured_issue_rate": issue / 1e12,
+            "frac_of_measured_issue_rate": executed / issue if cnt else None,
             "peak_note": "peak: the published FP32 vector rate (157.3 TFLOP/s = 78.6 T FMA lane-ops/s), two VALU "
                          "instructions per 4 cycles per SIMD from two waves (no packed FP32 in this build); "
                          "measured_issue_rate: the rate independent streams of the strip's instruction mix reach "
                          "on this device in this run (sfh_probe_valu_issue, four waves per SIMD)",
-            "algorithmic": f"{ops_per_pair:.3g} VALU lane-instructions per (point, bin) pair, the hardware's count of "
-                           f"both gathers on this workload (wide kernels on every fourth column, rows of one or two "
-                           f"merged Gauss-Legendre nodes) x {pairs:.4g} pairs per launch; "
-                           f"peak = 256 CUs x 4 SIMDs x 32 lanes x 2.4 GHz lane-instructions/s"}
+            "executed": "the wave64 VALU instructions that both gathers execute on this workload (SQ_INSTS_VALU of "
+                        "profiles/deposit_counters.json) x 64 lanes / the gathers' time in this run; "
+                        "active_lanes: the lanes of them that are not masked off (SQ_THREAD_CYCLES_VALU); "
+                        "peak = 256 CUs x 4 SIMDs x 32 lanes x 2.4 GHz lane-instructions/s"
+                        if cnt else "the counters of profiles/deposit_counters.json belong to another build or workload"}
     # the same templates through the host (NumPy) preparation, for comparison
     t0 = time.time()
     pc = [synth.template_points(s, 2000, edges, 120.0, correlation=0.6) for s in specs]
@@ -668,7 +689,7 @@ def templates_bench(sfh, torch, ctx, O, args, ncpu):
                    "IsochroneBatch), templates resident on the device out (upload, device preparation, "
                    "deposition); the isochrones themselves are synthetic inputs generated beforehand"}
     log(f"templates: {T} in {e2e_s * 1e3:.1f} ms end to end ({T / e2e_s:.4g}/s); kernels: prep {prep_ms:.2f} ms, "
-        f"deposit {dep_ms:.2f} ms ({pairs_per_s:.3g} pairs/s, VALU frac {roof['frac']:.2f}); host NumPy prep "
+        f"deposit {dep_ms:.2f} ms ({pairs_per_s:.3g} pairs/s, VALU frac {roof['frac'] or 0.0:.2f}); host NumPy prep "
         f"would take {host_prep_s:.2f} s")
     # parity of the bench's own templates on three of them
     ex, ey = (O.Range(e.first, e.step, e.length) for e in edges)
