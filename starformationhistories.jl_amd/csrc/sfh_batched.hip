@@ -1071,7 +1071,10 @@ static int fg_batched_impl(sfh_ctx* ctx, const sfh_templates* tpl, const sfh_dat
     // walkers per composite tile: 128, or for few of them a narrower FP64 tile (a
     // tile's walkers past B are matrix-core work for nothing: 24 walkers of 700
     // templates x 60,000 bins took 200 us in 128-wide tiles, 65 us in 128 x 32 and
-    // 62 us in 64 x 32 ones, whose 938 workgroups balance better)
+    // 62 us in 64 x 32 ones, whose 938 workgroups balance better).  Above 64 walkers
+    // both widths run the same products and the narrow one pads less: the whole
+    // call of 65, 128, 200, 387 and 512 walkers takes 265, 270, 471, 821 and 881 us
+    // in 64-wide tiles against 268, 273, 485, 945 and 953 here.
     const int cn = mode == F64 && B <= 32 ? 32 : mode == F64 && B <= 64 ? 64 : kBN;
     const int64_t Bpad = cdiv(B, cn) * cn;
     const int64_t nrb1 = ops->npad / 32, nkb1 = ops->tpad1 / 16, ncb = Bpad / 32, nct = Bpad / cn;

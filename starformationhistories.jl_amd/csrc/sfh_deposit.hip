@@ -22,14 +22,15 @@
 //   k_dep_finish  small launches, whose points are split into slices: their sums.
 // The pair work is VALU bound; HBM traffic is the descriptors in, the wide sums
 // out and in again (0.1 GB for 700 templates of 200 x 300 bins) and one write
-// of each template.  700 such templates (2.9e10 pairs, 74% of them in rows of
-// one node, 22% in rows of two): 7.5 ms with three nodes per row and every
-// column evaluated, 6.0 ms with the nodes merged, 4.0 ms (1.76 wide + 2.23)
-// with the wide kernels on a quarter of their columns and the accumulators
-// reached by LDS instead of flat accesses (VGPRs 112 -> 89), 3.4 ms with the
-// kernels of 0.026 <= e < 0.2 in the sum form, 2.8 ms with the wide gather's
-// FP64 sums in registers and its workgroups by cost, 2.7 ms (1.13 + 1.59) with
-// 8-byte keys for the hit search.
+// of each template.  700 such templates (2.8e10 pairs, most of them in rows of
+// one node or two): 7.5 ms with three nodes per row and every column evaluated,
+// 6.0 ms with the nodes merged, 4.0 ms (1.76 wide + 2.23) with the wide kernels
+// on a quarter of their columns and the accumulators reached by LDS instead of
+// flat accesses (VGPRs 112 -> 89), 3.4 ms with the sum form, 2.8 ms with the wide
+// gather's FP64 sums in registers and its workgroups by cost, 2.7 ms (1.13 +
+// 1.59) with 8-byte keys for the hit search; 2.9 ms (1.16 + 1.75) since every
+// node of a masked strip forms its own multiplier and the merged rows and the
+// sum form end where a template's tails would lose accuracy (sfh_psf.h).
 #include "sfh_internal.h"
 #include "sfh_psf.h"
 
@@ -149,8 +150,8 @@ __device__ __forceinline__ void each(const PointDesc* __restrict__ chunk, uint64
 // kStep-th column: the gather below with 16 nodes of one row per thread and
 // one form per loop, into the FP64 sums [slice][template][row][node] that
 // k_dep_gather (or k_dep_finish) interpolates.
-// VALU bound: 6.4e8 wave instructions for 700 templates, 94% of their lanes
-// active, 4.0 cycles each per SIMD; 1.13 ms (1.76 with the FP64 sums in LDS).
+// VALU bound: 6.3e8 wave instructions for 700 templates, 94% of their lanes
+// active, 3.9 cycles each per SIMD; 1.16 ms (1.76 with the FP64 sums in LDS).
 __global__ __launch_bounds__(kDepBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_dep_wide(
     const PointDesc* __restrict__ desc, const PointKey* __restrict__ keys, const int64_t* __restrict__ offsets,
     const int32_t* __restrict__ order, GatherArgs a)
@@ -246,8 +247,8 @@ __device__ inline void finish_cols(const GatherArgs& a, int64_t t, int row, int 
 // workgroups per CU), touched once per 64 points, so that the FP32 strip and
 // the per-point constants fit the registers of five waves per SIMD (the sums
 // in registers measured the same: 1577 against 1576 us for 700 templates).
-// VALU bound: 9.65e8 wave instructions, 57% of their lanes active (the short
-// footprints of the sum and erf-difference forms), 3.7 cycles each per SIMD.
+// VALU bound: 1.03e9 wave instructions, 68% of their lanes active (the short
+// footprints of the sum and erf-difference forms), 3.8 cycles each per SIMD.
 template <bool kAsym>
 __global__ __launch_bounds__(kDepBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_dep_gather(
     const PointDesc* __restrict__ desc, const PointKey* __restrict__ keys, const int64_t* __restrict__ offsets,

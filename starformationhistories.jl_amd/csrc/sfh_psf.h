@@ -657,7 +657,7 @@ __host__ __device__ __forceinline__ void static_for(F&& f)
 //   (m + s du)^2 = m^2 + 2 s m du + s^2 du^2,
 // so E(8 + j) = P B^j q[j] and E(7 - j) = P B^-(j+1) q[j], P = 2^-(m^2 + m du),
 // B = 2^(-2 m du), q[j] = 2^-(du (j + 1/2))^2 (prepared per point).  A row takes
-// three exp2 per node instead of one per node and column (an exp2 takes two
+// three exp2 per node (the two merged nodes four) instead of one per column (an exp2 takes two
 // VALU issue slots, an FMA or multiply one), and a column costs one FMA and one
 // multiply per node.  Each column adds the nodes in order k = 0, 1, 2.
 //
